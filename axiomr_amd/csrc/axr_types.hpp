@@ -133,8 +133,6 @@ constexpr uint64_t MAX_BATCH_FACES = 0x7FFFFFFFull;
 enum Counter : uint32_t {
     CNT_CLIP_FACES = 0,   // faces queued for the full clipper
     CNT_CLIP_RECS = 1,    // clip records reserved
-    CNT_OVF_PAIRS = 2,    // pairs placed in the overflow pool
-    CNT_ACTIVE = 3,       // non-empty bins listed by the scan
     CNT_ERROR = 4,        // sticky error bits, see ERR_*
     CNT_NEED_CLIP_FACES = 5,
     CNT_NEED_CLIP_RECS = 6,
@@ -150,6 +148,14 @@ constexpr uint32_t ERR_CLIP_RECS = 2u;
 constexpr uint32_t ERR_PAIRS = 4u;
 constexpr uint32_t ERR_BIG = 8u;
 constexpr uint32_t ERR_SKIPPED = 16u;   // a pass the host skipped had work: the frame is redrawn with it
+
+// Bins of binned mode: level k of a bin holds 2^(bin0_shift + k) entries, so
+// BIN_LEVELS levels reach past 2^31 entries for the smallest first level.
+constexpr uint32_t BIN0_MIN_SHIFT = 5, BIN0_MAX_SHIFT = 12;
+constexpr uint32_t BIN_LEVELS = 27;
+constexpr uint32_t CHUNK_NONE = 0xFFFFFFFFu;   // a level the pools had no room for
+constexpr uint32_t POOL_SUBS = 64;
+constexpr uint32_t POOL_STRIDE = 32;           // words between the pools' counters
 
 // Raster modes (axr_config.raster_mode).
 enum RasterMode : int32_t {
@@ -171,22 +177,23 @@ struct Arena {
     uint32_t* clip_faces;      // global face slots queued for clipping
     TriRec* clip_rec;          // clipped sub-triangles
     Vertex56* clip_verts;      // 3 per clip record
-    uint32_t* tile_count;      // per bin
-    uint32_t* tile_off;        // exclusive prefix of tile_count (+1 entry)
-    uint4* pairs;              // (bin, slot in bin, record ref, 0) per overlap:
-                               // wave_cap per setup wave, then the overflow pool
-    uint32_t* wave_pairs;      // pairs each setup wave wrote into its own region
-    uint32_t* bins;            // refs, grouped by bin
-    uint32_t* active;          // non-empty bins, in bin order
-    unsigned long long* scan_sums;   // per-scan-block partial sums (active << 32 | pairs)
+    uint32_t* tile_count;      // per bin: its entries (binned mode), whether it holds
+                               // keys (visibility mode)
+    // binned mode: record refs by bin (see bin_put in raster.hip)
+    uint32_t* bins;            // 2^bin0_shift first entries of every bin
+    uint32_t* bin_chunks;      // BIN_LEVELS words per bin: where its further entries
+                               // are (first entry in bin_pool + 1); 0: not allocated
+    uint32_t* bin_pool;        // POOL_SUBS sub-pools of sub_cap entries, then a shared
+                               // one of pool_cap
+    uint32_t* pool_next;       // the pools' fill, POOL_STRIDE words apart
     uint32_t cap_clip_faces;
     uint32_t cap_clip_recs;
-    uint32_t cap_waves;        // setup waves with a region
-    uint32_t wave_cap;         // pairs per setup-wave region (a wave that needs
-                               // more takes them from the overflow pool with
-                               // a single atomic)
-    uint32_t cap_ovf;          // overflow pool entries (after the regions)
-    uint32_t cap_bins;
+    uint32_t clip_static;      // queue entries with two clip records of their own
+                               // (clip_rec[2q], [2q + 1])
+    uint32_t bin0_shift;
+    uint32_t sub_cap;
+    uint32_t pool_cap;
+    uint32_t cap_chunks;       // words of bin_chunks (0: no binned-mode arrays)
     // visibility mode
     unsigned long long* vkeys; // per pixel of every view: (ordered depth << 32 | key),
                                // all ones when empty; the resolve leaves it empty

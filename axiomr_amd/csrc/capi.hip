@@ -126,18 +126,16 @@ static int grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, DevBuf& b, size_t by
     return AXR_OK;
 }
 
-FrameSize frame_size(const KArgs& ka, uint32_t wave_cap) {
+FrameSize frame_size(const KArgs& ka) {
     FrameSize fs;
     fs.faces = ka.total_faces;
     fs.tiles = ka.total_tiles;
     fs.pixels = ka.mode == RASTER_VISIBILITY ? ka.total_pixels : 0;
-    fs.wave_cap = wave_cap;
     return fs;
 }
 
 int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs, const ArenaNeeds& need) {
     const uint64_t faces = fs.faces, tiles = fs.tiles;
-    const uint32_t wave_cap = fs.wave_cap;
     if (faces > 0x7FFFFFFFull || tiles > 0x7FFFFFFFull || fs.pixels > 0xFFFFFFFFull)
         return fail(err, AXR_ERR_INVALID, "draw too large (%llu faces, %llu bins, %llu pixels)",
                     (unsigned long long)faces, (unsigned long long)tiles, (unsigned long long)fs.pixels);
@@ -147,12 +145,15 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     // bin pairs; binned mode keeps a 48-byte record per face slot
     const bool vis = fs.pixels != 0;
     uint64_t clip_faces = std::max<uint64_t>({4096, faces / 16, need.clip_faces, a.cap_clip_faces});
-    uint64_t clip_recs = std::max<uint64_t>({2 * clip_faces, need.clip_recs, a.cap_clip_recs});
-    // one pair region per setup wave (setup runs 4 waves per 256 faces)
-    uint64_t waves = vis ? a.cap_waves : std::max<uint64_t>(4 * ((faces + 255) / 256), a.cap_waves);
-    uint64_t ovf = vis ? a.cap_ovf : std::max<uint64_t>({faces / 4 + 16 * tiles + 4096, need.pairs, a.cap_ovf});
-    uint64_t nbins = vis ? a.cap_bins : std::max<uint64_t>({2 * faces + 16 * tiles + 4096, need.pairs, a.cap_bins});
-    uint64_t scan_blocks = (tiles + 4095) / 4096 + 1;
+    // binned mode: the first level of a bin holds four times the mean of faces
+    // per bin (a power of two of at least 32 entries), the shared pool what
+    // any spread of 2 faces + 16 bins + 4096 entries over the bins needs (a
+    // bin's further levels hold less than twice its entries), the sub-pools
+    // half as much again
+    uint32_t bin0_shift = BIN0_MIN_SHIFT;
+    while (bin0_shift < BIN0_MAX_SHIFT && (tiles << bin0_shift) < 4 * faces) ++bin0_shift;
+    const uint64_t pool = std::max<uint64_t>({2 * (2 * faces + 16 * tiles + 4096), need.pairs, a.pool_cap});
+    const uint64_t sub = std::max<uint64_t>((2 * faces + 16 * tiles + 4096) / POOL_SUBS, a.sub_cap);
     // visibility mode: large triangles and their 256-pixel work items
     uint64_t big_recs = 0, big_items = 0;
     if (fs.pixels) {
@@ -163,16 +164,18 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     int r;
     if ((r = grow(ctx, err, fa, fa.counters, CNT_COUNT * 4)) ||
         (r = grow(ctx, err, fa, fa.rec, std::max<uint64_t>(faces, 1) * (vis ? 4 : sizeof(TriRec)))) ||
-        (r = grow(ctx, err, fa, fa.clip_faces, clip_faces * 4)) ||
-        (r = grow(ctx, err, fa, fa.clip_rec, clip_recs * sizeof(TriRec))) ||
+        (r = grow(ctx, err, fa, fa.clip_faces, clip_faces * 4)))
+        return r;
+    // two records for every queue entry, and as many again for the faces with more
+    const uint64_t cap_clip_faces = std::min<uint64_t>(fa.clip_faces.bytes / 4, 0x1FFFFFFFull);
+    const uint64_t clip_recs = std::max<uint64_t>({2 * cap_clip_faces + 2 * clip_faces, need.clip_recs, a.cap_clip_recs});
+    if ((r = grow(ctx, err, fa, fa.clip_rec, clip_recs * sizeof(TriRec))) ||
         (r = grow(ctx, err, fa, fa.clip_verts, clip_recs * 3 * sizeof(Vertex56))) ||
         (r = grow(ctx, err, fa, fa.tile_count, (tiles + 1) * 4)) ||
-        (r = grow(ctx, err, fa, fa.tile_off, (tiles + 1) * 4)) ||
-        (r = grow(ctx, err, fa, fa.pairs, (waves * wave_cap + ovf) * 16)) ||
-        (r = grow(ctx, err, fa, fa.wave_pairs, waves * 4)) ||
-        (r = grow(ctx, err, fa, fa.bins, nbins * 4)) ||
-        (r = grow(ctx, err, fa, fa.active, (tiles + 1) * 4)) ||
-        (r = grow(ctx, err, fa, fa.scan_sums, scan_blocks * 8)) ||
+        (!vis && ((r = grow(ctx, err, fa, fa.bins, (tiles << bin0_shift) * 4)) ||
+                  (r = grow(ctx, err, fa, fa.bin_chunks, tiles * BIN_LEVELS * 4)) ||
+                  (r = grow(ctx, err, fa, fa.bin_pool, (POOL_SUBS * sub + pool) * 4)) ||
+                  (r = grow(ctx, err, fa, fa.pool_next, (POOL_SUBS + 1) * POOL_STRIDE * 4)))) ||
         (r = grow(ctx, err, fa, fa.vkeys, fs.pixels * 8)) ||
         (r = grow(ctx, err, fa, fa.big_rec, big_recs * sizeof(TriRec))) ||
         (r = grow(ctx, err, fa, fa.big_start, big_recs * 4)) ||
@@ -186,25 +189,26 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     a.clip_rec = (TriRec*)fa.clip_rec.p;
     a.clip_verts = (Vertex56*)fa.clip_verts.p;
     a.tile_count = (uint32_t*)fa.tile_count.p;
-    a.tile_off = (uint32_t*)fa.tile_off.p;
-    a.pairs = (uint4*)fa.pairs.p;
-    a.wave_pairs = (uint32_t*)fa.wave_pairs.p;
     a.bins = (uint32_t*)fa.bins.p;
-    a.active = (uint32_t*)fa.active.p;
-    a.scan_sums = (unsigned long long*)fa.scan_sums.p;
+    a.bin_chunks = (uint32_t*)fa.bin_chunks.p;
+    a.bin_pool = (uint32_t*)fa.bin_pool.p;
+    a.pool_next = (uint32_t*)fa.pool_next.p;
     a.vkeys = (unsigned long long*)fa.vkeys.p;
     a.big_rec = (TriRec*)fa.big_rec.p;
     a.big_start = (uint32_t*)fa.big_start.p;
     a.vcol = (uint32_t*)fa.vcol.p;
-    a.cap_clip_faces = (uint32_t)std::min<uint64_t>(fa.clip_faces.bytes / 4, 0xFFFFFFFFull);
+    a.cap_clip_faces = (uint32_t)cap_clip_faces;
+    a.clip_static = (uint32_t)cap_clip_faces;
     a.cap_clip_recs = (uint32_t)std::min<uint64_t>(
         {fa.clip_rec.bytes / sizeof(TriRec), fa.clip_verts.bytes / (3 * sizeof(Vertex56)), 0x7FFFFFFFull});
-    if (a.wave_cap != wave_cap) ++fa.gen;   // the pair layout changed: captured graphs are stale
-    a.wave_cap = wave_cap;
-    a.cap_waves = (uint32_t)std::min<uint64_t>(
-        {fa.wave_pairs.bytes / 4, 0x7FFFFFFFull / wave_cap, fa.pairs.bytes / 16 / wave_cap});
-    a.cap_ovf = (uint32_t)std::min<uint64_t>(fa.pairs.bytes / 16 - (uint64_t)a.cap_waves * wave_cap, 0x7FFFFFFFull);
-    a.cap_bins = (uint32_t)std::min<uint64_t>(fa.bins.bytes / 4, 0x7FFFFFFFull);
+    if (!vis) {
+        // sub-pool sizes keep their place between draws; a captured graph
+        // holds its own copy of these, and its buffers' moves change gen
+        a.bin0_shift = bin0_shift;
+        a.sub_cap = (uint32_t)std::min<uint64_t>(sub, 0x7FFFFFFFull / POOL_SUBS / 2);
+        a.pool_cap = (uint32_t)std::min<uint64_t>(fa.bin_pool.bytes / 4 - (uint64_t)POOL_SUBS * a.sub_cap, 0x7FFFFFFFull);
+        a.cap_chunks = (uint32_t)std::min<uint64_t>(fa.bin_chunks.bytes / 4, 0xFFFFFFFFull);
+    }
     a.cap_vkeys = (uint32_t)std::min<uint64_t>(fa.vkeys.bytes / 8, 0xFFFFFFFFull);
     a.cap_big_recs = (uint32_t)std::min<uint64_t>(
         {fa.big_rec.bytes / sizeof(TriRec), fa.big_start.bytes / 4, 0x7FFFFFFFull});
@@ -286,7 +290,6 @@ int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa) {
     FrameSize fs;
     fs.faces = 1024;
     fs.tiles = 1024;
-    fs.wave_cap = (uint32_t)ctx->cfg.bin_capacity;
     int r = arena_ensure(ctx, err, fa, fs);
     // null: this arena's draws hand over with events.  The value starts at
     // 0 (arena_reset waits for the stream).
@@ -298,11 +301,11 @@ int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa) {
     return r ? r : arena_reset(err, fa);
 }
 
-constexpr int kArenaBufs = 16;
+constexpr int kArenaBufs = 14;
 static void arena_buffers(FrameArena& fa, DevBuf* (&out)[kArenaBufs]) {
-    DevBuf* bufs[kArenaBufs] = {&fa.counters,  &fa.rec,      &fa.clip_faces, &fa.clip_rec,   &fa.clip_verts, &fa.tile_count,
-                                &fa.tile_off,  &fa.pairs,    &fa.wave_pairs, &fa.bins,       &fa.active,     &fa.scan_sums,
-                                &fa.vkeys,     &fa.big_rec,  &fa.big_start,  &fa.vcol};
+    DevBuf* bufs[kArenaBufs] = {&fa.counters, &fa.rec,        &fa.clip_faces, &fa.clip_rec,  &fa.clip_verts,
+                                &fa.tile_count, &fa.bins,     &fa.bin_chunks, &fa.bin_pool,  &fa.pool_next,
+                                &fa.vkeys,    &fa.big_rec,    &fa.big_start,  &fa.vcol};
     for (int i = 0; i < kArenaBufs; ++i) out[i] = bufs[i];
 }
 
@@ -740,7 +743,6 @@ static int arena_settle_overflow(axr_ctx* ctx, FrameArena& fa) {
     fs.faces = fa.rec.bytes / sizeof(TriRec);
     fs.tiles = fa.tile_count.bytes / 4 - 1;
     fs.pixels = fa.vkeys.bytes / 8;
-    fs.wave_cap = fa.a.wave_cap;
     return arena_check_overflow(ctx, ctx->err, fa, fs);
 }
 
@@ -1106,7 +1108,7 @@ int axr_draw(axr_ctx* ctx, axr_fb* fb, const axr_mesh* mesh, const axr_draw_para
     // of the same kernels); with an id plane the winners' colours wait in
     // the arena's colour slots
     ka.two_pass = async && ka.clear;
-    FrameSize fs = frame_size(ka, (uint32_t)ctx->cfg.bin_capacity);
+    FrameSize fs = frame_size(ka);
     if (ka.two_pass && fb->ids) fs.color_slots = fs.pixels;
     if (async && ka.mode == RASTER_VISIBILITY && overlap_enabled()) return draw_pipelined(ctx, fb, ka, fs, next_events(ctx));
     int r;
@@ -1294,7 +1296,7 @@ int axr_batch_create(axr_ctx* ctx, uint32_t nviews, axr_fb* const* fbs, const ax
     // binned mode: every view inside its frustum, so neither the setup's
     // classification nor the clipper is run
     ka.skip_clip = all_inside && ka.mode != RASTER_VISIBILITY;
-    b->fs = frame_size(ka, (uint32_t)ctx->cfg.bin_capacity);
+    b->fs = frame_size(ka);
     if ((r = arena_ensure(ctx, err, ctx->main, b->fs))) { axr_batch_destroy(b); return r; }
     // the batch's tables and captured graph hold the views' device pointers:
     // their framebuffers and meshes cannot be destroyed before the batch

@@ -65,8 +65,8 @@ struct ArenaNeeds {
 // so batches on different lanes overlap on the device.
 struct FrameArena {
     hipStream_t stream = nullptr;
-    DevBuf counters, rec, clip_faces, clip_rec, clip_verts, tile_count, tile_off, pairs, wave_pairs, bins, active,
-        scan_sums, vkeys, big_rec, big_start, vcol;
+    DevBuf counters, rec, clip_faces, clip_rec, clip_verts, tile_count, bins, bin_chunks, bin_pool, pool_next, vkeys,
+        big_rec, big_start, vcol;
     Arena a{};
     uint64_t gen = 0;          // bumped whenever a buffer moves: captured graphs are stale
     bool dirty = true;         // bin counts / counters need a k_prep before the next frame
@@ -175,10 +175,9 @@ struct FrameSize {
     uint64_t tiles = 0;      // bins over all views
     uint64_t pixels = 0;     // visibility-buffer pixels (0 in binned mode)
     uint64_t color_slots = 0; // pixels of a two-pass resolve into a framebuffer with ids
-    uint32_t wave_cap = 128; // pairs per setup-wave region (binned mode)
 };
 // High-water marks the kernels reported after an overflow.
-FrameSize frame_size(const KArgs& ka, uint32_t wave_cap);
+FrameSize frame_size(const KArgs& ka);
 
 int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa);
 void arena_destroy(axr_ctx* ctx, FrameArena& fa);

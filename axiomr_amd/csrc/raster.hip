@@ -3,11 +3,10 @@
 // Stage map (reference: src/tiled_pipeline.cpp:143-322 drawMesh):
 //   k_prep        zero the per-frame counters and bin counters
 //   k_setup       one lane per face: transform, frustum classification, cull,
-//                 triangle setup, bin counting           (tpl.cpp:185-240, 53-119)
+//                 triangle setup                         (tpl.cpp:185-240, 53-119)
+//                 and an entry in every bin it touches   (tpl.cpp:368-393)
 //   k_clip        faces that cross a frustum plane: the full 6-plane clipper
-//                 (pipeline.cpp:176-370), then cull/setup/count as above
-//   k_scan_*      exclusive prefix sum of the bin counts (the frame arena layout)
-//   k_scatter     write every (bin, record) pair          (tpl.cpp:368-393)
+//                 (pipeline.cpp:176-370), then cull/setup/bins as above
 //   k_raster      one workgroup per bin: coverage and early-Z into LDS keys,
 //                 then per-pixel resolve: depth test against the framebuffer,
 //                 shading of the winner, BGRA/depth store  (tpl.cpp:395-594,
@@ -29,10 +28,6 @@
 #pragma clang fp contract(off)
 
 namespace axr {
-
-constexpr int SCAN_THREADS = 1024;
-constexpr int SCAN_ITEMS = 4;
-constexpr int SCAN_BLOCK = SCAN_THREADS * SCAN_ITEMS;
 
 // ---------------------------------------------------------------------------
 // helpers
@@ -300,18 +295,19 @@ constexpr unsigned long long EMPTY_KEY = ~0ull;
 
 // ---------------------------------------------------------------------------
 // k_prep: zero per-frame counters (the sticky error word and the "need"
-// high-water marks are left alone) and the bin counters/cursors.
+// high-water marks are left alone), the bin counters and the bins' chunk
+// table.
 
-// The arena cleans itself during a frame (k_raster zeroes the bin counts it
-// consumed and the per-frame counters), so k_prep runs only after the arena
-// is (re)allocated or after an overflow.
+// The arena cleans itself during a frame (k_raster zeroes what it consumed),
+// so k_prep runs only after the arena is (re)allocated or after an overflow.
 __global__ void k_prep(Arena ar, uint32_t ntiles) {
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     if (tid < CNT_ERROR || tid == CNT_BIG_ITEMS || tid == CNT_BIG_RECS) ar.counters[tid] = 0;
-    for (uint32_t i = tid; i < ntiles; i += gridDim.x * blockDim.x) {
-        ar.tile_count[i] = 0;
-    }
-    for (uint32_t i = tid; i < ar.cap_vkeys; i += gridDim.x * blockDim.x) ar.vkeys[i] = ~0ull;
+    const uint32_t stride = gridDim.x * blockDim.x;
+    for (uint32_t i = tid; i < ntiles; i += stride) ar.tile_count[i] = 0;
+    for (uint32_t i = tid; i < ar.cap_chunks; i += stride) ar.bin_chunks[i] = 0;
+    if (ar.cap_chunks && tid < (POOL_SUBS + 1) * POOL_STRIDE) ar.pool_next[tid] = 0;
+    for (uint32_t i = tid; i < ar.cap_vkeys; i += stride) ar.vkeys[i] = ~0ull;
 }
 
 // ---------------------------------------------------------------------------
@@ -344,71 +340,148 @@ struct BinRange {
     }
 };
 
-// Emit the (bin, slot, ref) pairs of one record per lane, for a whole wave
-// (all 64 lanes must call it).  The wave writes into its own region of the
-// pair array (no shared counter); lanes that hit the same bin in the same
-// round share one atomic on that bin's counter, which also hands every pair
-// its final slot inside the bin, so the scatter pass needs no atomics.
-template <int T>
-__device__ __forceinline__ void emit_pairs_wave(const Arena& ar, const ViewDesc& V, bool on, const Rect& rc,
-                                                uint32_t ref, uint32_t wave) {
-    const BinRange<T> br(rc, on);
-    const uint32_t n = br.count();
-    const uint32_t incl = wave_incl_scan(n);
-    const uint32_t total = __shfl(incl, 63);
-    uint32_t base = wave * ar.wave_cap;
-    bool fits = true;
-    if (total > ar.wave_cap) {
-        uint32_t o = 0;
-        if (__lane_id() == 0) o = atomicAdd(&ar.counters[CNT_OVF_PAIRS], total);
-        o = __shfl(o, 0);
-        fits = o + total <= ar.cap_ovf;
-        if (!fits && __lane_id() == 0) set_error(ar, ERR_PAIRS, CNT_NEED_PAIRS, o + total);
-        base = ar.cap_waves * ar.wave_cap + o;
-    }
-    if (__lane_id() == 0) ar.wave_pairs[wave] = total > ar.wave_cap ? 0u : total;
-    if (total == 0) return;
-    const uint32_t p0 = base + incl - n;
-    const uint32_t lane = __lane_id();
-    for (uint32_t k = 0; __ballot(k < n); ++k) {
-        const bool act = k < n;
-        const uint32_t bin = act ? br.bin(k, V) : 0u;
-        // group the lanes by bin (register work only), then every group's
-        // first lane takes the group's slots with one atomic, all groups'
-        // atomics in flight together
-        unsigned long long pending = __ballot(act), mine = 0ull;
-        int leader_of_mine = 0;
-        while (pending) {
-            const int leader = __ffsll((long long)pending) - 1;
-            const uint32_t lb = __builtin_amdgcn_readlane(bin, leader);
-            const unsigned long long m = __ballot(act && bin == lb) & pending;
-            if ((m >> lane) & 1ull) {
-                mine = m;
-                leader_of_mine = leader;
-            }
-            pending &= ~m;
-        }
-        uint32_t slot = 0;
-        if (act && leader_of_mine == (int)lane) slot = atomicAdd(&ar.tile_count[bin], (uint32_t)__popcll(mine));
-        slot = __shfl(slot, leader_of_mine);
-        if (act && fits) ar.pairs[p0 + k] = make_uint4(bin, slot + (uint32_t)__popcll(mine & __lanemask_lt()), ref, 0u);
-    }
+// Bins (binned mode).  A bin's entries, record references, fill levels: the
+// first holds 2^bin0_shift entries at a place of the bin's own, level k holds
+// 2^(bin0_shift + k) wherever the pools had room (bin_chunks names the place).
+// The lane that takes an entry writes it there at once, so no pass after the
+// setup sorts pairs into bins (pairs of 16 bytes, a prefix sum over the bins
+// and a scatter took two launches, 8 us of a small frame, and 120 us of the
+// 4M-triangle soup's 730).  The host sizes the first level for four times the
+// mean of faces per bin, so most bins of most frames never leave it.
+struct BinSlot {
+    uint32_t level, offset;   // entry `offset` of level `level`
+};
+__device__ __forceinline__ BinSlot bin_slot(const Arena& ar, uint32_t slot) {
+    const uint32_t level = 31u - (uint32_t)__clz((int)((slot >> ar.bin0_shift) + 1u));
+    return BinSlot{level, slot - (((1u << level) - 1u) << ar.bin0_shift)};
 }
 
-// Same for one lane on its own (divergent code such as the clipper).
-// The pairs go to the overflow pool.
+// Room for one chunk of n entries: from the sub-pool that the bin's number
+// picks (one counter for all bins would serialize the allocations, ~11 ns
+// each) or, when that is full or the chunk a large part of it, the shared
+// pool, whose size alone decides whether a frame fits.  0 if it does not,
+// else the chunk's first entry + 1.
+__device__ __forceinline__ uint32_t pool_take(const Arena& ar, uint32_t bin, uint32_t n) {
+    const uint32_t sub = bin % POOL_SUBS;
+    uint32_t* next = ar.pool_next + sub * POOL_STRIDE;
+    if (n <= ar.sub_cap / 4u && __hip_atomic_load(next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ar.sub_cap) {
+        const uint32_t o = atomicAdd(next, n);
+        if (o + n <= ar.sub_cap) return sub * ar.sub_cap + o + 1u;
+    }
+    const uint32_t o = atomicAdd(ar.pool_next + POOL_SUBS * POOL_STRIDE, n);
+    if ((unsigned long long)o + n <= ar.pool_cap) return POOL_SUBS * ar.sub_cap + o + 1u;
+    set_error(ar, ERR_PAIRS, CNT_NEED_PAIRS, o + n);
+    return 0u;
+}
+
+// Store entry `slot` of `bin` (act: this lane has one; all 64 lanes call
+// it).  The lane that took a level's first slot allocates the level and
+// publishes it in the chunk table; the others wait for that word.  The wait
+// ends: a level's first slot was taken before any later one of it, and
+// between taking it and publishing that lane waits for nothing (the loop
+// below comes after the publishing in every lane of the wave; the ballots
+// keep the wave together).
+constexpr uint32_t BIN_WAIT_TRIES = 1u << 20;   // about a second
+__device__ __forceinline__ void bin_put(const Arena& ar, bool act, uint32_t bin, uint32_t slot, uint32_t ref) {
+    const BinSlot b = bin_slot(ar, slot);
+    const bool spill = act && b.level != 0u;
+    if (act && !spill) ar.bins[((size_t)bin << ar.bin0_shift) + slot] = ref;
+    if (__ballot(spill) == 0ull) return;
+    uint32_t* cell = ar.bin_chunks + (size_t)bin * BIN_LEVELS + b.level;
+    if (spill && b.offset == 0u) {
+        const uint32_t at = pool_take(ar, bin, 1u << (ar.bin0_shift + b.level));
+        __hip_atomic_store(cell, at ? at : CHUNK_NONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    uint32_t at = 0u;
+    for (uint32_t tries = 0; __ballot(spill && at == 0u) != 0ull; ++tries) {
+        if (spill && at == 0u) at = __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tries == BIN_WAIT_TRIES && spill && at == 0u) {   // never seen; a frame that is redrawn, not a hang
+            raise_error(ar, ERR_PAIRS);
+            at = CHUNK_NONE;
+        }
+    }
+    if (spill && at != CHUNK_NONE) ar.bin_pool[(size_t)(at - 1u) + b.offset] = ref;
+}
+
+// Entry i of bin t.
+__device__ __forceinline__ uint32_t bin_get(const Arena& ar, uint32_t t, uint32_t i) {
+    const BinSlot b = bin_slot(ar, i);
+    if (b.level == 0u) return ar.bins[((size_t)t << ar.bin0_shift) + i];
+    return ar.bin_pool[(size_t)(ar.bin_chunks[(size_t)t * BIN_LEVELS + b.level] - 1u) + b.offset];
+}
+
+// Put one record per lane (on) into every bin of its rectangle, for a whole
+// wave (all 64 lanes must call it).
+// Lanes with a handful of bins each go round by round, a bin per lane: where
+// at least half the lanes repeat their neighbour's bin (a mesh's consecutive
+// faces), lanes of one bin share one atomic on its count; else (a soup)
+// every lane takes its own.  A lane with more bins would keep the others
+// waiting, so then the wave's (lane, bin) pairs are laid end to end and the
+// lanes take them in turn, EMIT_AHEAD atomics in flight each.
+constexpr uint32_t EMIT_ROUNDS = 6, EMIT_AHEAD = 4;
+
 template <int T>
-__device__ __forceinline__ void emit_pairs_lane(const Arena& ar, const ViewDesc& V, const Rect& rc, uint32_t ref) {
-    const BinRange<T> br(rc, true);
-    const uint32_t n = br.count();
-    const uint32_t o = atomicAdd(&ar.counters[CNT_OVF_PAIRS], n);
-    const bool fits = o + n <= ar.cap_ovf;
-    if (!fits) set_error(ar, ERR_PAIRS, CNT_NEED_PAIRS, o + n);
-    const uint32_t p0 = ar.cap_waves * ar.wave_cap + o;
-    for (uint32_t k = 0; k < n; ++k) {
-        const uint32_t bin = br.bin(k, V);
-        const uint32_t slot = atomicAdd(&ar.tile_count[bin], 1u);
-        if (fits) ar.pairs[p0 + k] = make_uint4(bin, slot, ref, 0u);
+__device__ __forceinline__ void emit_bins_wave(const Arena& ar, const ViewDesc& V, bool on, const Rect& rc,
+                                               uint32_t ref) {
+    const BinRange<T> br(rc, on);
+    const uint32_t n = br.count(), lane = __lane_id();
+    if (__ballot(n > EMIT_ROUNDS) == 0ull) {
+        for (uint32_t k = 0;; ++k) {
+            const bool act = k < n;
+            const unsigned long long live = __ballot(act);
+            if (live == 0ull) return;
+            const uint32_t bin = act ? br.bin(k, V) : ~0u;
+            const uint32_t before = __shfl_up(bin, 1);
+            uint32_t slot = 0;
+            if (2 * __popcll(__ballot(act && bin == before)) >= __popcll(live)) {
+                // group the lanes by bin (register work only), then every
+                // group's first lane takes the group's slots with one atomic,
+                // all groups' atomics in flight together
+                unsigned long long pending = live, mine = 0ull;
+                int leader_of_mine = 0;
+                while (pending) {
+                    const int leader = __ffsll((long long)pending) - 1;
+                    const uint32_t lb = __builtin_amdgcn_readlane(bin, leader);
+                    const unsigned long long m = __ballot(act && bin == lb);
+                    if ((m >> lane) & 1ull) {
+                        mine = m;
+                        leader_of_mine = leader;
+                    }
+                    pending &= ~m;
+                }
+                if (act && leader_of_mine == (int)lane) slot = atomicAdd(&ar.tile_count[bin], (uint32_t)__popcll(mine));
+                slot = __shfl(slot, leader_of_mine) + (uint32_t)__popcll(mine & __lanemask_lt());
+            } else if (act) {
+                slot = atomicAdd(&ar.tile_count[bin], 1u);
+            }
+            bin_put(ar, act, bin, slot, ref);
+        }
+    }
+    const uint32_t incl = wave_incl_scan(n), start = incl - n, total = __shfl(incl, 63);
+    for (uint32_t j0 = 0; j0 < total; j0 += 64u * EMIT_AHEAD) {
+        uint32_t bin[EMIT_AHEAD], slot[EMIT_AHEAD], r[EMIT_AHEAD];
+#pragma unroll
+        for (uint32_t q = 0; q < EMIT_AHEAD; ++q) {
+            const uint32_t j = j0 + 64u * q + lane;
+            // the last lane whose pairs start at or before j (a lane without
+            // pairs shares its start with the next lane that has some)
+            int o = 0;
+            for (int step = 32; step; step >>= 1)
+                if (__shfl(start, o + step) <= j) o += step;
+            BinRange<T> b(rc, false);
+            b.tx0 = __shfl(br.tx0, o);
+            b.ty0 = __shfl(br.ty0, o);
+            b.nx = __shfl(br.nx, o);
+            const uint32_t k = j - __shfl(start, o);
+            r[q] = __shfl(ref, o);
+            slot[q] = bin[q] = 0u;
+            if (j < total) {
+                bin[q] = b.bin(k, V);
+                slot[q] = atomicAdd(&ar.tile_count[bin[q]], 1u);
+            }
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < EMIT_AHEAD; ++q) bin_put(ar, j0 + 64u * q + lane < total, bin[q], slot[q], r[q]);
     }
 }
 
@@ -429,6 +502,14 @@ __device__ __forceinline__ void flag_bins(const Arena& ar, const ViewDesc& V, co
     const int tx1 = (rc.x1 - 1) / T, ty1 = (rc.y1 - 1) / T;
     for (int ty = rc.y0 / T; ty <= ty1; ++ty)
         for (int tx = rc.x0 / T; tx <= tx1; ++tx) ar.tile_count[V.tile_base + (uint32_t)(ty * V.tiles_x + tx)] = 1u;
+}
+
+// The same by a whole wave (the same rc in every lane).
+template <int T>
+__device__ __forceinline__ void flag_bins_wave(const Arena& ar, const ViewDesc& V, const Rect& rc) {
+    const int tx0 = rc.x0 / T, ty0 = rc.y0 / T, nx = (rc.x1 - 1) / T - tx0 + 1, ny = (rc.y1 - 1) / T - ty0 + 1;
+    for (int k = (int)__lane_id(); k < nx * ny; k += 64)
+        ar.tile_count[V.tile_base + (uint32_t)((ty0 + k / nx) * V.tiles_x + tx0 + k % nx)] = 1u;
 }
 
 // One lane rasterizes a whole (small) triangle: every covered pixel of rc
@@ -476,13 +557,6 @@ __device__ __forceinline__ void big_append_wave(const Arena& ar, bool big, const
     const uint32_t lo = __shfl((uint32_t)old, 0), hi = __shfl((uint32_t)(old >> 32), 0);
     if (!big) return;
     big_store(ar, r, hi + (uint32_t)__popcll(mask & __lanemask_lt()), lo + incl - nch, nch);
-}
-
-// Same for one lane on its own (the clipper).
-__device__ __forceinline__ void big_append_lane(const Arena& ar, const TriRec& r, uint32_t area) {
-    const uint32_t nch = big_chunks(area);
-    const unsigned long long old = atomicAdd(big_counter(ar), (1ull << 32) | nch);
-    big_store(ar, r, (uint32_t)(old >> 32), (uint32_t)old, nch);
 }
 
 // ---------------------------------------------------------------------------
@@ -534,7 +608,7 @@ __device__ __forceinline__ void setup_face(const KArgs& ka, const Arena& ar, uin
         else set_error(ar, ERR_CLIP_FACES, CNT_NEED_CLIP_FACES, cslot + 1);
         if (ka.skip_clip) raise_error(ar, ERR_SKIPPED);
     }
-    emit_pairs_wave<T>(ar, V, binnable, rc, g, g >> 6);
+    emit_bins_wave<T>(ar, V, binnable, rc, g);
 }
 
 // INSIDE: the host's bound put every view's mesh inside every frustum plane
@@ -674,28 +748,58 @@ __global__ __launch_bounds__(256) void k_vis(KArgs ka, Arena ar) {
 }
 
 // ---------------------------------------------------------------------------
-// k_clip: the reference's clipper on the faces k_setup queued.  A clipped
-// vertex is the 14 vertex floats followed by the clip position.
+// k_clip: the reference's clipper on the faces k_setup queued, one wave per
+// face.  A clipped vertex is the 14 vertex floats followed by the clip
+// position; the polygon (at most 8 triangles) lives in LDS, twice, and a
+// plane that some vertex is not inside of moves it from one copy to the
+// other: a lane per vertex takes the plane distances, a lane per triangle
+// decides the case and names the sources of its output vertices, then all
+// lanes compute the output floats (18 per vertex), every float by the
+// reference's operations in its order.  A queue rarely holds more than a few
+// thousand faces and each is a long chain of dependent steps, so the latency
+// of one face bounds the pass: one lane per face kept both copies in scratch
+// (3.4 KB a lane) and walked each float in turn.
 
-struct CV { float f[18]; };
+constexpr int CLIP_FLOATS = 18;
+constexpr int MAX_CLIPPED_VERTS = 24;
 
-__device__ __forceinline__ vec4 cv_clip(const CV& v) { return make4(v.f[14], v.f[15], v.f[16], v.f[17]); }
+struct ClipPoly { float f[MAX_CLIPPED_VERTS][CLIP_FLOATS]; };
+// Sources of an output vertex: a copy of vertex src & 255, or (bit 16 set)
+// the point at t between it and vertex (src >> 8) & 255.
+struct ClipPlan {
+    uint32_t src[MAX_CLIPPED_VERTS];
+    float t[MAX_CLIPPED_VERTS];
+};
+constexpr uint32_t CLIP_LERP = 1u << 16;
+struct ClipWave {
+    ClipPoly poly[2];
+    ClipPlan plan;
+};
 
-__device__ void cv_interp(const CV& a, const CV& b, float t, CV& o) {  // pipeline.cpp:243-272
+// The wave's LDS writes before its reads of other lanes' entries.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ vec4 cv_clip(const float* v) { return make4(v[14], v[15], v[16], v[17]); }
+
+// Float c of the vertex at t between a and b (reference pipeline.cpp:243-272).
+__device__ __forceinline__ float cv_interp(const float* a, const float* b, float t, int c) {
     const float s = 1.0f - t;
-    for (int i = 0; i < 3; ++i) o.f[i] = a.f[i] * s + b.f[i] * t;   // position
-    for (int k = 5; k < 14; k += 3) {                                 // normal, tangent, bitangent
-        vec3 m = make3(a.f[k] * s + b.f[k] * t, a.f[k + 1] * s + b.f[k + 1] * t, a.f[k + 2] * s + b.f[k + 2] * t);
-        m = normalize(m);
-        o.f[k] = m.x; o.f[k + 1] = m.y; o.f[k + 2] = m.z;
+    if (c >= 5 && c < 14) {   // normal, tangent, bitangent: normalized
+        const int k = 5 + (c - 5) / 3 * 3;
+        const vec3 m = make3(a[k] * s + b[k] * t, a[k + 1] * s + b[k + 1] * t, a[k + 2] * s + b[k + 2] * t);
+        return (a[c] * s + b[c] * t) * (1.0f / sqrtf(dot(m, m)));
     }
-    for (int i = 14; i < 18; ++i) o.f[i] = a.f[i] * s + b.f[i] * t;  // clip position
-    const float w0 = a.f[17], w1 = b.f[17];
-    const float u = (a.f[3] * w0) * s + (b.f[3] * w1) * t;
-    const float v = (a.f[4] * w0) * s + (b.f[4] * w1) * t;
-    const float iw = w0 * s + w1 * t;
-    o.f[3] = u / iw;
-    o.f[4] = v / iw;
+    if (c == 3 || c == 4) {   // uv: perspective-correct
+        const float w0 = a[17], w1 = b[17];
+        const float u = (a[c] * w0) * s + (b[c] * w1) * t;
+        const float iw = w0 * s + w1 * t;
+        return u / iw;
+    }
+    return a[c] * s + b[c] * t;   // position, clip position
 }
 
 __device__ __forceinline__ float edge_t(float din, float dout) {
@@ -703,310 +807,204 @@ __device__ __forceinline__ float edge_t(float din, float dout) {
     return (fabsf(denom) < 1e-7f) ? 0.5f : (din / denom);
 }
 
-__device__ __forceinline__ void cv_swap(CV& a, CV& b) { CV t = a; a = b; b = t; }
-
-// reference pipeline.cpp:302-370
-__device__ int clip_one_plane(int plane, CV& v0, CV& v1, CV& v2, CV& v3) {
-    float d0 = plane_dist(cv_clip(v0), plane), d1 = plane_dist(cv_clip(v1), plane), d2 = plane_dist(cv_clip(v2), plane);
-    if (d0 < 0.f && d1 < 0.f && d2 < 0.f) return 0;
-    if (d0 >= 0.f && d1 >= 0.f && d2 >= 0.f) { v3 = v0; return 3; }
-    const bool in0 = d0 >= 0.f, in1 = d1 >= 0.f, in2 = d2 >= 0.f;
-    if (in1 && !in0) {
-        cv_swap(v0, v1); float t = d0; d0 = d1; d1 = t;
-        cv_swap(v1, v2); t = d1; d1 = d2; d2 = t;
-    } else if (in2 && !in1) {
-        cv_swap(v2, v1); float t = d2; d2 = d1; d1 = t;
-        cv_swap(v1, v0); t = d1; d1 = d0; d0 = t;
-    }
-    cv_interp(v0, v2, edge_t(d0, d2), v3);
-    if (d1 >= 0.f) {
-        CV n2;
-        cv_interp(v1, v2, edge_t(d1, d2), n2);
-        v2 = n2;
-        return 4;
-    }
-    CV n1;
-    cv_interp(v0, v1, edge_t(d0, d1), n1);
-    v1 = n1;
-    v2 = v3;
-    return 3;
-}
-
-constexpr int MAX_CLIPPED_VERTS = 24;
-
-// reference pipeline.cpp:176-228; returns the vertex count (multiple of 3)
-__device__ int clip_triangle(CV* tris, CV* next) {
-    int count = 3;
-    for (int plane = 0; plane < 6; ++plane) {
-        int n = 0;
-        for (int i = 0; i < count; i += 3) {
-            CV v3;
-            int r = clip_one_plane(plane, tris[i], tris[i + 1], tris[i + 2], v3);
-            if (r == 3) {
-                if (n + 3 <= MAX_CLIPPED_VERTS) {
-                    next[n] = tris[i]; next[n + 1] = tris[i + 1]; next[n + 2] = tris[i + 2]; n += 3;
-                }
-            } else if (r == 4) {
-                if (n + 6 <= MAX_CLIPPED_VERTS) {
-                    next[n] = tris[i]; next[n + 1] = tris[i + 1]; next[n + 2] = tris[i + 2];
-                    next[n + 3] = tris[i]; next[n + 4] = tris[i + 2]; next[n + 5] = v3;
-                    n += 6;
-                }
-            }
+// One plane (reference pipeline.cpp:196-228, 302-370): the polygon of
+// `count` vertices in w->poly[cur] against `plane`.  Returns the new vertex
+// count; cur names the copy that holds it.  All 64 lanes call it.
+__device__ __forceinline__ int clip_plane_wave(ClipWave* w, int& cur, int count, int plane) {
+    const int lane = (int)__lane_id();
+    const float d = lane < count ? plane_dist(cv_clip(w->poly[cur].f[lane]), plane) : 0.0f;
+    // every vertex inside: every triangle passes through unchanged
+    if (__ballot(lane < count && !(d >= 0.f)) == 0ull) return count;
+    const int ntri = count / 3, v = 3 * (lane < ntri ? lane : 0);
+    float d0 = __shfl(d, v), d1 = __shfl(d, v + 1), d2 = __shfl(d, v + 2);
+    int a = v, b = v + 1, c = v + 2, r = 0;
+    if (d0 >= 0.f && d1 >= 0.f && d2 >= 0.f) {
+        r = 1;   // unchanged
+    } else if (!(d0 < 0.f && d1 < 0.f && d2 < 0.f)) {
+        const bool in0 = d0 >= 0.f, in1 = d1 >= 0.f, in2 = d2 >= 0.f;
+        if (in1 && !in0) {
+            a = v + 1; b = v + 2; c = v;
+            const float t = d0; d0 = d1; d1 = d2; d2 = t;
+        } else if (in2 && !in1) {
+            a = v + 2; b = v; c = v + 1;
+            const float t = d2; d2 = d1; d1 = d0; d0 = t;
         }
-        count = n;
-        for (int i = 0; i < n; ++i) tris[i] = next[i];
-        if (count == 0) break;
+        r = d1 >= 0.f ? 3 : 2;   // two triangles, or one cut off
     }
-    return count;
+    if (lane >= ntri) r = 0;
+    // output positions in triangle order; a triangle whose vertices no longer
+    // fit the 24 is dropped, a later smaller one may still fit
+    int n = 0, at = 0;
+    bool fits = false;
+    for (int i = 0; i < ntri; ++i) {
+        const int ri = __builtin_amdgcn_readlane(r, i);
+        const int need = ri == 0 ? 0 : (ri == 3 ? 6 : 3);
+        const bool ok = n + need <= MAX_CLIPPED_VERTS;
+        if (lane == i) {
+            at = n;
+            fits = ok;
+        }
+        if (ok) n += need;
+    }
+    if (fits && r) {
+        uint32_t* src = w->plan.src + at;
+        float* tt = w->plan.t + at;
+        const uint32_t ac = (uint32_t)a | ((uint32_t)c << 8) | CLIP_LERP;
+        src[0] = (uint32_t)a;
+        if (r == 1) {
+            src[1] = (uint32_t)b;
+            src[2] = (uint32_t)c;
+        } else if (r == 2) {
+            src[1] = (uint32_t)a | ((uint32_t)b << 8) | CLIP_LERP;
+            tt[1] = edge_t(d0, d1);
+            src[2] = ac;
+            tt[2] = edge_t(d0, d2);
+        } else {
+            const uint32_t bc = (uint32_t)b | ((uint32_t)c << 8) | CLIP_LERP;
+            const float tb = edge_t(d1, d2);
+            src[1] = (uint32_t)b;
+            src[2] = bc;
+            tt[2] = tb;
+            src[3] = (uint32_t)a;
+            src[4] = bc;
+            tt[4] = tb;
+            src[5] = ac;
+            tt[5] = edge_t(d0, d2);
+        }
+    }
+    wave_lds_fence();
+    const ClipPoly& in = w->poly[cur];
+    ClipPoly& out = w->poly[cur ^ 1];
+    for (int i = lane; i < n * CLIP_FLOATS; i += 64) {
+        const int ov = i / CLIP_FLOATS, c2 = i % CLIP_FLOATS;
+        const uint32_t src = w->plan.src[ov];
+        const float* p = in.f[src & 255u];
+        out.f[ov][c2] = (src & CLIP_LERP) ? cv_interp(p, in.f[(src >> 8) & 255u], w->plan.t[ov], c2) : p[c2];
+    }
+    wave_lds_fence();
+    cur ^= 1;
+    return n;
 }
+
+// One lane's edge setup and rectangle as every lane of the wave sees it.
+__device__ __forceinline__ RasterTri bcast_tri(const RasterTri& t, int lane) {
+    RasterTri r;
+    uint32_t w[sizeof(RasterTri) / 4];
+    __builtin_memcpy(w, &t, sizeof(RasterTri));
+    for (int i = 0; i < (int)(sizeof(RasterTri) / 4); ++i) w[i] = __builtin_amdgcn_readlane(w[i], lane);
+    __builtin_memcpy(&r, w, sizeof(RasterTri));
+    return r;
+}
+
+// Waves per workgroup and workgroups of the clipper: 4,096 waves, which the
+// queues of the measured scenes (hundreds to a few ten thousand faces) keep
+// busy for a handful of faces each.
+constexpr int CLIP_WAVES = 4;
+constexpr int CLIP_BLOCKS = 1024;
 
 template <int T, bool BATCH, bool VIS>
-__global__ __launch_bounds__(64) void k_clip(KArgs ka, Arena ar) {
+__global__ __launch_bounds__(64 * CLIP_WAVES) void k_clip(KArgs ka, Arena ar) {
+    __shared__ ClipWave lds[CLIP_WAVES];
     if (ar.counters[CNT_ERROR]) return;
     const uint32_t n = imin((int)ar.counters[CNT_CLIP_FACES], (int)ar.cap_clip_faces);
-    CV tris[MAX_CLIPPED_VERTS], next[MAX_CLIPPED_VERTS];
-    for (uint32_t q = blockIdx.x * 64u + threadIdx.x; q < n; q += gridDim.x * 64u) {
-        const uint32_t g = ar.clip_faces[q];
+    const int lane = (int)__lane_id();
+    ClipWave* w = lds + (threadIdx.x >> 6);
+    // the same queue entry for the whole wave
+    for (uint32_t q = __builtin_amdgcn_readfirstlane(blockIdx.x * CLIP_WAVES + (threadIdx.x >> 6)); q < n;
+         q += gridDim.x * CLIP_WAVES) {
+        const uint32_t g = __builtin_amdgcn_readfirstlane(ar.clip_faces[q]);
         uint32_t vi = 0;
-        if constexpr (BATCH) vi = find_le(ka.face_bases, ka.nviews, g);
+        if constexpr (BATCH) vi = wave_find_le(ka.face_bases, ka.nviews, g);
         const ViewDesc& V = view_at<BATCH>(ka, vi);
         const uint32_t s = g - V.face_base;
         const DevGroup G = group_of(V, s);
         const uint32_t face = G.first + (s - G.rank_base);
-        for (int k = 0; k < 3; ++k) {
-            const uint32_t vtx = gld(V.idx, 3 * (size_t)face + k);
-            const Vertex56 src = gld(V.verts, vtx);
-            __builtin_memcpy(tris[k].f, &src, sizeof(Vertex56));
-            vec4 c = V.mvp * make4(load_pos(V.pos, vtx), 1.0f);
-            tris[k].f[14] = c.x; tris[k].f[15] = c.y; tris[k].f[16] = c.z; tris[k].f[17] = c.w;
+        int cur = 0;
+        wave_lds_fence();   // the previous face's reads of the polygon are done
+        if (lane < 3 * 14) {
+            const uint32_t vtx = gld(V.idx, 3 * (size_t)face + (size_t)(lane / 14));
+            w->poly[0].f[lane / 14][lane % 14] = gld(reinterpret_cast<const float*>(V.verts), 14 * (size_t)vtx + (size_t)(lane % 14));
         }
-        const int nv = clip_triangle(tris, next);
-        const uint32_t ntri = (uint32_t)(nv / 3);
+        if (lane < 3) {
+            const uint32_t vtx = gld(V.idx, 3 * (size_t)face + (size_t)lane);
+            const vec4 c = V.mvp * make4(load_pos(V.pos, vtx), 1.0f);
+            float* f = w->poly[0].f[lane];
+            f[14] = c.x; f[15] = c.y; f[16] = c.z; f[17] = c.w;
+        }
+        wave_lds_fence();
+        int count = 3;
+        for (int plane = 0; plane < 6 && count; ++plane) count = clip_plane_wave(w, cur, count, plane);
+        const uint32_t ntri = (uint32_t)(count / 3);
         if (ntri == 0) continue;
-        const uint32_t base = atomicAdd(&ar.counters[CNT_CLIP_RECS], ntri);
+        // one or two pieces (all but the faces across several planes) go to
+        // the queue entry's own two records; one counter for every face would
+        // serialize them (~11 ns each, 0.3 ms over the 4M-triangle soup)
+        uint32_t base = 2u * q;
+        if (ntri > 2u || q >= ar.clip_static) {
+            if (lane == 0) base = 2u * ar.clip_static + atomicAdd(&ar.counters[CNT_CLIP_RECS], ntri);
+            base = __builtin_amdgcn_readfirstlane(base);
+        }
         if (base + ntri > ar.cap_clip_recs) {
-            set_error(ar, ERR_CLIP_RECS, CNT_NEED_CLIP_RECS, base + ntri);
+            if (lane == 0) set_error(ar, ERR_CLIP_RECS, CNT_NEED_CLIP_RECS, base + ntri);
             continue;
         }
-        for (uint32_t j = 0; j < ntri; ++j) {
-            TriRec r = make_rec(cv_clip(tris[3 * j]), cv_clip(tris[3 * j + 1]), cv_clip(tris[3 * j + 2]), V.W, V.H);
-            if (is_backface(r)) continue;
-            RasterTri rt;
-            if (!raster_setup(r, rt)) continue;
-            Rect rc = screen_rect(rt, V.W, V.H);
-            if (!(rc.x0 < rc.x1 && rc.y0 < rc.y1)) continue;
-            const uint32_t slot = base + j;
-            r.c.y = s * 8u + j;
-            r.c.z = vi;
-            r.c.w = G.material & REC_MATERIAL_MASK;
-            ar.clip_rec[slot] = r;
-            for (int k = 0; k < 3; ++k) {
-                float* dst = reinterpret_cast<float*>(ar.clip_verts + 3 * (size_t)slot + k);
-                for (int i = 0; i < 14; ++i) dst[i] = tris[3 * j + k].f[i];
+        // one lane per triangle: cull, setup, record
+        bool on = false;
+        TriRec r;
+        RasterTri rt;
+        Rect rc{0, 0, 0, 0};
+        if (lane < (int)ntri) {
+            const float(*f)[CLIP_FLOATS] = w->poly[cur].f + 3 * lane;
+            r = make_rec(cv_clip(f[0]), cv_clip(f[1]), cv_clip(f[2]), V.W, V.H);
+            if (!is_backface(r) && raster_setup(r, rt)) {
+                rc = screen_rect(rt, V.W, V.H);
+                on = rc.x0 < rc.x1 && rc.y0 < rc.y1;
             }
-            if constexpr (VIS) {
-                const uint32_t area = (uint32_t)((rc.x1 - rc.x0) * (rc.y1 - rc.y0));
-                if (area <= (uint32_t)ka.small_footprint) vis_raster_rect<T>(ar, V, rt, rc, r.c.y);
-                else big_append_lane(ar, r, area);
-            } else {
-                emit_pairs_lane<T>(ar, V, rc, REF_CLIP | slot);
+            if (on) {
+                r.c.y = s * 8u + (uint32_t)lane;
+                r.c.z = vi;
+                r.c.w = G.material & REC_MATERIAL_MASK;
+                ar.clip_rec[base + lane] = r;
             }
+        }
+        const unsigned long long live = __ballot(on);
+        float* dst = reinterpret_cast<float*>(ar.clip_verts + 3 * (size_t)base);
+        for (int i = lane; i < count * 14; i += 64) {
+            const int v = i / 14;
+            if ((live >> (v / 3)) & 1ull) dst[i] = w->poly[cur].f[v][i % 14];
         }
         if constexpr (VIS) {
-            ar.clip_base[g] = base;
+            const uint32_t area = on ? (uint32_t)((rc.x1 - rc.x0) * (rc.y1 - rc.y0)) : 0u;
+            const bool big = area > (uint32_t)ka.small_footprint;
+            unsigned long long* vk = ar.vkeys + V.pix_base;
+            for (unsigned long long m = __ballot(on && !big); m; m &= m - 1ull) {
+                const int j = __ffsll((long long)m) - 1;
+                const RasterTri t = bcast_tri(rt, j);
+                const Rect tc = screen_rect(t, V.W, V.H);
+                const uint32_t tw = (uint32_t)(tc.x1 - tc.x0), np = tw * (uint32_t)(tc.y1 - tc.y0);
+                bool any = false;
+                for (uint32_t p = (uint32_t)lane; p < np; p += 64u) {
+                    const int px = tc.x0 + (int)(p % tw), py = tc.y0 + (int)(p / tw);
+                    float al, be, ga, z;
+                    if (cover(t, px, py, al, be, ga, z) && z < INFINITY) {
+                        atomicMin(&vk[(size_t)py * (size_t)V.W + (size_t)px], depth_key(z, s * 8u + (uint32_t)j));
+                        any = true;
+                    }
+                }
+                if (__ballot(any)) flag_bins_wave<T>(ar, V, tc);
+            }
+            big_append_wave(ar, big, r, area);
+            if (lane == 0) ar.clip_base[g] = base;
         } else {
-            TriRec m;
-            m.a = make_float4(0, 0, 0, 0);
-            m.b = make_float4(0, 0, 0, 0);
-            m.c = make_uint4(0u, s * 8u, base, REC_CLIPPED | (G.material & REC_MATERIAL_MASK));
-            ar.rec[g] = m;
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// prefix sum of the bin counts.  Each bin contributes the 64-bit value
-// (count > 0) << 32 | count, so one scan gives both the bin's offset in the
-// bins array (low word) and its position in the list of non-empty bins
-// (high word), which the raster walks instead of every bin.
-
-typedef unsigned long long u64;
-
-__device__ __forceinline__ u64 shfl_up64(u64 v, int o) {
-    uint32_t lo = __shfl_up((uint32_t)v, o), hi = __shfl_up((uint32_t)(v >> 32), o);
-    return ((u64)hi << 32) | lo;
-}
-
-__device__ __forceinline__ u64 wave_incl_scan64(u64 v) {
-    const int lane = (int)__lane_id();
-    for (int o = 1; o < 64; o <<= 1) {
-        u64 t = shfl_up64(v, o);
-        if (lane >= o) v += t;
-    }
-    return v;
-}
-
-// Exclusive scan across the 1024 threads of a block; returns the prefix and
-// the block total.
-__device__ __forceinline__ u64 block_excl_scan64(u64 v, u64* lds, u64& total) {
-    const int lane = (int)__lane_id(), wave = threadIdx.x >> 6;
-    u64 incl = wave_incl_scan64(v);
-    if (lane == 63) lds[wave] = incl;
-    __syncthreads();
-    if (wave == 0) {
-        u64 w = lane < (SCAN_THREADS / 64) ? lds[lane] : 0ull;
-        u64 wi = wave_incl_scan64(w);
-        if (lane < (SCAN_THREADS / 64)) lds[16 + lane] = wi - w;
-        if (lane == (SCAN_THREADS / 64) - 1) lds[32] = wi;
-    }
-    __syncthreads();
-    total = lds[32];
-    u64 r = lds[16 + wave] + incl - v;
-    __syncthreads();
-    return r;
-}
-
-__device__ __forceinline__ u64 bin_value(uint32_t count) { return ((u64)(count != 0) << 32) | count; }
-
-// Write the offsets of SCAN_ITEMS consecutive bins starting at `base` and
-// list the non-empty ones.
-__device__ __forceinline__ void write_offsets(const Arena& ar, uint32_t base, uint32_t ntiles, const uint32_t* c, u64 ex) {
-    for (int k = 0; k < SCAN_ITEMS; ++k) {
-        if (base + k < ntiles) {
-            ar.tile_off[base + k] = (uint32_t)ex;
-            if (c[k]) ar.active[ex >> 32] = base + k;
-        }
-        ex += bin_value(c[k]);
-    }
-}
-
-// The per-frame counters the scan is the last to need: the clip queue and
-// the clip records have been consumed by now.
-__device__ __forceinline__ void reset_consumed_counters(const Arena& ar) {
-    ar.counters[CNT_CLIP_FACES] = 0;
-    ar.counters[CNT_CLIP_RECS] = 0;
-}
-
-__device__ __forceinline__ void finish_scan(const Arena& ar, u64 total) {
-    const uint32_t pairs = (uint32_t)total;
-    ar.counters[CNT_ACTIVE] = (uint32_t)(total >> 32);
-    reset_consumed_counters(ar);
-    if (pairs > ar.cap_bins) set_error(ar, ERR_PAIRS, CNT_NEED_PAIRS, pairs);
-}
-
-// One block scans all bin counts (used when there are at most
-// SMALL_SCAN_TILES bins).
-constexpr uint32_t SMALL_SCAN_TILES = 65536;
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_single(Arena ar, uint32_t ntiles) {
-    __shared__ u64 lds[64];
-    __shared__ u64 carry;
-    if (ar.counters[CNT_ERROR]) return;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (uint32_t start = 0; start < ntiles; start += SCAN_BLOCK) {
-        const uint32_t base = start + threadIdx.x * SCAN_ITEMS;
-        uint32_t c[SCAN_ITEMS];
-        u64 s = 0;
-        for (int k = 0; k < SCAN_ITEMS; ++k) { c[k] = (base + k < ntiles) ? ar.tile_count[base + k] : 0u; s += bin_value(c[k]); }
-        u64 total;
-        const u64 ex = block_excl_scan64(s, lds, total) + carry;
-        write_offsets(ar, base, ntiles, c, ex);
-        __syncthreads();
-        if (threadIdx.x == 0) carry += total;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) finish_scan(ar, carry);
-}
-
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(Arena ar, uint32_t ntiles) {
-    __shared__ u64 lds[64];
-    if (ar.counters[CNT_ERROR]) return;
-    const uint32_t base = blockIdx.x * SCAN_BLOCK + threadIdx.x * SCAN_ITEMS;
-    u64 s = 0;
-    for (int k = 0; k < SCAN_ITEMS; ++k) if (base + k < ntiles) s += bin_value(ar.tile_count[base + k]);
-    u64 total;
-    block_excl_scan64(s, lds, total);
-    if (threadIdx.x == 0) ar.scan_sums[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_top(Arena ar, uint32_t nblocks) {
-    __shared__ u64 lds[64];
-    __shared__ u64 carry;
-    if (ar.counters[CNT_ERROR]) return;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (uint32_t start = 0; start < nblocks; start += SCAN_THREADS) {
-        const uint32_t i = start + threadIdx.x;
-        u64 v = i < nblocks ? ar.scan_sums[i] : 0ull;
-        u64 total;
-        u64 ex = block_excl_scan64(v, lds, total);
-        const u64 c = carry;
-        if (i < nblocks) ar.scan_sums[i] = c + ex;
-        __syncthreads();
-        if (threadIdx.x == 0) carry = c + total;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) finish_scan(ar, carry);
-}
-
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_down(Arena ar, uint32_t ntiles) {
-    __shared__ u64 lds[64];
-    if (ar.counters[CNT_ERROR]) return;
-    const uint32_t base = blockIdx.x * SCAN_BLOCK + threadIdx.x * SCAN_ITEMS;
-    uint32_t c[SCAN_ITEMS];
-    u64 s = 0;
-    for (int k = 0; k < SCAN_ITEMS; ++k) { c[k] = (base + k < ntiles) ? ar.tile_count[base + k] : 0u; s += bin_value(c[k]); }
-    u64 total;
-    const u64 ex = block_excl_scan64(s, lds, total) + ar.scan_sums[blockIdx.x];
-    write_offsets(ar, base, ntiles, c, ex);
-}
-
-// ---------------------------------------------------------------------------
-// k_scatter: every pair already knows its slot inside its bin; place it.
-// First the per-wave regions, then the overflow pool.
-
-__global__ __launch_bounds__(256) void k_scatter(Arena ar, uint32_t nwaves) {
-    if (ar.counters[CNT_ERROR]) return;
-    const uint32_t stride = gridDim.x * 256u;
-    const uint32_t cap = ar.wave_cap;
-    // one wave per setup wave's region: its pair count is read once and
-    // only the pairs it holds are visited.  A wave takes SCATTER_REGIONS
-    // regions at a time with their loads in flight together (each region's
-    // chain is count -> pair -> bin offset -> store; a region rarely holds
-    // more than 64 pairs)
-    constexpr uint32_t SCATTER_REGIONS = 4;
-    const uint32_t lane = __lane_id();
-    const uint32_t nw = gridDim.x * 4u;
-    for (uint32_t w0 = (blockIdx.x * 256u + threadIdx.x) >> 6; w0 < nwaves; w0 += nw * SCATTER_REGIONS) {
-        uint32_t n[SCATTER_REGIONS], off[SCATTER_REGIONS];
-        uint4 p[SCATTER_REGIONS];
-#pragma unroll
-        for (uint32_t k = 0; k < SCATTER_REGIONS; ++k) {
-            const uint32_t w = w0 + k * nw;
-            n[k] = w < nwaves ? ar.wave_pairs[w] : 0u;
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < SCATTER_REGIONS; ++k)
-            if (lane < n[k]) p[k] = ar.pairs[(size_t)(w0 + k * nw) * cap + lane];
-#pragma unroll
-        for (uint32_t k = 0; k < SCATTER_REGIONS; ++k)
-            if (lane < n[k]) off[k] = ar.tile_off[p[k].x];
-#pragma unroll
-        for (uint32_t k = 0; k < SCATTER_REGIONS; ++k) {
-            if (lane < n[k]) ar.bins[off[k] + p[k].y] = p[k].z;
-            const uint4* reg = ar.pairs + (size_t)(w0 + k * nw) * cap;
-            for (uint32_t i = lane + 64u; i < n[k]; i += 64u) {
-                const uint4 q = reg[i];
-                ar.bins[ar.tile_off[q.x] + q.y] = q.z;
+            emit_bins_wave<T>(ar, V, on, rc, REF_CLIP | (base + (uint32_t)lane));
+            if (lane == 0) {
+                TriRec m;
+                m.a = make_float4(0, 0, 0, 0);
+                m.b = make_float4(0, 0, 0, 0);
+                m.c = make_uint4(0u, s * 8u, base, REC_CLIPPED | (G.material & REC_MATERIAL_MASK));
+                ar.rec[g] = m;
             }
         }
-    }
-    const uint32_t novf = imin((int)ar.counters[CNT_OVF_PAIRS], (int)ar.cap_ovf);
-    const uint4* ovf = ar.pairs + (size_t)ar.cap_waves * ar.wave_cap;
-    for (uint32_t q = blockIdx.x * 256u + threadIdx.x; q < novf; q += stride) {
-        const uint4 p = ovf[q];
-        ar.bins[ar.tile_off[p.x] + p.y] = p.z;
     }
 }
 
@@ -1257,10 +1255,7 @@ __device__ __forceinline__ void walk_wave(P* wp, const Arena& ar, const RasterTr
     if (pieces)
         put_piece(wp, lane, rt, ref, (uint32_t)x0 | ((uint32_t)y0 << 8) | ((uint32_t)w << 16) | ((uint32_t)h << 24),
                   key);
-    // the wave's LDS writes before its reads of other lanes' entries
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_fence();
     for (uint32_t j = lane; j < total; j += 64u) {
         // owner: the last lane whose pieces start at or before j (a lane
         // without pieces shares its start with the next lane that has some)
@@ -1292,7 +1287,7 @@ __device__ __forceinline__ const ViewDesc& bin_view(const KArgs& ka, const ViewD
 // sview (batches): the bin's view is copied into LDS once per bin, so that
 // every per-pixel read of its uniforms and pointers is an LDS read.
 template <int T, int NT, bool BATCH, int SK>
-__device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uint32_t t, unsigned long long* keys,
+__device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uint32_t t, uint32_t n, unsigned long long* keys,
                                            uint32_t* bigq, uint32_t& nbig, uint16_t* plist, ViewDesc* sview,
                                            typename PiecesOf<SK>::type* pieces) {
     if constexpr (BATCH) {
@@ -1301,8 +1296,6 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
         for (uint32_t i = threadIdx.x; i < sizeof(ViewDesc) / 4; i += NT)
             reinterpret_cast<uint32_t*>(sview)[i] = gld(src, i);
     }
-    const uint32_t n = ar.tile_count[t];
-    const uint32_t off = ar.tile_off[t];
     for (int p = threadIdx.x; p < T * T; p += NT) keys[p] = EMPTY_KEY;
     if (threadIdx.x == 0) nbig = 0;
     __syncthreads();
@@ -1320,7 +1313,7 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
         int x0 = 0, y0 = 0, w = 0, h = 0;
         uint32_t key = 0, ref = 0;
         if (i < n) {
-            ref = ar.bins[off + i];
+            ref = bin_get(ar, t, i);
             const TriRec r = rec_of(ar, ref);
             if (raster_setup(r, rt)) {
                 x0 = imax(ox, rt.fx0);
@@ -1362,17 +1355,21 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
         __syncthreads();
     }
 
+    // every entry has been read: leave the chunk table empty as well
+    if (threadIdx.x > 0 && threadIdx.x <= bin_slot(ar, n - 1).level) ar.bin_chunks[(size_t)t * BIN_LEVELS + threadIdx.x] = 0;
+
     // nbig is zero again here: it counts the covered pixels
     resolve_tile_kind<T, NT, SK>(V, ar, keys, ox, oy, ka.depth_is_clear != 0, ka.clear_depth, plist, &nbig);
 }
 
-// One workgroup per entry of the list of non-empty bins (the grid covers
-// every bin; blocks past the list exit after one load).  Workgroups are
-// dispatched to the 8 XCDs round-robin, so block ids are permuted to give
-// each XCD a contiguous run of the list: neighbouring bins share triangles,
-// vertices and texels in that XCD's L2.  SK >= 0: built for one shader kind
-// (see k_resolve).
+// One workgroup per bin; an empty bin's leaves after one load.  Workgroups
+// are dispatched to the 8 XCDs round-robin, so block ids are permuted to give
+// an XCD runs of XCD_RUN neighbouring bins, which share triangles, vertices
+// and texels in its L2; short runs, because the bins of a frame are not
+// equally full (one run per XCD of a small frame's bins put its whole object
+// on one XCD).  SK >= 0: built for one shader kind (see k_resolve).
 constexpr uint32_t NUM_XCD = 8;
+constexpr uint32_t XCD_RUN = 4;
 
 // Register bounds per shader kind (waves per SIMD the registers allow; the
 // LDS of a 128-thread block at 32 px bins, 19.9 KB with the full walk
@@ -1398,14 +1395,20 @@ __global__ __launch_bounds__(NT, raster_min_waves(SK)) void k_raster(KArgs ka, A
     __shared__ ViewDesc sview[1];
     __shared__ typename PiecesOf<SK>::type pieces[NT / 64];
     if (ar.counters[CNT_ERROR]) return;
-    // the pair overflow count was last needed by the scatter
-    if (blockIdx.x == 0 && threadIdx.x == 0) ar.counters[CNT_OVF_PAIRS] = 0;
-    const uint32_t nactive = ar.counters[CNT_ACTIVE];
-    const uint32_t chunk = (nactive + NUM_XCD - 1) / NUM_XCD;
-    const uint32_t j = blockIdx.x / NUM_XCD;
-    const uint32_t a = (blockIdx.x % NUM_XCD) * chunk + j;
-    if (j >= chunk || a >= nactive) return;
-    raster_bin<T, NT, BATCH, SK>(ka, ar, ar.active[a], keys, bigq, nbig, plist, sview, pieces);
+    if (blockIdx.x == 0) {
+        // the per-frame counters were last needed by k_clip
+        if (threadIdx.x == 0) {
+            ar.counters[CNT_CLIP_FACES] = 0;
+            ar.counters[CNT_CLIP_RECS] = 0;
+        }
+        for (uint32_t i = threadIdx.x; i <= POOL_SUBS; i += NT) ar.pool_next[i * POOL_STRIDE] = 0;
+    }
+    const uint32_t x = blockIdx.x % NUM_XCD, j = blockIdx.x / NUM_XCD;
+    const uint32_t t = (j / XCD_RUN * NUM_XCD + x) * XCD_RUN + j % XCD_RUN;
+    if (t >= ka.total_tiles) return;
+    const uint32_t n = ar.tile_count[t];
+    if (n == 0u) return;
+    raster_bin<T, NT, BATCH, SK>(ka, ar, t, n, keys, bigq, nbig, plist, sview, pieces);
 }
 
 // ---------------------------------------------------------------------------
@@ -2043,7 +2046,7 @@ static hipError_t launch_vis_t(const KArgs& ka, const Arena& ar, hipStream_t st,
         else stage_launch1(k_vis<T, BATCH>, dim3(vis_blocks), dim3(256), st, ev, 0, ka, ar);
     }
     // passes the host showed to have no work are not launched
-    if (BATCH || !ka.skip_clip) stage_launch1(k_clip<T, BATCH, true>, dim3(256), dim3(64), st, ev, 1, ka, ar);
+    if (BATCH || !ka.skip_clip) stage_launch1(k_clip<T, BATCH, true>, dim3(CLIP_BLOCKS), dim3(64 * CLIP_WAVES), st, ev, 1, ka, ar);
     if (BATCH || !ka.skip_big) stage_launch1(k_big<T, BATCH>, dim3(1024), dim3(256), st, ev, 2, ka, ar);
     if (!BATCH && ka.two_pass && ka.clear && ka.shader >= 0 && ka.shader < SHADER_COUNT) {
         // shade at once, write the framebuffer after the earlier draws
@@ -2062,7 +2065,7 @@ static hipError_t launch_vis_t(const KArgs& ka, const Arena& ar, hipStream_t st,
     return hipGetLastError();
 }
 
-// Binned mode: stage 0 k_setup, 1 k_clip, 2 the scan, 3 k_scatter, 4 k_raster.
+// Binned mode: stage 0 k_setup, 1 k_clip, 4 k_raster.
 template <int T, int NT, bool BATCH>
 static hipError_t launch_frame_t(const KArgs& ka, const Arena& ar, hipStream_t st, StageEvents* ev,
                                  const FbWait& wait) {
@@ -2074,19 +2077,9 @@ static hipError_t launch_frame_t(const KArgs& ka, const Arena& ar, hipStream_t s
         if (ka.skip_clip) stage_launch1(k_setup<T, BATCH, true>, dim3(setup_blocks), dim3(256), st, ev, 0, ka, ar);
         else stage_launch1(k_setup<T, BATCH>, dim3(setup_blocks), dim3(256), st, ev, 0, ka, ar);
     }
-    if (!ka.skip_clip) stage_launch1(k_clip<T, BATCH, false>, dim3(256), dim3(64), st, ev, 1, ka, ar);
-    if (ntiles <= SMALL_SCAN_TILES) {
-        stage_launch1(k_scan_single, dim3(1), dim3(SCAN_THREADS), st, ev, 2, ar, ntiles);
-    } else {
-        const uint32_t scan_blocks = (ntiles + SCAN_BLOCK - 1) / SCAN_BLOCK;
-        stage_launch(k_scan_reduce, dim3(scan_blocks), dim3(SCAN_THREADS), st, ev, 2, true, false, ar, ntiles);
-        stage_launch(k_scan_top, dim3(1), dim3(SCAN_THREADS), st, ev, 2, false, false, ar, scan_blocks);
-        stage_launch(k_scan_down, dim3(scan_blocks), dim3(SCAN_THREADS), st, ev, 2, false, true, ar, ntiles);
-    }
-    const uint32_t nwaves = setup_blocks * 4;
-    const uint32_t sblocks = imax(64, imin(8192, (int)((nwaves + 3) / 4)));
-    stage_launch1(k_scatter, dim3(sblocks), dim3(256), st, ev, 3, ar, nwaves);
-    const uint32_t rblocks = ((imax(1, (int)ntiles) + NUM_XCD - 1) / NUM_XCD) * NUM_XCD;
+    if (!ka.skip_clip) stage_launch1(k_clip<T, BATCH, false>, dim3(CLIP_BLOCKS), dim3(64 * CLIP_WAVES), st, ev, 1, ka, ar);
+    const uint32_t round = NUM_XCD * XCD_RUN;
+    const uint32_t rblocks = ((uint32_t)imax(1, (int)ntiles) + round - 1) / round * round;
     hipError_t e = fb_wait(st, wait);
     if (e != hipSuccess) return e;
     stage_launch1(by_shader<RasterK<T, NT, BATCH>::template K>(ka.shader), dim3(rblocks), dim3(NT), st, ev, 4, ka, ar);

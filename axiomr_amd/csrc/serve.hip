@@ -52,7 +52,6 @@ public:
 
     HipDevice(axr_ctx* ctx, const axr_server_config& cfg) : ctx_(ctx), cfg_(cfg) {
         tile_ = ctx->cfg.tile_size;
-        wave_cap_ = (uint32_t)ctx->cfg.bin_capacity;
         raster_threads_ = ctx->cfg.raster_threads;
         small_footprint_ = ctx->cfg.small_footprint;
         mode_ = ctx->cfg.raster_mode;
@@ -85,7 +84,6 @@ public:
             fs.faces = cfg_.max_batch_faces;
             fs.tiles = std::min<uint64_t>(cfg_.max_batch_tiles, lane_tiles());
             fs.pixels = mode_ == RASTER_VISIBILITY ? cfg_.max_batch_pixels : 0;
-            fs.wave_cap = wave_cap_;
             if ((r = arena_ensure(ctx_, err_, l.fa, fs))) return r;
             if ((r = dev_alloc(ctx_, err_, (void**)&l.d_views, views_bytes())) ||
                 (r = dev_alloc(ctx_, err_, (void**)&l.d_bases, bases_bytes())) ||
@@ -186,7 +184,7 @@ public:
                                        __builtin_huge_valf(), st);
         }
         if (e != hipSuccess) return hip_fail(err_, e, "server batch upload");
-        L.fs = frame_size(ka, wave_cap_);
+        L.fs = frame_size(ka);
         L.attempts = 0;
         int r = arena_ensure(ctx_, err_, L.fa, L.fs);
         if (r) return r;
@@ -238,7 +236,6 @@ private:
     ErrSink err_;
     std::vector<Lane> lanes_;
     int tile_ = 16, raster_threads_ = 64, small_footprint_ = 12, mode_ = RASTER_BINNED;
-    uint32_t wave_cap_ = 128;
     uint64_t overflow_retries_ = 0;
 };
 

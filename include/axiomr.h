@@ -110,27 +110,27 @@ typedef struct axr_draw_params {
 typedef struct axr_config {
     int32_t tile_size;           /* GPU bin edge: 8, 16 or 32 pixels (default 16) */
     int32_t raster_threads;      /* threads per bin workgroup: 64, 128 or 256 (default 64) */
-    int32_t bin_capacity;        /* (bin, triangle) pairs each setup wave keeps in its own
-                                    region, 64..1024 (default 128); more go to a shared pool */
+    int32_t bin_capacity;        /* 64..1024 (default 128); no effect: a bin's storage is
+                                    sized from the draw's faces and bins, and grows */
     int32_t small_footprint;     /* triangles covering at most this many pixels of a bin are
                                     walked by one lane, 1..1024 (default 12) */
     int32_t raster_mode;         /* AXR_RASTER_BINNED (default) or AXR_RASTER_VISIBILITY */
     int32_t reserved[3];
 } axr_config;
 
-/* Raster modes; both give the same pixels.  BINNED: setup, per-bin lists
- * (prefix sum + scatter), one workgroup per bin rasterizes into LDS and
- * resolves.  VISIBILITY: setup rasterizes small triangles straight into a
+/* Raster modes; both give the same pixels.  BINNED: setup puts every
+ * triangle into the lists of the bins it touches, one workgroup per bin
+ * rasterizes into LDS and resolves.  VISIBILITY: setup rasterizes small triangles straight into a
  * per-pixel 64-bit (depth, submission) key buffer with atomics, large ones
  * as work items; a per-bin pass shades the winners.  tile_size is the
- * resolve bin there; bin_capacity is unused. */
+ * resolve bin there. */
 enum { AXR_RASTER_BINNED = 0, AXR_RASTER_VISIBILITY = 1 };
 
 /* Kernel time per stage, from HIP events attached to the stage kernels'
  * own dispatches, summed over the frames drawn while profiling is on
  * (frames keep overlapping).  Binned mode: 0 setup (transform,
- * classification, cull, triangle setup, bin counts), 1 clip, 2 prefix sum
- * of the bin counts, 3 bin scatter, 4 per-bin raster + resolve.
+ * classification, cull, triangle setup, bin entries), 1 clip, 2 and 3
+ * unused, 4 per-bin raster + resolve.
  * Visibility mode: 0 setup + small-triangle raster, 1 clip, 2 large-triangle
  * work items, 3 shading of a two-pass resolve (else unused), 4 resolve or
  * the two-pass framebuffer pass.  Both: 5 the batched form's vertex stage
