@@ -231,16 +231,17 @@ struct KArgs {
     uint32_t total_faces;
     uint32_t total_tiles;
     int32_t tile_size;          // bin edge in pixels: 8, 16 or 32
-    int32_t raster_threads;     // workgroup size of k_raster: 64, 128 or 256
-    int32_t small_footprint;    // a triangle covering at most this many pixels
-                                // of a bin is walked by one lane
+    int32_t raster_threads;     // least workgroup size of k_raster: 64, 128 or 256
+    int32_t small_footprint;    // visibility mode: a triangle whose rectangle has at
+                                // most this many pixels is walked by k_vis
     int32_t mode;               // RasterMode
+    int32_t face_shift = 6;     // 2^face_shift faces per wave of the setup passes
     uint32_t total_pixels;
     int32_t shader = -1;        // the shader kind every view uses, -1 if they differ:
                                 // selects a resolve kernel built for that shader alone
-    int32_t clear = 0;          // visibility mode: k_resolve also clears every view's
-    uint32_t clear_bgra = 0;    // framebuffer to these values (a clear the draw
-    float clear_depth = 0.0f;   // absorbs instead of a pass of its own)
+    int32_t clear = 0;          // the last pass (k_resolve, k_finish, a plain draw's
+    uint32_t clear_bgra = 0;    // k_raster) also clears every view's framebuffer to these
+    float clear_depth = 0.0f;   // values (a clear the draw absorbs)
     int32_t two_pass = 0;       // plain visibility-mode draw with a clear: shade
                                 // (k_shade) apart from the framebuffer writes
                                 // (k_finish), which alone wait for earlier draws
@@ -264,10 +265,10 @@ struct KArgs {
     float cull_eye[3] = {0.0f, 0.0f, 0.0f};
     float cull_sign = 0.0f;
     float cull_tau = 0.0f;
-    int32_t depth_is_clear = 0; // binned mode: every framebuffer's depth plane holds
-                                // clear_depth (written just before, by k_clear /
-                                // k_clear_views): winners are tested against that
-                                // value instead of a load of the plane
+    int32_t depth_is_clear = 0; // binned batches: every framebuffer's depth plane holds
+                                // clear_depth (written just before, by k_clear_views):
+                                // winners are tested against that value instead of a
+                                // load of the plane
     ViewDesc one;
 };
 

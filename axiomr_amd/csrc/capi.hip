@@ -1096,8 +1096,8 @@ int axr_draw(axr_ctx* ctx, axr_fb* fb, const axr_mesh* mesh, const axr_draw_para
         }
         ctx->stats.passes_skipped += (uint64_t)ka.skip_clip + (uint64_t)ka.skip_big;
     }
-    if (fb->clear_pending && ka.mode == RASTER_VISIBILITY) {
-        // the resolve pass writes the clear (k_resolve, ka.clear)
+    if (fb->clear_pending) {
+        // the pass that writes the frame writes the clear (ka.clear)
         ka.clear = 1;
         ka.clear_bgra = fb->clear_bgra;
         ka.clear_depth = fb->clear_depth;
@@ -1107,18 +1107,11 @@ int axr_draw(axr_ctx* ctx, axr_fb* fb, const axr_mesh* mesh, const axr_draw_para
     // framebuffer writes (also when profiled, so the stage times are those
     // of the same kernels); with an id plane the winners' colours wait in
     // the arena's colour slots
-    ka.two_pass = async && ka.clear;
+    ka.two_pass = async && ka.clear && ka.mode == RASTER_VISIBILITY;
     FrameSize fs = frame_size(ka);
     if (ka.two_pass && fb->ids) fs.color_slots = fs.pixels;
     if (async && ka.mode == RASTER_VISIBILITY && overlap_enabled()) return draw_pipelined(ctx, fb, ka, fs, next_events(ctx));
     int r;
-    if (fb->clear_pending && !ka.clear) {
-        // binned mode: the clear is written now, so the winners are tested
-        // against its depth without loading the plane
-        if ((r = fb_settle(fb))) return r;
-        ka.depth_is_clear = 1;
-        ka.clear_depth = fb->clear_depth;
-    }
     if ((r = ctx_join(ctx)) || (r = arena_ensure(ctx, ctx->err, ctx->main, fs, ctx->need_floor))) return r;
     for (int attempt = 0; attempt < 8; ++attempt) {
         if ((r = ctx_launch(ctx, ka))) return r;

@@ -126,6 +126,13 @@ __device__ __forceinline__ X wave_uniform(const X& v) {
     return r;
 }
 
+// The wave's LDS writes before its reads of other lanes' entries.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Wave-aggregated append: returns this lane's slot for lanes with pred set.
 __device__ __forceinline__ uint32_t wave_append(uint32_t* counter, bool pred) {
     unsigned long long mask = __ballot(pred);
@@ -322,23 +329,25 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
     return v;
 }
 
-// Bin range of a pixel rectangle for bins of T x T pixels.
+// Bins of T x T pixels that a pixel rectangle of view V touches: nx x ny from
+// bin `first` on, rows `pitch` bins apart.
 template <int T>
 struct BinRange {
-    int tx0, ty0, nx, ny;
-    __device__ __forceinline__ BinRange(const Rect& rc, bool on) {
+    uint32_t first, pitch, nx, n;
+    __device__ __forceinline__ BinRange(const ViewDesc& V, const Rect& rc, bool on) {
+        first = pitch = nx = n = 0;
         if (on) {
-            tx0 = rc.x0 / T; ty0 = rc.y0 / T;
-            nx = (rc.x1 - 1) / T - tx0 + 1; ny = (rc.y1 - 1) / T - ty0 + 1;
-        } else {
-            tx0 = ty0 = nx = ny = 0;
+            const int tx0 = rc.x0 / T, ty0 = rc.y0 / T;
+            nx = (uint32_t)((rc.x1 - 1) / T - tx0 + 1);
+            n = nx * (uint32_t)((rc.y1 - 1) / T - ty0 + 1);
+            pitch = (uint32_t)V.tiles_x;
+            first = V.tile_base + (uint32_t)ty0 * pitch + (uint32_t)tx0;
         }
     }
-    __device__ __forceinline__ uint32_t count() const { return (uint32_t)(nx * ny); }
-    __device__ __forceinline__ uint32_t bin(uint32_t k, const ViewDesc& V) const {
-        return V.tile_base + (uint32_t)((ty0 + (int)(k / (uint32_t)nx)) * V.tiles_x + tx0 + (int)(k % (uint32_t)nx));
-    }
 };
+__device__ __forceinline__ uint32_t bin_of(uint32_t first, uint32_t pitch, uint32_t nx, uint32_t k) {
+    return first + k / nx * pitch + k % nx;
+}
 
 // Bins (binned mode).  A bin's entries, record references, fill levels: the
 // first holds 2^bin0_shift entries at a place of the bin's own, level k holds
@@ -412,48 +421,47 @@ __device__ __forceinline__ uint32_t bin_get(const Arena& ar, uint32_t t, uint32_
 
 // Put one record per lane (on) into every bin of its rectangle, for a whole
 // wave (all 64 lanes must call it).
-// Lanes with a handful of bins each go round by round, a bin per lane: where
-// at least half the lanes repeat their neighbour's bin (a mesh's consecutive
-// faces), lanes of one bin share one atomic on its count; else (a soup)
-// every lane takes its own.  A lane with more bins would keep the others
-// waiting, so then the wave's (lane, bin) pairs are laid end to end and the
-// lanes take them in turn, EMIT_AHEAD atomics in flight each.
+// Where at least half the lanes repeat their neighbour's first bin (a mesh's
+// consecutive faces) and none has more than a handful of bins, the wave goes
+// round by round, a bin per lane, and lanes of one bin share one atomic on
+// its count.  Else (a soup; large triangles) sharing finds nothing and a
+// lane with more bins would keep the others waiting, so the wave's (lane,
+// bin) pairs are laid end to end and the lanes take them in turn, EMIT_AHEAD
+// atomics in flight each.
 constexpr uint32_t EMIT_ROUNDS = 6, EMIT_AHEAD = 4;
 
 template <int T>
 __device__ __forceinline__ void emit_bins_wave(const Arena& ar, const ViewDesc& V, bool on, const Rect& rc,
                                                uint32_t ref) {
-    const BinRange<T> br(rc, on);
-    const uint32_t n = br.count(), lane = __lane_id();
-    if (__ballot(n > EMIT_ROUNDS) == 0ull) {
+    const BinRange<T> br(V, rc, on);
+    const uint32_t n = br.n, lane = __lane_id();
+    const uint32_t bin0 = n ? br.first : ~0u, prev0 = __shfl_up(bin0, 1);
+    const unsigned long long any = __ballot(n != 0u);
+    if (any == 0ull) return;
+    if (__ballot(n > EMIT_ROUNDS) == 0ull && 2 * __popcll(__ballot(n != 0u && bin0 == prev0)) >= __popcll(any)) {
         for (uint32_t k = 0;; ++k) {
             const bool act = k < n;
             const unsigned long long live = __ballot(act);
             if (live == 0ull) return;
-            const uint32_t bin = act ? br.bin(k, V) : ~0u;
-            const uint32_t before = __shfl_up(bin, 1);
+            const uint32_t bin = act ? bin_of(br.first, br.pitch, br.nx, k) : ~0u;
             uint32_t slot = 0;
-            if (2 * __popcll(__ballot(act && bin == before)) >= __popcll(live)) {
-                // group the lanes by bin (register work only), then every
-                // group's first lane takes the group's slots with one atomic,
-                // all groups' atomics in flight together
-                unsigned long long pending = live, mine = 0ull;
-                int leader_of_mine = 0;
-                while (pending) {
-                    const int leader = __ffsll((long long)pending) - 1;
-                    const uint32_t lb = __builtin_amdgcn_readlane(bin, leader);
-                    const unsigned long long m = __ballot(act && bin == lb);
-                    if ((m >> lane) & 1ull) {
-                        mine = m;
-                        leader_of_mine = leader;
-                    }
-                    pending &= ~m;
+            // group the lanes by bin (register work only), then every
+            // group's first lane takes the group's slots with one atomic,
+            // all groups' atomics in flight together
+            unsigned long long pending = live, mine = 0ull;
+            int leader_of_mine = 0;
+            while (pending) {
+                const int leader = __ffsll((long long)pending) - 1;
+                const uint32_t lb = __builtin_amdgcn_readlane(bin, leader);
+                const unsigned long long m = __ballot(act && bin == lb);
+                if ((m >> lane) & 1ull) {
+                    mine = m;
+                    leader_of_mine = leader;
                 }
-                if (act && leader_of_mine == (int)lane) slot = atomicAdd(&ar.tile_count[bin], (uint32_t)__popcll(mine));
-                slot = __shfl(slot, leader_of_mine) + (uint32_t)__popcll(mine & __lanemask_lt());
-            } else if (act) {
-                slot = atomicAdd(&ar.tile_count[bin], 1u);
+                pending &= ~m;
             }
+            if (act && leader_of_mine == (int)lane) slot = atomicAdd(&ar.tile_count[bin], (uint32_t)__popcll(mine));
+            slot = __shfl(slot, leader_of_mine) + (uint32_t)__popcll(mine & __lanemask_lt());
             bin_put(ar, act, bin, slot, ref);
         }
     }
@@ -468,15 +476,13 @@ __device__ __forceinline__ void emit_bins_wave(const Arena& ar, const ViewDesc& 
             int o = 0;
             for (int step = 32; step; step >>= 1)
                 if (__shfl(start, o + step) <= j) o += step;
-            BinRange<T> b(rc, false);
-            b.tx0 = __shfl(br.tx0, o);
-            b.ty0 = __shfl(br.ty0, o);
-            b.nx = __shfl(br.nx, o);
+            // the owner's own: the lanes of a batch's wave may lie in two views
+            const uint32_t first = __shfl(br.first, o), pitch = __shfl(br.pitch, o), nx = __shfl(br.nx, o);
             const uint32_t k = j - __shfl(start, o);
             r[q] = __shfl(ref, o);
             slot[q] = bin[q] = 0u;
             if (j < total) {
-                bin[q] = b.bin(k, V);
+                bin[q] = bin_of(first, pitch, nx, k);
                 slot[q] = atomicAdd(&ar.tile_count[bin[q]], 1u);
             }
         }
@@ -562,7 +568,15 @@ __device__ __forceinline__ void big_append_wave(const Arena& ar, bool big, const
 // ---------------------------------------------------------------------------
 // k_setup: one lane per face (submission order across views).
 
-// Face slot g of view V (all 64 lanes of the wave call it).
+// Face slot of this lane: 2^face_shift consecutive faces per wave, in its
+// first lanes (~0: none).  A draw of few faces takes 16 faces per wave, so
+// that the wave's other lanes help with what comes after the setup: bin
+// entries, coverage.
+__device__ __forceinline__ uint32_t face_slot(const KArgs& ka) {
+    const uint32_t wave = (blockIdx.x * 256u + threadIdx.x) >> 6, lane = __lane_id();
+    return (lane >> ka.face_shift) == 0u ? (wave << ka.face_shift) + lane : ~0u;
+}
+
 // A triangle record stored with the non-temporal hint: the batch's records
 // far exceed the caches and are read back only after the scatter.
 __device__ __forceinline__ void store_rec_nt(TriRec* p, const TriRec& r) {
@@ -573,9 +587,9 @@ __device__ __forceinline__ void store_rec_nt(TriRec* p, const TriRec& r) {
     gst_nt(q, 2, v4u{r.c.x, r.c.y, r.c.z, r.c.w});
 }
 
+// Face slot g of view V (all 64 lanes of the wave call it).
 template <int T, bool INSIDE>
-__device__ __forceinline__ void setup_face(const KArgs& ka, const Arena& ar, uint32_t g, const ViewDesc& V) {
-    bool active = g < ka.total_faces;
+__device__ __forceinline__ void setup_face(const KArgs& ka, const Arena& ar, uint32_t g, bool active, const ViewDesc& V) {
     bool want_clip = false, binnable = false;
     Rect rc{0, 0, 0, 0};
     if (active) {
@@ -617,7 +631,8 @@ __device__ __forceinline__ void setup_face(const KArgs& ka, const Arena& ar, uin
 // inside (ViewDesc::inside), a branch on a value the wave holds in common.
 template <int T, bool BATCH, bool INSIDE = false>
 __global__ __launch_bounds__(256) void k_setup(KArgs ka, Arena ar) {
-    const uint32_t g = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t g = face_slot(ka);
+    const bool active = g < ka.total_faces;
     if (ar.counters[CNT_ERROR]) return;
     if constexpr (BATCH) {
         const uint32_t vi = wave_view_of(ka.face_bases, ka.nviews, g, ka.total_faces);
@@ -626,14 +641,46 @@ __global__ __launch_bounds__(256) void k_setup(KArgs ka, Arena ar) {
             // the whole wave in one view (the usual case): the view's fields
             // in scalar registers, loaded once for the wave
             const ViewDesc V = wave_uniform(ka.table[v0]);
-            if (INSIDE || V.inside) setup_face<T, true>(ka, ar, g, V);
-            else setup_face<T, false>(ka, ar, g, V);
+            if (INSIDE || V.inside) setup_face<T, true>(ka, ar, g, active, V);
+            else setup_face<T, false>(ka, ar, g, active, V);
         } else {
-            setup_face<T, INSIDE>(ka, ar, g, ka.table[vi]);
+            setup_face<T, INSIDE>(ka, ar, g, active, ka.table[vi]);
         }
     } else {
-        setup_face<T, INSIDE>(ka, ar, g, ka.one);
+        setup_face<T, INSIDE>(ka, ar, g, active, ka.one);
     }
+}
+
+// ---------------------------------------------------------------------------
+// Walks of triangles' pixel rectangles by a wave (k_vis, k_raster): a lane
+// walks at most WALK_CAP pixels of its own rectangle, the rest of every
+// longer one is cut into pieces of WALK_CAP pixels that the wave's lanes take
+// in turn.  What a walker needs of a triangle, per lane, and the first piece
+// of each lane in the wave's numbering:
+constexpr int WALK_CAP = 8;
+struct WalkPieces {
+    float4 e0[64];        // a0, b0, c0, a1
+    float4 e1[64];        // b1, c1, a2, b2
+    float4 e2[64];        // c2, inv_area, z0, z1
+    float4 e3[64];        // z2, bits(fx0), bits(rect), bits(key)
+    uint32_t start[64];
+};
+__device__ __forceinline__ void put_piece(WalkPieces* wp, uint32_t lane, const RasterTri& rt, uint32_t, uint32_t rect,
+                                          uint32_t key) {
+    wp->e0[lane] = make_float4(rt.a0, rt.b0, rt.c0, rt.a1);
+    wp->e1[lane] = make_float4(rt.b1, rt.c1, rt.a2, rt.b2);
+    wp->e2[lane] = make_float4(rt.c2, rt.inv_area, rt.z0, rt.z1);
+    wp->e3[lane] = make_float4(rt.z2, __int_as_float(rt.fx0), __uint_as_float(rect), __uint_as_float(key));
+}
+__device__ __forceinline__ void get_piece(const WalkPieces* wp, const Arena&, uint32_t o, RasterTri& t, uint32_t& rect,
+                                          uint32_t& key) {
+    const float4 f0 = wp->e0[o], f1 = wp->e1[o], f2 = wp->e2[o], f3 = wp->e3[o];
+    t.a0 = f0.x; t.b0 = f0.y; t.c0 = f0.z; t.a1 = f0.w;
+    t.b1 = f1.x; t.c1 = f1.y; t.a2 = f1.z; t.b2 = f1.w;
+    t.c2 = f2.x; t.inv_area = f2.y; t.z0 = f2.z; t.z1 = f2.w;
+    t.z2 = f3.x; t.fx0 = __float_as_int(f3.y);
+    rect = __float_as_uint(f3.z);
+    key = __float_as_uint(f3.w);
 }
 
 // ---------------------------------------------------------------------------
@@ -643,108 +690,160 @@ __global__ __launch_bounds__(256) void k_setup(KArgs ka, Arena ar) {
 // straight into the key buffer, a larger one is queued as work items,
 // faces that cross a plane go to the clipper.
 
-// Faces per lane (their loads issued together: indices, then positions); a
-// 256-thread block covers 256 * VIS_FACES_PER_LANE consecutive faces.  Two
-// per lane measured slower than one on MI355X (fewer waves for small
-// draws, no gain at 1M faces).
-constexpr uint32_t VIS_FACES_PER_LANE = 1;
+// SHARE: where a rectangle of the wave outlasts VIS_SHARE pixels, its lanes
+// would idle while one walks it; then a lane walks WALK_CAP pixels of its own
+// rectangle and the rest goes in pieces of WALK_CAP to all lanes in turn, as
+// in k_raster.  At 1080p k_vis takes 38 us without and 18 with it for 32,000
+// faces, 22 and 10 for 2,000; but 21.2 and 22.1 for a million faces and 23.0
+// and 24.3 for 200,000, whose rectangles are a few pixels.  So the host takes
+// it where the target has at least VIS_SHARE pixels per face.
+constexpr uint32_t VIS_SHARE = 16;
+
+struct VisPieces : WalkPieces {   // rect: x0 | y0 << 16
+    uint32_t size[64];            // w | h << 16
+    uint32_t view[64];
+};
+
+// Pixels [q0, q1) of the rectangle [x0, x0 + w) x [y0, ...) of view V in
+// row-major order: every covered one takes the minimum of its key and flags
+// its bin.
+template <int T>
+__device__ __forceinline__ void vis_span(const Arena& ar, const ViewDesc& V, const RasterTri& rt, int x0, int y0, int w,
+                                         int q0, int q1, uint32_t key, float inv_w) {
+    unsigned long long* vk = ar.vkeys + V.pix_base;
+    // row of q0 as in walk_span (q0 <= 1024, the footprint limit)
+    const int dy = q0 == 0 ? 0 : (int)(((float)q0 + 0.5f) * inv_w);
+    int px = x0 + (q0 - dy * w), py = y0 + dy;
+    uint32_t flagged = ~0u;
+    for (int q = q0; q < q1; ++q) {
+        float al, be, ga, z;
+        if (cover(rt, px, py, al, be, ga, z) && z < INFINITY) {
+            atomicMin(&vk[(size_t)py * (size_t)V.W + (size_t)px], depth_key(z, key));
+            const uint32_t b = V.tile_base + (uint32_t)(py / T * V.tiles_x + px / T);
+            if (b != flagged) ar.tile_count[b] = 1u;
+            flagged = b;
+        }
+        if (++px == x0 + w) {
+            px = x0;
+            ++py;
+        }
+    }
+}
+
+// All 64 lanes call it; on: this lane has a triangle of view vi with
+// rectangle rc.
+template <int T, bool BATCH>
+__device__ __forceinline__ void vis_walk_wave(VisPieces* wp, const KArgs& ka, const Arena& ar, bool on, const RasterTri& rt,
+                                              const Rect& rc, uint32_t vi, uint32_t key) {
+    const uint32_t lane = __lane_id();
+    const int w = on ? rc.x1 - rc.x0 : 0, fp = on ? w * (rc.y1 - rc.y0) : 0;
+    if (on) vis_span<T>(ar, view_at<BATCH>(ka, vi), rt, rc.x0, rc.y0, w, 0, imin(fp, WALK_CAP), key, 0.0f);
+    const uint32_t pieces = fp > WALK_CAP ? (uint32_t)(fp - 1) / WALK_CAP : 0u;
+    const uint32_t incl = wave_incl_scan(pieces), total = __shfl(incl, 63);
+    wp->start[lane] = incl - pieces;
+    if (pieces) {
+        put_piece(wp, lane, rt, 0u, (uint32_t)rc.x0 | ((uint32_t)rc.y0 << 16), key);
+        wp->size[lane] = (uint32_t)w | ((uint32_t)(rc.y1 - rc.y0) << 16);
+        wp->view[lane] = vi;
+    }
+    wave_lds_fence();
+    for (uint32_t j = lane; j < total; j += 64u) {
+        uint32_t o = 0;   // the owner, as in walk_wave
+        for (uint32_t step = 32; step; step >>= 1)
+            if (wp->start[o + step] <= j) o += step;
+        RasterTri t;
+        uint32_t rect, pkey;
+        get_piece(wp, ar, o, t, rect, pkey);
+        const int tw = (int)(wp->size[o] & 0xFFFFu), th = (int)(wp->size[o] >> 16);
+        const int q0 = WALK_CAP * (int)(j - wp->start[o] + 1);
+        vis_span<T>(ar, view_at<BATCH>(ka, BATCH ? wp->view[o] : 0u), t, (int)(rect & 0xFFFFu), (int)(rect >> 16), tw, q0,
+                    imin(q0 + WALK_CAP, tw * th), pkey, 1.0f / (float)tw);
+    }
+}
 
 // INSIDE: the host's bound put the mesh's bounding sphere inside every
 // frustum plane (ka.skip_clip), so every face classifies as inside and the
 // classification is left out (a separate instantiation: a runtime test of the
 // flag is compiled to a select, which still computes it).
-template <int T, bool BATCH, bool INSIDE = false>
-__global__ __launch_bounds__(256) void k_vis(KArgs ka, Arena ar) {
-    constexpr uint32_t F = VIS_FACES_PER_LANE;
+template <int T, bool BATCH, bool INSIDE, bool SHARE>
+__global__ __launch_bounds__(256, BATCH && SHARE ? 6 : 8) void k_vis(KArgs ka, Arena ar) {
     if (ar.counters[CNT_ERROR]) return;
-    uint32_t g[F], vi[F], s[F], face[F], i0[F], i1[F], i2[F];
-    DevGroup G[F];
-    bool act[F];
-#pragma unroll
-    for (uint32_t k = 0; k < F; ++k) {
-        g[k] = blockIdx.x * (256u * F) + k * 256u + threadIdx.x;
-        act[k] = g[k] < ka.total_faces;
-        vi[k] = 0;
-        if constexpr (BATCH) vi[k] = wave_view_of(ka.face_bases, ka.nviews, g[k], ka.total_faces);
-        const ViewDesc& V = view_at<BATCH>(ka, vi[k]);
-        s[k] = g[k] - V.face_base;
-        if (act[k]) {
-            G[k] = group_of(V, s[k]);
-            face[k] = G[k].first + (s[k] - G[k].rank_base);
-            const uint3 ix = gld(reinterpret_cast<const uint3*>(V.idx), face[k]);
-            i0[k] = ix.x;
-            i1[k] = ix.y;
-            i2[k] = ix.z;
-        }
-    }
-    vec3 p0[F], p1[F], p2[F];
-#pragma unroll
-    for (uint32_t k = 0; k < F; ++k) {
-        if (act[k]) {
-            const ViewDesc& V = view_at<BATCH>(ka, vi[k]);
-            p0[k] = load_pos(V.pos, i0[k]);
-            p1[k] = load_pos(V.pos, i1[k]);
-            p2[k] = load_pos(V.pos, i2[k]);
-        }
+    const uint32_t g = face_slot(ka);
+    bool act = g < ka.total_faces;
+    uint32_t vi = 0, s = 0, face = 0;
+    if constexpr (BATCH) vi = wave_view_of(ka.face_bases, ka.nviews, g, ka.total_faces);
+    const ViewDesc& V = view_at<BATCH>(ka, vi);
+    DevGroup G;
+    vec3 p0, p1, p2;
+    if (act) {
+        s = g - V.face_base;
+        G = group_of(V, s);
+        face = G.first + (s - G.rank_base);
+        const uint3 ix = gld(reinterpret_cast<const uint3*>(V.idx), face);
+        p0 = load_pos(V.pos, ix.x);
+        p1 = load_pos(V.pos, ix.y);
+        p2 = load_pos(V.pos, ix.z);
     }
     if constexpr (INSIDE) {
         // faces clearly facing away from the eye are culled before the
         // transform (the pre-test of KArgs::cull_sign; a face within its
         // margin goes on to the exact screen-space test)
-        if (ka.cull_sign != 0.0f) {
+        if (ka.cull_sign != 0.0f && act) {
             const vec3 e = make3(ka.cull_eye[0], ka.cull_eye[1], ka.cull_eye[2]);
             const float le = fabsf(e.x) + fabsf(e.y) + fabsf(e.z);
-#pragma unroll
-            for (uint32_t k = 0; k < F; ++k) {
-                if (!act[k]) continue;
-                const vec3 a = p0[k] - e, b = p1[k] - p0[k], c = p2[k] - p0[k];
-                const float d = ka.cull_sign * dot(a, cross(b, c));
-                const float la = fabsf(a.x) + fabsf(a.y) + fabsf(a.z) + le;
-                const float lb = fabsf(b.x) + fabsf(b.y) + fabsf(b.z), lc = fabsf(c.x) + fabsf(c.y) + fabsf(c.z);
-                if (d < -fmaxf(ka.cull_tau, 1e-3f * la * lb * lc)) act[k] = false;
-            }
+            const vec3 a = p0 - e, b = p1 - p0, c = p2 - p0;
+            const float d = ka.cull_sign * dot(a, cross(b, c));
+            const float la = fabsf(a.x) + fabsf(a.y) + fabsf(a.z) + le;
+            const float lb = fabsf(b.x) + fabsf(b.y) + fabsf(b.z), lc = fabsf(c.x) + fabsf(c.y) + fabsf(c.z);
+            if (d < -fmaxf(ka.cull_tau, 1e-3f * la * lb * lc)) act = false;
         }
     }
-#pragma unroll
-    for (uint32_t k = 0; k < F; ++k) {
-        bool want_clip = false, big = false;
-        TriRec r;
-        uint32_t area = 0;
-        if (act[k]) {
-            const ViewDesc& V = view_at<BATCH>(ka, vi[k]);
-            const vec4 c0 = V.mvp * make4(p0[k], 1.0f);
-            const vec4 c1 = V.mvp * make4(p1[k], 1.0f);
-            const vec4 c2 = V.mvp * make4(p2[k], 1.0f);
-            int cls = CLS_INSIDE;
-            if constexpr (!INSIDE) cls = classify(c0, c1, c2);
-            want_clip = cls == CLS_CLIP;
-            if (cls == CLS_INSIDE) {
-                r = make_rec(c0, c1, c2, V.W, V.H);
-                RasterTri rt;
-                if (!is_backface(r) && raster_setup(r, rt)) {
-                    const Rect rc = screen_rect(rt, V.W, V.H);
-                    if (rc.x0 < rc.x1 && rc.y0 < rc.y1) {
-                        area = (uint32_t)((rc.x1 - rc.x0) * (rc.y1 - rc.y0));
-                        if (area <= (uint32_t)ka.small_footprint) {
-                            vis_raster_rect<T>(ar, V, rt, rc, s[k] * 8u);
-                        } else {
-                            big = true;
-                            r.c.y = s[k] * 8u;
-                            r.c.z = vi[k];
-                            r.c.w = G[k].material & REC_MATERIAL_MASK;
-                        }
+    bool want_clip = false, small = false, big = false;
+    TriRec r;
+    RasterTri rt;
+    Rect rc{0, 0, 0, 0};
+    uint32_t area = 0;
+    if (act) {
+        const vec4 c0 = V.mvp * make4(p0, 1.0f);
+        const vec4 c1 = V.mvp * make4(p1, 1.0f);
+        const vec4 c2 = V.mvp * make4(p2, 1.0f);
+        int cls = CLS_INSIDE;
+        if constexpr (!INSIDE) cls = classify(c0, c1, c2);
+        want_clip = cls == CLS_CLIP;
+        if (cls == CLS_INSIDE) {
+            r = make_rec(c0, c1, c2, V.W, V.H);
+            if (!is_backface(r) && raster_setup(r, rt)) {
+                rc = screen_rect(rt, V.W, V.H);
+                if (rc.x0 < rc.x1 && rc.y0 < rc.y1) {
+                    area = (uint32_t)((rc.x1 - rc.x0) * (rc.y1 - rc.y0));
+                    big = area > (uint32_t)ka.small_footprint;
+                    small = !big;
+                    if (big) {
+                        r.c.y = s * 8u;
+                        r.c.z = vi;
+                        r.c.w = G.material & REC_MATERIAL_MASK;
                     }
                 }
             }
         }
-        const uint32_t cslot = wave_append(&ar.counters[CNT_CLIP_FACES], want_clip);
-        if (want_clip) {
-            if (cslot < ar.cap_clip_faces) ar.clip_faces[cslot] = g[k];
-            else set_error(ar, ERR_CLIP_FACES, CNT_NEED_CLIP_FACES, cslot + 1);
-        }
-        if ((want_clip && ka.skip_clip) || (big && ka.skip_big)) raise_error(ar, ERR_SKIPPED);
-        big_append_wave(ar, big, r, area);
     }
+    if constexpr (SHARE) {
+        __shared__ VisPieces pieces[4];
+        if (__ballot(small && area > VIS_SHARE) == 0ull) {
+            if (small) vis_raster_rect<T>(ar, V, rt, rc, s * 8u);
+        } else {
+            vis_walk_wave<T, BATCH>(pieces + (threadIdx.x >> 6), ka, ar, small, rt, rc, vi, s * 8u);
+        }
+    } else {
+        if (small) vis_raster_rect<T>(ar, V, rt, rc, s * 8u);
+    }
+    const uint32_t cslot = wave_append(&ar.counters[CNT_CLIP_FACES], want_clip);
+    if (want_clip) {
+        if (cslot < ar.cap_clip_faces) ar.clip_faces[cslot] = g;
+        else set_error(ar, ERR_CLIP_FACES, CNT_NEED_CLIP_FACES, cslot + 1);
+    }
+    if ((want_clip && ka.skip_clip) || (big && ka.skip_big)) raise_error(ar, ERR_SKIPPED);
+    big_append_wave(ar, big, r, area);
 }
 
 // ---------------------------------------------------------------------------
@@ -775,13 +874,6 @@ struct ClipWave {
     ClipPoly poly[2];
     ClipPlan plan;
 };
-
-// The wave's LDS writes before its reads of other lanes' entries.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 __device__ __forceinline__ vec4 cv_clip(const float* v) { return make4(v[14], v[15], v[16], v[17]); }
 
@@ -1070,11 +1162,38 @@ __device__ __forceinline__ vec4 shade_winner(const ViewDesc& V, const Arena& ar,
     return shade_at<S>(V, ar, r.c.w, prim, clipped, slot, i0, i1, i2, bar, um);
 }
 
+// A clear that a draw absorbs (its values; on = false: none).
+struct ClearSpec {
+    bool on;
+    uint32_t bgra;
+    float depth;
+};
+
+__device__ __forceinline__ void clear_pixel(const ViewDesc& V, size_t pix, const ClearSpec& cs) {
+    gst(V.color, pix, cs.bgra);
+    gst(V.depth, pix, cs.depth);
+    if (V.ids) gst(V.ids, pix, 0xFFFFFFFFu);
+}
+
+// Pixel p (row-major) of the bin at (ox, oy), if it lies on the screen.
+template <int T>
+__device__ __forceinline__ void clear_bin_pixel(const ViewDesc& V, int ox, int oy, int p, const ClearSpec& cs) {
+    const int px = ox + (p % T), py = oy + (p / T);
+    if (px < V.W && py < V.H) clear_pixel(V, (size_t)py * (size_t)V.W + (size_t)px, cs);
+}
+
+// Pixels p0, p0 + step, ... of a bin without keys, when the draw absorbs a
+// clear.
+template <int T>
+__device__ __forceinline__ void clear_bin(const ViewDesc& V, int ox, int oy, const ClearSpec& cs, int p0, int step) {
+    for (int p = p0; p < T * T; p += step) clear_bin_pixel<T>(V, ox, oy, p, cs);
+}
+
 // known: the depth plane is known to hold known_depth here (a clear written
 // just before the draw); else it is loaded.
 template <class S>
 __device__ __forceinline__ void resolve_pixel(const ViewDesc& V, const Arena& ar, unsigned long long k, int px, int py,
-                                              bool known, float known_depth, const DevMaterial* um) {
+                                              bool known, float known_depth, const ClearSpec& cs, const DevMaterial* um) {
     const uint32_t key = (uint32_t)k;
     const uint32_t rank = key >> 3, j = key & 7u;
     TriRec r = ar.rec[V.face_base + rank];
@@ -1090,7 +1209,10 @@ __device__ __forceinline__ void resolve_pixel(const ViewDesc& V, const Arena& ar
     float al, be, ga, z;
     cover(rt, px, py, al, be, ga, z);
     const size_t pix = (size_t)py * (size_t)V.W + (size_t)px;
-    if (!(z < (known ? known_depth : gld(V.depth, pix)))) return;   // reference mergeTileResults: strict less
+    if (!(z < (known ? known_depth : gld(V.depth, pix)))) {   // reference mergeTileResults: strict less
+        if (cs.on) clear_pixel(V, pix, cs);
+        return;
+    }
     const vec4 col = shade_winner<S>(V, ar, r, slot, clipped, rank, make3(al, be, ga), um);
     gst_nt(V.depth, pix, z);
     gst_nt(V.color, pix, pack_bgra(col));
@@ -1102,13 +1224,14 @@ template <int T, int NT, class S>
 // starts at zero), so that every wave shades covered pixels only: a bin on
 // a silhouette takes fewer shading rounds than one pass over its rows.
 __device__ __forceinline__ void resolve_tile(const ViewDesc& V, const Arena& ar, const unsigned long long* keys,
-                                             int ox, int oy, bool known, float known_depth, uint16_t* plist,
-                                             uint32_t* ncov) {
+                                             int ox, int oy, bool known, float known_depth, const ClearSpec& cs,
+                                             uint16_t* plist, uint32_t* ncov) {
     static_assert((T * T) % 64 == 0 && NT % 64 == 0, "every wave makes the same number of passes");
     for (int p = threadIdx.x; p < T * T; p += NT) {
         const bool cov = keys[p] != EMPTY_KEY;
         const uint32_t slot = wave_append(ncov, cov);
         if (cov) plist[slot] = (uint16_t)p;
+        else if (cs.on) clear_bin_pixel<T>(V, ox, oy, p, cs);
     }
     __syncthreads();
     const uint32_t n = *ncov;
@@ -1118,12 +1241,12 @@ __device__ __forceinline__ void resolve_tile(const ViewDesc& V, const Arena& ar,
         const DevMaterial um = wave_uniform(gld(V.materials, V.g0.material & REC_MATERIAL_MASK));
         for (uint32_t i = threadIdx.x; i < n; i += NT) {
             const int p = plist[i];
-            resolve_pixel<S>(V, ar, keys[p], ox + (p % T), oy + (p / T), known, known_depth, &um);
+            resolve_pixel<S>(V, ar, keys[p], ox + (p % T), oy + (p / T), known, known_depth, cs, &um);
         }
     } else {
         for (uint32_t i = threadIdx.x; i < n; i += NT) {
             const int p = plist[i];
-            resolve_pixel<S>(V, ar, keys[p], ox + (p % T), oy + (p / T), known, known_depth, nullptr);
+            resolve_pixel<S>(V, ar, keys[p], ox + (p % T), oy + (p / T), known, known_depth, cs, nullptr);
         }
     }
 }
@@ -1139,17 +1262,18 @@ template <> struct ShaderOf<SHADER_FLAT_COLOR> { using type = FlatColorShader; }
 
 template <int T, int NT, int SK>
 __device__ __forceinline__ void resolve_tile_kind(const ViewDesc& V, const Arena& ar, const unsigned long long* keys,
-                                                  int ox, int oy, bool kn, float kd, uint16_t* pl, uint32_t* nc) {
+                                                  int ox, int oy, bool kn, float kd, const ClearSpec& cs, uint16_t* pl,
+                                                  uint32_t* nc) {
     if constexpr (SK >= 0) {
-        resolve_tile<T, NT, typename ShaderOf<SK>::type>(V, ar, keys, ox, oy, kn, kd, pl, nc);
+        resolve_tile<T, NT, typename ShaderOf<SK>::type>(V, ar, keys, ox, oy, kn, kd, cs, pl, nc);
     } else {
         switch (V.u.kind) {
-        case SHADER_FLAT: resolve_tile<T, NT, FlatShader>(V, ar, keys, ox, oy, kn, kd, pl, nc); break;
-        case SHADER_PHONG: resolve_tile<T, NT, PhongShader>(V, ar, keys, ox, oy, kn, kd, pl, nc); break;
-        case SHADER_PBR: resolve_tile<T, NT, PBRShader>(V, ar, keys, ox, oy, kn, kd, pl, nc); break;
-        case SHADER_GOURAUD: resolve_tile<T, NT, GouraudShader>(V, ar, keys, ox, oy, kn, kd, pl, nc); break;
-        case SHADER_PHONG_POINT: resolve_tile<T, NT, PhongPointShader>(V, ar, keys, ox, oy, kn, kd, pl, nc); break;
-        default: resolve_tile<T, NT, FlatColorShader>(V, ar, keys, ox, oy, kn, kd, pl, nc); break;
+        case SHADER_FLAT: resolve_tile<T, NT, FlatShader>(V, ar, keys, ox, oy, kn, kd, cs, pl, nc); break;
+        case SHADER_PHONG: resolve_tile<T, NT, PhongShader>(V, ar, keys, ox, oy, kn, kd, cs, pl, nc); break;
+        case SHADER_PBR: resolve_tile<T, NT, PBRShader>(V, ar, keys, ox, oy, kn, kd, cs, pl, nc); break;
+        case SHADER_GOURAUD: resolve_tile<T, NT, GouraudShader>(V, ar, keys, ox, oy, kn, kd, cs, pl, nc); break;
+        case SHADER_PHONG_POINT: resolve_tile<T, NT, PhongPointShader>(V, ar, keys, ox, oy, kn, kd, cs, pl, nc); break;
+        default: resolve_tile<T, NT, FlatColorShader>(V, ar, keys, ox, oy, kn, kd, cs, pl, nc); break;
         }
     }
 }
@@ -1162,8 +1286,6 @@ __device__ __forceinline__ void resolve_tile_kind(const ViewDesc& V, const Arena
 // 42% of the lane slots did work.  So a lane walks at most WALK_CAP pixels
 // of its own rectangle; the rest of every longer rectangle is cut into
 // pieces of WALK_CAP pixels that the wave's lanes then take in turn.
-
-constexpr int WALK_CAP = 8;
 
 // Pixels [q0, q1) of the rectangle [x0, x0 + w) x [y0, ...) in row-major
 // order; every covered pixel takes the minimum of its key.
@@ -1194,13 +1316,6 @@ __device__ __forceinline__ void walk_span(const RasterTri& rt, int x0, int y0, i
 //               the walker loads the record again and repeats the edge setup
 //               (the same operations on the same bits), for a raster kernel
 //               whose occupancy its LDS would otherwise bound.
-struct WalkPieces {
-    float4 e0[64];        // a0, b0, c0, a1
-    float4 e1[64];        // b1, c1, a2, b2
-    float4 e2[64];        // c2, inv_area, z0, z1
-    float4 e3[64];        // z2, bits(fx0), bits(rect), bits(key)
-    uint32_t start[64];
-};
 struct WalkRefs {
     uint32_t ref[64];
     uint32_t rect[64];
@@ -1208,23 +1323,6 @@ struct WalkRefs {
 };
 // rect: x0 | y0 << 8 | w << 16 | h << 24, in bin coordinates
 
-__device__ __forceinline__ void put_piece(WalkPieces* wp, uint32_t lane, const RasterTri& rt, uint32_t, uint32_t rect,
-                                          uint32_t key) {
-    wp->e0[lane] = make_float4(rt.a0, rt.b0, rt.c0, rt.a1);
-    wp->e1[lane] = make_float4(rt.b1, rt.c1, rt.a2, rt.b2);
-    wp->e2[lane] = make_float4(rt.c2, rt.inv_area, rt.z0, rt.z1);
-    wp->e3[lane] = make_float4(rt.z2, __int_as_float(rt.fx0), __uint_as_float(rect), __uint_as_float(key));
-}
-__device__ __forceinline__ void get_piece(const WalkPieces* wp, const Arena&, uint32_t o, RasterTri& t, uint32_t& rect,
-                                          uint32_t& key) {
-    const float4 f0 = wp->e0[o], f1 = wp->e1[o], f2 = wp->e2[o], f3 = wp->e3[o];
-    t.a0 = f0.x; t.b0 = f0.y; t.c0 = f0.z; t.a1 = f0.w;
-    t.b1 = f1.x; t.c1 = f1.y; t.a2 = f1.z; t.b2 = f1.w;
-    t.c2 = f2.x; t.inv_area = f2.y; t.z0 = f2.z; t.z1 = f2.w;
-    t.z2 = f3.x; t.fx0 = __float_as_int(f3.y);
-    rect = __float_as_uint(f3.z);
-    key = __float_as_uint(f3.w);
-}
 __device__ __forceinline__ void put_piece(WalkRefs* wp, uint32_t lane, const RasterTri&, uint32_t ref, uint32_t rect,
                                           uint32_t) {
     wp->ref[lane] = ref;
@@ -1288,7 +1386,7 @@ __device__ __forceinline__ const ViewDesc& bin_view(const KArgs& ka, const ViewD
 // every per-pixel read of its uniforms and pointers is an LDS read.
 template <int T, int NT, bool BATCH, int SK>
 __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uint32_t t, uint32_t n, unsigned long long* keys,
-                                           uint32_t* bigq, uint32_t& nbig, uint16_t* plist, ViewDesc* sview,
+                                           uint32_t& ncov, uint16_t* plist, ViewDesc* sview,
                                            typename PiecesOf<SK>::type* pieces) {
     if constexpr (BATCH) {
         const uint32_t vi = ka.tile_views[t];
@@ -1297,7 +1395,7 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
             reinterpret_cast<uint32_t*>(sview)[i] = gld(src, i);
     }
     for (int p = threadIdx.x; p < T * T; p += NT) keys[p] = EMPTY_KEY;
-    if (threadIdx.x == 0) nbig = 0;
+    if (threadIdx.x == 0) ncov = 0;
     __syncthreads();
     const ViewDesc& V = bin_view<BATCH>(ka, sview);
     const uint32_t local = t - V.tile_base;
@@ -1306,9 +1404,12 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
     // every wave has read n: the count is consumed, leave it zero for the next frame
     if (threadIdx.x == 0) ar.tile_count[t] = 0;
 
+    // entries go to the waves in turn, so that a bin with fewer entries than
+    // the workgroup has lanes keeps every wave at work
     typename PiecesOf<SK>::type* wp = pieces + (threadIdx.x >> 6);
+    const uint32_t first = (threadIdx.x & 63u) * (NT / 64) + (threadIdx.x >> 6);
     for (uint32_t b0 = 0; b0 < n; b0 += NT) {
-        const uint32_t i = b0 + threadIdx.x;
+        const uint32_t i = b0 + first;
         RasterTri rt;
         int x0 = 0, y0 = 0, w = 0, h = 0;
         uint32_t key = 0, ref = 0;
@@ -1320,49 +1421,28 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
                 y0 = imax(oy, rt.fy0);
                 w = imin(ex, rt.cx1) - x0;
                 h = imin(ey, rt.cy1) - y0;
-                if (w <= 0 || h <= 0) {
-                    w = h = 0;
-                } else if (w * h > ka.small_footprint) {
-                    bigq[atomicAdd(&nbig, 1u)] = ref;
-                    w = h = 0;
-                }
+                if (w <= 0 || h <= 0) w = h = 0;
                 key = r.c.y;
             }
         }
         walk_wave<T>(wp, ar, rt, ref, x0 - ox, y0 - oy, w, h, key, keys, ox, oy);
-        __syncthreads();
-        const uint32_t nb = nbig;
-        for (uint32_t q = 0; q < nb; ++q) {
-            const TriRec r = rec_of(ar, bigq[q]);
-            RasterTri rt;
-            raster_setup(r, rt);
-            const int x0 = imax(ox, rt.fx0), x1 = imin(ex, rt.cx1);
-            const int y0 = imax(oy, rt.fy0), y1 = imin(ey, rt.cy1);
-            const int w = x1 - x0, np = w * (y1 - y0);
-            const uint32_t key = r.c.y;
-            const float inv_w = 1.0f / (float)w;
-            for (int p = threadIdx.x; p < np; p += NT) {
-                // p / w as in walk_span (p < 2^16, w <= 32)
-                const int dy = (int)(((float)p + 0.5f) * inv_w);
-                const int px = x0 + (p - dy * w), py = y0 + dy;
-                float al, be, ga, z;
-                if (cover(rt, px, py, al, be, ga, z) && z < INFINITY)
-                    atomicMin(&keys[(py - oy) * T + (px - ox)], depth_key(z, key));
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) nbig = 0;
-        __syncthreads();
+        wave_lds_fence();   // the pieces are read before the next entries' are written
     }
+    __syncthreads();
 
     // every entry has been read: leave the chunk table empty as well
     if (threadIdx.x > 0 && threadIdx.x <= bin_slot(ar, n - 1).level) ar.bin_chunks[(size_t)t * BIN_LEVELS + threadIdx.x] = 0;
 
-    // nbig is zero again here: it counts the covered pixels
-    resolve_tile_kind<T, NT, SK>(V, ar, keys, ox, oy, ka.depth_is_clear != 0, ka.clear_depth, plist, &nbig);
+    // a batch's clear is a pass of its own before the frame (k_clear_views)
+    const ClearSpec cs{!BATCH && ka.clear != 0, ka.clear_bgra, ka.clear_depth};
+    resolve_tile_kind<T, NT, SK>(V, ar, keys, ox, oy, cs.on || (BATCH && ka.depth_is_clear != 0), ka.clear_depth, cs,
+                                 plist, &ncov);
 }
 
-// One workgroup per bin; an empty bin's leaves after one load.  Workgroups
+// One workgroup per bin; an empty bin's leaves after one load, or after
+// writing the clear that a plain draw absorbs (ka.clear: a pass of its own
+// took 6 us of a 1080p frame, and as long again to start; the 256-view batch,
+// mostly empty bins, keeps its streaming pass).  Workgroups
 // are dispatched to the 8 XCDs round-robin, so block ids are permuted to give
 // an XCD runs of XCD_RUN neighbouring bins, which share triangles, vertices
 // and texels in its L2; short runs, because the bins of a frame are not
@@ -1389,13 +1469,14 @@ constexpr int raster_min_waves(int sk) {
 template <int T, int NT, bool BATCH, int SK>
 __global__ __launch_bounds__(NT, raster_min_waves(SK)) void k_raster(KArgs ka, Arena ar) {
     __shared__ unsigned long long keys[T * T];
-    __shared__ uint32_t bigq[NT];
     __shared__ uint16_t plist[T * T];
-    __shared__ uint32_t nbig;
+    __shared__ uint32_t ncov;
     __shared__ ViewDesc sview[1];
     __shared__ typename PiecesOf<SK>::type pieces[NT / 64];
-    if (ar.counters[CNT_ERROR]) return;
-    if (blockIdx.x == 0) {
+    const bool failed = ar.counters[CNT_ERROR] != 0u;
+    const bool clear = !BATCH && ka.clear != 0;
+    if (failed && !clear) return;
+    if (blockIdx.x == 0 && !failed) {
         // the per-frame counters were last needed by k_clip
         if (threadIdx.x == 0) {
             ar.counters[CNT_CLIP_FACES] = 0;
@@ -1406,9 +1487,18 @@ __global__ __launch_bounds__(NT, raster_min_waves(SK)) void k_raster(KArgs ka, A
     const uint32_t x = blockIdx.x % NUM_XCD, j = blockIdx.x / NUM_XCD;
     const uint32_t t = (j / XCD_RUN * NUM_XCD + x) * XCD_RUN + j % XCD_RUN;
     if (t >= ka.total_tiles) return;
-    const uint32_t n = ar.tile_count[t];
-    if (n == 0u) return;
-    raster_bin<T, NT, BATCH, SK>(ka, ar, t, n, keys, bigq, nbig, plist, sview, pieces);
+    const uint32_t n = failed ? 0u : ar.tile_count[t];
+    if (n == 0u) {
+        // an empty bin, or a failed frame: only the clear, if the draw absorbs
+        // one, as a separate clear pass would have
+        if (clear) {
+            const ViewDesc& V = ka.one;
+            const int tx = (int)(t % (uint32_t)V.tiles_x), ty = (int)(t / (uint32_t)V.tiles_x);
+            clear_bin<T>(V, tx * T, ty * T, ClearSpec{true, ka.clear_bgra, ka.clear_depth}, (int)threadIdx.x, NT);
+        }
+        return;
+    }
+    raster_bin<T, NT, BATCH, SK>(ka, ar, t, n, keys, ncov, plist, sview, pieces);
 }
 
 // ---------------------------------------------------------------------------
@@ -1545,19 +1635,6 @@ __device__ __forceinline__ bool resolve_vis_pixel(const ViewDesc& V, const Arena
     return true;
 }
 
-// A clear that a draw absorbs (its values; on = false: none).
-struct ClearSpec {
-    bool on;
-    uint32_t bgra;
-    float depth;
-};
-
-__device__ __forceinline__ void clear_pixel(const ViewDesc& V, size_t pix, const ClearSpec& cs) {
-    gst(V.color, pix, cs.bgra);
-    gst(V.depth, pix, cs.depth);
-    if (V.ids) gst(V.ids, pix, 0xFFFFFFFFu);
-}
-
 // Pixels p0, p0 + step, ... of the bin at (ox, oy), row-major.
 template <int T, class S, bool VARY, bool INSIDE>
 __device__ __forceinline__ void resolve_vis_tile(const ViewDesc& V, const Arena& ar, int ox, int oy,
@@ -1574,18 +1651,6 @@ __device__ __forceinline__ void resolve_vis_tile(const ViewDesc& V, const Arena&
             drawn = resolve_vis_pixel<S, VARY, INSIDE>(V, ar, k, px, py, pix, cs.on ? cs.depth : gld(V.depth, pix));
         }
         if (!drawn && cs.on) clear_pixel(V, pix, cs);
-    }
-}
-
-// Pixels p0, p0 + step, ... of a bin without keys, when the draw absorbs a
-// clear.
-template <int T>
-__device__ __forceinline__ void clear_vis_tile(const ViewDesc& V, int ox, int oy, const ClearSpec& cs, int p0,
-                                               int step) {
-    for (int p = p0; p < T * T; p += step) {
-        const int px = ox + (p % T), py = oy + (p / T);
-        if (px >= V.W || py >= V.H) continue;
-        clear_pixel(V, (size_t)py * (size_t)V.W + (size_t)px, cs);
     }
 }
 
@@ -1648,7 +1713,7 @@ __global__ __launch_bounds__(256) void k_resolve(KArgs ka, Arena ar) {
             const uint32_t local = t - V.tile_base;
             const int ox = (int)(local % (uint32_t)V.tiles_x) * T, oy = (int)(local / (uint32_t)V.tiles_x) * T;
             if (keys) resolve_vis_tile_kind<T, SK, BATCH, INSIDE>(V, ar, ox, oy, cs, (int)__lane_id(), 64);
-            else clear_vis_tile<T>(V, ox, oy, cs, (int)__lane_id(), 64);
+            else clear_bin<T>(V, ox, oy, cs, (int)__lane_id(), 64);
         }
     } else {
         // one workgroup (four waves, a pixel or more per thread) per bin:
@@ -1665,7 +1730,7 @@ __global__ __launch_bounds__(256) void k_resolve(KArgs ka, Arena ar) {
             const uint32_t local = t - V.tile_base;
             const int ox = (int)(local % (uint32_t)V.tiles_x) * T, oy = (int)(local / (uint32_t)V.tiles_x) * T;
             if (keys) resolve_vis_tile_kind<T, SK, BATCH, INSIDE>(V, ar, ox, oy, cs, (int)threadIdx.x, 256);
-            else clear_vis_tile<T>(V, ox, oy, cs, (int)threadIdx.x, 256);
+            else clear_bin<T>(V, ox, oy, cs, (int)threadIdx.x, 256);
         }
     }
 }
@@ -2010,11 +2075,16 @@ template <int T, bool IDS, bool INSIDE> struct ShadeK {
         static constexpr auto fn = &k_shade<T, (SK < 0 ? SHADER_FLAT_COLOR : SK), IDS, INSIDE>;
     };
 };
+// only a batch's views may differ in their shader kind
 template <int T, bool BATCH, bool INSIDE> struct ResolveK {
-    template <int SK> struct K { static constexpr auto fn = &k_resolve<T, BATCH, SK, INSIDE>; };
+    template <int SK> struct K {
+        static constexpr auto fn = &k_resolve<T, BATCH, (!BATCH && SK < 0 ? SHADER_FLAT_COLOR : SK), INSIDE>;
+    };
 };
 template <int T, int NT, bool BATCH> struct RasterK {
-    template <int SK> struct K { static constexpr auto fn = &k_raster<T, NT, BATCH, SK>; };
+    template <int SK> struct K {
+        static constexpr auto fn = &k_raster<T, NT, BATCH, (!BATCH && SK < 0 ? SHADER_FLAT_COLOR : SK)>;
+    };
 };
 
 // k_shade, then (after the wait) k_finish4 or k_finish: stages 3 and 4.
@@ -2035,15 +2105,30 @@ static hipError_t launch_two_pass(const KArgs& ka, const Arena& ar, hipStream_t 
     return hipGetLastError();
 }
 
+// At most this many faces go 16 to a wave (2,048 waves, two to a SIMD) instead
+// of 64.
+constexpr uint32_t FEW_FACES = 32768;
+
+// Workgroups (four waves) of the passes over faces.
+static uint32_t face_blocks(const KArgs& ka) {
+    const uint32_t per = 4u << ka.face_shift;
+    return (uint32_t)(((uint64_t)ka.total_faces + per - 1) / per);
+}
+
 // Visibility mode: stage 0 k_vis, 1 k_clip, 2 k_big, then either 4
 // k_resolve or (two-pass) 3 k_shade and 4 k_finish.
 template <int T, bool BATCH>
 static hipError_t launch_vis_t(const KArgs& ka, const Arena& ar, hipStream_t st, StageEvents* ev, const FbWait& wait) {
     t_phases = kVisPhases;
-    const uint32_t vis_blocks = (ka.total_faces + 256u * VIS_FACES_PER_LANE - 1) / (256u * VIS_FACES_PER_LANE);
+    const uint32_t vis_blocks = face_blocks(ka);
     if (vis_blocks) {
-        if (!BATCH && ka.skip_clip) stage_launch1(k_vis<T, false, true>, dim3(vis_blocks), dim3(256), st, ev, 0, ka, ar);
-        else stage_launch1(k_vis<T, BATCH>, dim3(vis_blocks), dim3(256), st, ev, 0, ka, ar);
+        const bool share = (uint64_t)ka.total_faces * VIS_SHARE <= ka.total_pixels;
+        if (!BATCH && ka.skip_clip)
+            stage_launch1(share ? &k_vis<T, false, true, true> : &k_vis<T, false, true, false>, dim3(vis_blocks), dim3(256), st,
+                          ev, 0, ka, ar);
+        else
+            stage_launch1(share ? &k_vis<T, BATCH, false, true> : &k_vis<T, BATCH, false, false>, dim3(vis_blocks), dim3(256), st,
+                          ev, 0, ka, ar);
     }
     // passes the host showed to have no work are not launched
     if (BATCH || !ka.skip_clip) stage_launch1(k_clip<T, BATCH, true>, dim3(CLIP_BLOCKS), dim3(64 * CLIP_WAVES), st, ev, 1, ka, ar);
@@ -2072,7 +2157,7 @@ static hipError_t launch_frame_t(const KArgs& ka, const Arena& ar, hipStream_t s
     if (ka.mode == RASTER_VISIBILITY) return launch_vis_t<T, BATCH>(ka, ar, st, ev, wait);
     t_phases = kBinnedPhases;
     const uint32_t ntiles = ka.total_tiles;
-    const uint32_t setup_blocks = (ka.total_faces + 255) / 256;
+    const uint32_t setup_blocks = face_blocks(ka);
     if (setup_blocks) {
         if (ka.skip_clip) stage_launch1(k_setup<T, BATCH, true>, dim3(setup_blocks), dim3(256), st, ev, 0, ka, ar);
         else stage_launch1(k_setup<T, BATCH>, dim3(setup_blocks), dim3(256), st, ev, 0, ka, ar);
@@ -2086,13 +2171,22 @@ static hipError_t launch_frame_t(const KArgs& ka, const Arena& ar, hipStream_t s
     return hipGetLastError();
 }
 
+// Threads per bin of k_raster: ka.raster_threads, or more.  A bin's pixels
+// are shaded by its workgroup alone, and few of a single view's bins hold
+// most of its pixels, so bins of 16 or 32 px take 256 threads (a 1M-triangle
+// 1080p frame: 97 us at 64, 57 at 128, 39 at 256; a PBR object at 1241x719:
+// 37, 24, 18).  Where there is little to shade per pixel (one colour per
+// face) or a batch's many views fill the chip, 128 (a 400k-triangle soup at
+// 1080p: 49, 42, 59 us; 24 mixed views at 16 px: 130, 82, 99).  A bin of 8 px
+// has 64 pixels.
 template <int T, bool BATCH>
 static hipError_t launch_frame_nt(const KArgs& ka, const Arena& ar, hipStream_t st, StageEvents* ev, const FbWait& w) {
-    switch (ka.raster_threads) {
-    case 64: return launch_frame_t<T, 64, BATCH>(ka, ar, st, ev, w);
-    case 128: return launch_frame_t<T, 128, BATCH>(ka, ar, st, ev, w);
-    default: return launch_frame_t<T, 256, BATCH>(ka, ar, st, ev, w);
+    if constexpr (T == 8) {
+        if (ka.raster_threads <= 64) return launch_frame_t<T, 64, BATCH>(ka, ar, st, ev, w);
     }
+    const int least = T == 8 || BATCH || ka.shader == SHADER_FLAT_COLOR ? 128 : 256;
+    return imax(least, ka.raster_threads) <= 128 ? launch_frame_t<T, 128, BATCH>(ka, ar, st, ev, w)
+                                                 : launch_frame_t<T, 256, BATCH>(ka, ar, st, ev, w);
 }
 
 template <bool BATCH>
@@ -2104,7 +2198,9 @@ static hipError_t launch_frame_b(const KArgs& ka, const Arena& ar, hipStream_t s
     }
 }
 
-hipError_t launch_frame(const KArgs& ka, const Arena& ar, hipStream_t st, StageEvents* ev, const FbWait& wait) {
+hipError_t launch_frame(const KArgs& args, const Arena& ar, hipStream_t st, StageEvents* ev, const FbWait& wait) {
+    KArgs ka = args;
+    ka.face_shift = ka.total_faces <= FEW_FACES ? 4 : 6;
     // stage 5: a batch's vertex stage once per vertex of each shared mesh,
     // before the resolve reads it
     if (ka.table && ka.vary_total)

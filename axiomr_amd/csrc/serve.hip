@@ -154,20 +154,16 @@ public:
         ka.one = L.h_views[0];
         hipStream_t st = L.fa.stream;
         hipError_t e = hipSuccess;
-        // every request starts from a cleared framebuffer; in visibility mode
-        // the resolve pass writes that clear (k_resolve, ka.clear)
-        const bool absorb = mode_ == RASTER_VISIBILITY;
+        // every request starts from a cleared framebuffer; the pass that writes
+        // the frame writes that clear (ka.clear), except for a binned batch
+        const bool absorb = mode_ == RASTER_VISIBILITY || n == 1;
         if (absorb) {
             ka.clear = 1;
             ka.clear_bgra = cfg_.clear_bgra;
             ka.clear_depth = __builtin_huge_valf();
         }
-        if (n == 1) {
-            // one request: the plain path, no tables
-            const ViewDesc& v = L.h_views[0];
-            if (!absorb)
-                e = launch_clear(v.color, v.depth, v.ids, (size_t)v.W * v.H, cfg_.clear_bgra, __builtin_huge_valf(), st);
-        } else {
+        // one request: the plain path, no tables
+        if (n > 1) {
             uint32_t t = 0;
             for (uint32_t i = 0; i < n; ++i)
                 for (uint32_t k = L.h_bases[stride + i]; k < L.h_bases[stride + i + 1]; ++k) L.h_tile_views[t++] = i;

@@ -109,11 +109,13 @@ typedef struct axr_draw_params {
  * tiles. */
 typedef struct axr_config {
     int32_t tile_size;           /* GPU bin edge: 8, 16 or 32 pixels (default 16) */
-    int32_t raster_threads;      /* threads per bin workgroup: 64, 128 or 256 (default 64) */
+    int32_t raster_threads;      /* threads per bin workgroup: 64, 128 or 256 (default 64); bins of
+                                    16 and 32 px take at least 128, a single view's mostly 256 */
     int32_t bin_capacity;        /* 64..1024 (default 128); no effect: a bin's storage is
                                     sized from the draw's faces and bins, and grows */
-    int32_t small_footprint;     /* triangles covering at most this many pixels of a bin are
-                                    walked by one lane, 1..1024 (default 12) */
+    int32_t small_footprint;     /* visibility mode: triangles covering at most this many pixels
+                                    are walked by the setup, larger ones become work items,
+                                    1..1024 (default 12) */
     int32_t raster_mode;         /* AXR_RASTER_BINNED (default) or AXR_RASTER_VISIBILITY */
     int32_t reserved[3];
 } axr_config;
@@ -180,9 +182,8 @@ int axr_fb_create(axr_ctx* ctx, int w, int h, int with_ids, axr_fb** out);
 int axr_fb_destroy(axr_fb* fb);
 /* reference Framebuffer::clearColor/clearDepth (src/framebuffer.cpp:26-42):
  * bgra packed as a<<24 | r<<16 | g<<8 | b.  Not synchronous: the clear is
- * recorded, and the next axr_draw in visibility mode writes it in the same
- * pass that writes the frame (no pass of its own); a read-back, a binned
- * draw or a batch writes it first.  The pixels are always as if the clear
+ * recorded, and the next axr_draw writes it in the same pass that writes the
+ * frame (no pass of its own); a read-back or a batch writes it first.  The pixels are always as if the clear
  * had run at this call. */
 int axr_fb_clear(axr_fb* fb, uint32_t bgra, float depth);
 /* Synchronous read-back; any pointer may be null. */
