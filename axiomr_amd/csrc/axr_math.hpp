@@ -86,15 +86,16 @@ AXR_HD float sclamp(float v, float lo, float hi) { return (v < lo) ? lo : ((hi <
 // the rest take the division.  Four such reciprocals per triangle setup
 // cost a quarter of the instructions of the division sequence.
 #if defined(__HIP_DEVICE_COMPILE__)
+AXR_HD float rcp_rn_normal(float x) {   // exponent in that range
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
 AXR_HD float rcp_rn(float x) {
     const uint32_t ex = (__float_as_uint(x) >> 23) & 0xFFu;
-    if (ex - 2u <= 250u) {
-        const float r = __builtin_amdgcn_rcpf(x);
-        return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
-    }
-    return 1.0f / x;
+    return ex - 2u <= 250u ? rcp_rn_normal(x) : 1.0f / x;
 }
 #else
+AXR_HD float rcp_rn_normal(float x) { return 1.0f / x; }
 AXR_HD float rcp_rn(float x) { return 1.0f / x; }
 #endif
 AXR_HD int imin(int a, int b) { return (b < a) ? b : a; }

@@ -464,6 +464,10 @@ PassSkips pass_skips(const axr_mesh* m, const mat4& mvp, int W, int H, int footp
         for (int c = 0; c < 4; ++c) q[c] = r[3][c] + sg * r[axis][c];
         if (!(at_center(q) - slope(q) * m->radius > margin(q))) return s;
     }
+    // the kernels' INSIDE variants also rely on w's range (no clamping at
+    // 1e-6, no reciprocal outside the refined range)
+    const double w_mid = at_center(r[3]), w_span = slope(r[3]) * m->radius + margin(r[3]);
+    if (!(w_mid - w_span > 1e-5 && w_mid + w_span < 1e30)) return s;
     s.clip = true;
     // The back-face pre-test (k_vis): the eye in object space is where rows
     // x, y and w of the transform vanish, A3 e + a = 0 (A3: those rows'

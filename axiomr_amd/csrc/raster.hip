@@ -193,8 +193,14 @@ __device__ __forceinline__ int classify(const vec4& a, const vec4& b, const vec4
 
 // Triangle setup: screen position (y up) and ndc z of one corner
 // (reference tiled_pipeline.cpp:59-65).
+// INSIDE, here and in raster_setup: the host's bound (pass_skips) put the
+// mesh inside every frustum plane with w in [1e-5, 1e30], so w is not clamped
+// and lies in the exponent range of the refined reciprocal, and no screen
+// coordinate is NaN or outside int range: the same bits with some 40 fewer
+// instructions a face.
+template <bool INSIDE>
 __device__ __forceinline__ void to_screen(const vec4& c, int W, int H, float& sx, float& sy, float& z) {
-    float invW = rcp_rn(clampW(c.w));
+    float invW = INSIDE ? rcp_rn_normal(c.w) : rcp_rn(clampW(c.w));
     z = c.z * invW;
     sx = (((c.x * invW) + 1.0f) * 0.5f) * (float)W;
     sy = (((c.y * invW) + 1.0f) * 0.5f) * (float)H;
@@ -207,12 +213,13 @@ __device__ __forceinline__ bool is_backface(const TriRec& r) {
     return (dx1 * dy2 - dx2 * dy1) < 0;
 }
 
+template <bool INSIDE = false>
 __device__ __forceinline__ TriRec make_rec(const vec4& c0, const vec4& c1, const vec4& c2, int W, int H) {
     TriRec r;
     float z0, z1, z2;
-    to_screen(c0, W, H, r.a.x, r.a.y, z0);
-    to_screen(c1, W, H, r.a.z, r.a.w, z1);
-    to_screen(c2, W, H, r.b.x, r.b.y, z2);
+    to_screen<INSIDE>(c0, W, H, r.a.x, r.a.y, z0);
+    to_screen<INSIDE>(c1, W, H, r.a.z, r.a.w, z1);
+    to_screen<INSIDE>(c2, W, H, r.b.x, r.b.y, z2);
     r.b.z = z0; r.b.w = z1;
     r.c.x = __float_as_uint(z2);
     return r;
@@ -227,17 +234,30 @@ struct RasterTri {
     int fx0, fy0, cx1, cy1;   // (int)floor(min), (int)ceil(max)
 };
 
+// The largest float below 1e-12: the reference's area test compares in double
+// ((double)area < 1e-12), which for a float is area <= this.
+constexpr float AREA_NONE = 9.99999996e-13f;
+static_assert((double)AREA_NONE < 1.0e-12 && (double)1.00000011e-12f > 1.0e-12, "neighbours of 1e-12");
+
+template <bool INSIDE = false>
 __device__ __forceinline__ bool raster_setup(const TriRec& r, RasterTri& t) {
     const float x0 = r.a.x, y0 = r.a.y, x1 = r.a.z, y1 = r.a.w, x2 = r.b.x, y2 = r.b.y;
-    t.fx0 = cvt_i32(floorf(smin3(x0, x1, x2)));
-    t.fy0 = cvt_i32(floorf(smin3(y0, y1, y2)));
-    t.cx1 = cvt_i32(ceilf(smax3(x0, x1, x2)));
-    t.cy1 = cvt_i32(ceilf(smax3(y0, y1, y2)));
+    if constexpr (INSIDE) {
+        t.fx0 = (int)floorf(fminf(fminf(x0, x1), x2));
+        t.fy0 = (int)floorf(fminf(fminf(y0, y1), y2));
+        t.cx1 = (int)ceilf(fmaxf(fmaxf(x0, x1), x2));
+        t.cy1 = (int)ceilf(fmaxf(fmaxf(y0, y1), y2));
+    } else {
+        t.fx0 = cvt_i32(floorf(smin3(x0, x1, x2)));
+        t.fy0 = cvt_i32(floorf(smin3(y0, y1, y2)));
+        t.cx1 = cvt_i32(ceilf(smax3(x0, x1, x2)));
+        t.cy1 = cvt_i32(ceilf(smax3(y0, y1, y2)));
+    }
     float c0 = x1 * y2 - x2 * y1;
     float c1 = x2 * y0 - x0 * y2;
     float c2 = x0 * y1 - x1 * y0;
     float area = (c0 + c1) + c2;
-    if (area >= 0 && (double)area < 1.0e-12) return false;
+    if (area >= 0 && area <= AREA_NONE) return false;
     float a0 = y1 - y2, b0 = x2 - x1;
     float a1 = y2 - y0, b1 = x0 - x2;
     float a2 = y0 - y1, b2 = x1 - x0;
@@ -525,14 +545,40 @@ __device__ __forceinline__ void vis_raster_rect(const Arena& ar, const ViewDesc&
                                                 uint32_t key) {
     unsigned long long* vk = ar.vkeys + V.pix_base;
     bool any = false;
-    for (int py = rc.y0; py < rc.y1; ++py)
+    // Rectangles of at most 8 columns, as nearly all of a fine mesh's: no
+    // pixel lies 8 or more past its anchor, and by columns the anchor, its
+    // products and the pixel's step are taken once per column (the operations
+    // of cover() on the same values, so the same bits)
+    if (__ballot(rc.x1 - rc.x0 > 8 || rc.x0 != rt.fx0) == 0ull) {
         for (int px = rc.x0; px < rc.x1; ++px) {
-            float al, be, ga, z;
-            if (cover(rt, px, py, al, be, ga, z) && z < INFINITY) {
-                atomicMin(&vk[(size_t)py * (size_t)V.W + (size_t)px], depth_key(z, key));
-                any = true;
+            const int sx = imax(px & ~15, rt.fx0);
+            const float sxc = (float)sx + 0.5f, step = (float)(px - sx);
+            const float x0 = rt.a0 * sxc, x1 = rt.a1 * sxc, x2 = rt.a2 * sxc;
+            const float s0 = rt.a0 * step, s1 = rt.a1 * step, s2 = rt.a2 * step;
+            for (int py = rc.y0; py < rc.y1; ++py) {
+                const float pyc = (float)py + 0.5f;
+                const float e0 = ((x0 + rt.b0 * pyc) + rt.c0) + s0;
+                const float e1 = ((x1 + rt.b1 * pyc) + rt.c1) + s1;
+                const float e2 = ((x2 + rt.b2 * pyc) + rt.c2) + s2;
+                if (e0 >= 0.f && e1 >= 0.f && e2 >= 0.f) {
+                    const float z = (rt.z0 * (e0 * rt.inv_area) + rt.z1 * (e1 * rt.inv_area)) + rt.z2 * (e2 * rt.inv_area);
+                    if (z < INFINITY) {
+                        atomicMin(&vk[(size_t)py * (size_t)V.W + (size_t)px], depth_key(z, key));
+                        any = true;
+                    }
+                }
             }
         }
+    } else {
+        for (int py = rc.y0; py < rc.y1; ++py)
+            for (int px = rc.x0; px < rc.x1; ++px) {
+                float al, be, ga, z;
+                if (cover(rt, px, py, al, be, ga, z) && z < INFINITY) {
+                    atomicMin(&vk[(size_t)py * (size_t)V.W + (size_t)px], depth_key(z, key));
+                    any = true;
+                }
+            }
+    }
     if (any) flag_bins<T>(ar, V, rc);
 }
 
@@ -600,10 +646,10 @@ __device__ __forceinline__ void setup_face(const KArgs& ka, const Arena& ar, uin
         if constexpr (!INSIDE) cls = classify(f.c0, f.c1, f.c2);
         want_clip = cls == CLS_CLIP;
         if (cls == CLS_INSIDE) {
-            TriRec r = make_rec(f.c0, f.c1, f.c2, V.W, V.H);
+            TriRec r = make_rec<INSIDE>(f.c0, f.c1, f.c2, V.W, V.H);
             if (!is_backface(r)) {
                 RasterTri rt;
-                if (raster_setup(r, rt)) {
+                if (raster_setup<INSIDE>(r, rt)) {
                     rc = screen_rect(rt, V.W, V.H);
                     if (rc.x0 < rc.x1 && rc.y0 < rc.y1) {
                         r.c.y = s * 8u;
@@ -811,8 +857,8 @@ __global__ __launch_bounds__(256, BATCH && SHARE ? 6 : 8) void k_vis(KArgs ka, A
         if constexpr (!INSIDE) cls = classify(c0, c1, c2);
         want_clip = cls == CLS_CLIP;
         if (cls == CLS_INSIDE) {
-            r = make_rec(c0, c1, c2, V.W, V.H);
-            if (!is_backface(r) && raster_setup(r, rt)) {
+            r = make_rec<INSIDE>(c0, c1, c2, V.W, V.H);
+            if (!is_backface(r) && raster_setup<INSIDE>(r, rt)) {
                 rc = screen_rect(rt, V.W, V.H);
                 if (rc.x0 < rc.x1 && rc.y0 < rc.y1) {
                     area = (uint32_t)((rc.x1 - rc.x0) * (rc.y1 - rc.y0));
@@ -1552,9 +1598,10 @@ __global__ __launch_bounds__(256) void k_big(KArgs ka, Arena ar) {
 // absorbs): returns whether it did, with its depth and packed colour.
 // VARY: the view may carry the batch's vertex-stage outputs (V.vary); false
 // for plain draws, whose views never do.
-template <class S, bool VARY = true>
+// INSIDE: the draw's faces all lie inside the frustum (the host's bound).
+template <class S, bool VARY, bool INSIDE>
 __device__ __forceinline__ bool shade_vis_pixel(const ViewDesc& V, const Arena& ar, unsigned long long k, int px,
-                                                int py, float dfb, float& z, uint32_t& bgra, bool no_clip = false) {
+                                                int py, float dfb, float& z, uint32_t& bgra) {
     const uint32_t key = (uint32_t)k;
     const uint32_t s = key >> 3, j = key & 7u;
     const DevGroup G = group_of(V, s);
@@ -1582,16 +1629,15 @@ __device__ __forceinline__ bool shade_vis_pixel(const ViewDesc& V, const Arena& 
     TriRec r;
     bool clipped = false;
     uint32_t slot = 0;
-    // no_clip: the draw's faces all lie inside the frustum (the host's bound)
-    if (!no_clip && classify(c0, c1, c2) == CLS_CLIP) {
+    if (!INSIDE && classify(c0, c1, c2) == CLS_CLIP) {
         clipped = true;
         slot = ar.clip_base[V.face_base + s] + j;   // written by k_clip
         r = ar.clip_rec[slot];
     } else {
-        r = make_rec(c0, c1, c2, V.W, V.H);
+        r = make_rec<INSIDE>(c0, c1, c2, V.W, V.H);
     }
     RasterTri rt;
-    raster_setup(r, rt);
+    raster_setup<INSIDE>(r, rt);
     float al, be, ga;
     cover(rt, px, py, al, be, ga, z);
     if (!(z < dfb)) return false;   // reference mergeTileResults: strict less
@@ -1628,7 +1674,7 @@ __device__ __forceinline__ bool resolve_vis_pixel(const ViewDesc& V, const Arena
                                                   int py, size_t pix, float dfb) {
     float z;
     uint32_t bgra;
-    if (!shade_vis_pixel<S, VARY>(V, ar, k, px, py, dfb, z, bgra, INSIDE)) return false;
+    if (!shade_vis_pixel<S, VARY, INSIDE>(V, ar, k, px, py, dfb, z, bgra)) return false;
     gst(V.depth, pix, z);
     gst(V.color, pix, bgra);
     if (V.ids) gst(V.ids, pix, (uint32_t)k);
@@ -1782,7 +1828,7 @@ __global__ __launch_bounds__(256, (INSIDE && !IDS && SK != SHADER_PBR) ? 7 : 1) 
         if (k == EMPTY_KEY) continue;
         float z;
         uint32_t bgra;
-        const bool drawn = shade_vis_pixel<S, false>(V, ar, k, px, py, ka.clear_depth, z, bgra, INSIDE);
+        const bool drawn = shade_vis_pixel<S, false, INSIDE>(V, ar, k, px, py, ka.clear_depth, z, bgra);
         vk[pix] = drawn ? ((unsigned long long)__float_as_uint(z) << 32) | (IDS ? (uint32_t)k : bgra) : EMPTY_KEY;
         if (IDS && drawn) ar.vcol[V.pix_base + pix] = bgra;
     }
