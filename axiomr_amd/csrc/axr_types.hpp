@@ -141,6 +141,7 @@ enum Counter : uint32_t {
     CNT_BIG_RECS = 9,     // the next word one 64-bit counter (records << 32 | items)
     CNT_NEED_BIG_RECS = 10,
     CNT_NEED_BIG_ITEMS = 11,
+    CNT_READ_BLOCKS = 12, // workgroups of a read-back (k_read) that are done
     CNT_COUNT = 16,
 };
 constexpr uint32_t ERR_CLIP_FACES = 1u;
@@ -217,6 +218,14 @@ struct VaryJob {
     uint32_t count;
     uint32_t view;
     int32_t kind;
+};
+
+// A read-back of up to three planes of `words` 32-bit words each into pinned
+// host memory (null dst: not asked for).
+struct ReadJob {
+    const uint32_t* src[3];
+    uint32_t* dst[3];
+    uint64_t words;
 };
 
 // Kernel arguments common to every stage.  `table` points to `nviews`

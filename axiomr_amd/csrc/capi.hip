@@ -2,10 +2,12 @@
 // device resources, the frame arena, drawMesh, the graph-captured batch.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
 #include <new>
 #include "internal.hpp"
 
@@ -278,15 +280,19 @@ void sig_release(int device, uint64_t* p) {
 }  // namespace
 
 // The pinned block of an arena: the counters as last copied back, then the
-// error word the kernels set, 128-byte aligned past them.
+// error word the kernels set and the word that host waits poll, each on a
+// cache line of its own.
 constexpr uint32_t HOST_ERR_WORD = (CNT_COUNT + 31) / 32 * 32 + 32;
+constexpr uint32_t HOST_DONE_WORD = HOST_ERR_WORD + 32;
 
 int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa) {
     hipError_t e = hipStreamCreateWithFlags(&fa.stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&fa.host_counters, (HOST_ERR_WORD + 32) * 4, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&fa.host_counters, (HOST_DONE_WORD + 32) * 4, hipHostMallocDefault);
     if (e != hipSuccess) return hip_fail(err, e, "frame arena stream");
     fa.host_err = fa.host_counters + HOST_ERR_WORD;
     *fa.host_err = 0;
+    fa.host_done = fa.host_counters + HOST_DONE_WORD;
+    *fa.host_done = 0;
     FrameSize fs;
     fs.faces = 1024;
     fs.tiles = 1024;
@@ -332,6 +338,42 @@ int arena_read_counters(ErrSink& err, FrameArena& fa) {
     hipError_t e = hipMemcpyAsync(fa.host_counters, fa.counters.p, CNT_COUNT * 4, hipMemcpyDeviceToHost, fa.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(fa.stream);
     return e == hipSuccess ? AXR_OK : hip_fail(err, e, "read counters");
+}
+
+hipError_t wait_word(const uint32_t* word, uint32_t seq, hipStream_t st) {
+    // most waits end within a frame's time; a longer one (or a stream that
+    // failed and will never store the word) goes to the runtime
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(3);
+    for (uint32_t i = 1;; ++i) {
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == seq) return hipSuccess;
+        __builtin_ia32_pause();
+        if (i % 256 == 0 && std::chrono::steady_clock::now() > until) return hipStreamSynchronize(st);
+    }
+}
+
+int arena_wait(ErrSink& err, FrameArena& fa) {
+    hipError_t e = launch_done(fa.host_done, ++fa.done_seq, fa.stream);
+    if (e == hipSuccess) e = wait_word(fa.host_done, fa.done_seq, fa.stream);
+    return e == hipSuccess ? AXR_OK : hip_fail(err, e, "wait for a frame");
+}
+
+bool pinned_planes(ReadJob& job) {
+    for (auto& d : job.dst) {
+        if (!d) continue;
+        hipPointerAttribute_t a{}, b{};
+        char* const last = (char*)d + job.words * 4 - 1;
+        hipError_t e = hipPointerGetAttributes(&a, d);
+        if (e == hipSuccess) e = hipPointerGetAttributes(&b, last);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();   // memory the runtime does not know
+            return false;
+        }
+        if (a.type != hipMemoryTypeHost || b.type != hipMemoryTypeHost || !a.devicePointer || !b.devicePointer ||
+            (char*)b.devicePointer - (char*)a.devicePointer != last - (char*)d || (uintptr_t)a.devicePointer % 16)
+            return false;
+        d = (uint32_t*)a.devicePointer;
+    }
+    return true;
 }
 
 // Every device error bit also sets the pinned flag, so without the flag the
@@ -638,12 +680,11 @@ int axr_ctx_create(int device, uint64_t hbm_budget_bytes, axr_ctx** out) {
     ctx->cfg.bin_capacity = 128;
     ctx->cfg.small_footprint = 12;
     if (hipSetDevice(device) != hipSuccess) { delete ctx; return AXR_ERR_HIP; }
-    for (auto* evs : {ctx->join_ev, ctx->sync_ev})
-        for (int k = 0; k < axr_ctx::kArenas; ++k)
-            if (hipEventCreateWithFlags(&evs[k], hipEventDisableTiming) != hipSuccess) {
-                axr_ctx_destroy(ctx);
-                return AXR_ERR_HIP;
-            }
+    for (auto& ev : ctx->join_ev)
+        if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+            axr_ctx_destroy(ctx);
+            return AXR_ERR_HIP;
+        }
     if (hipHostMalloc((void**)&ctx->noalloc_counters, CNT_COUNT * 4, hipHostMallocDefault) != hipSuccess) {
         axr_ctx_destroy(ctx);
         return AXR_ERR_OOM;
@@ -662,9 +703,8 @@ int axr_ctx_destroy(axr_ctx* ctx) {
     if (ctx->main.stream) (void)ctx_sync_all(ctx);
     for (auto& a : ctx->alt) arena_destroy(ctx, a);
     arena_destroy(ctx, ctx->main);
-    for (auto* evs : {ctx->join_ev, ctx->sync_ev})
-        for (int k = 0; k < axr_ctx::kArenas; ++k)
-            if (evs[k]) (void)hipEventDestroy(evs[k]);
+    for (auto& ev : ctx->join_ev)
+        if (ev) (void)hipEventDestroy(ev);
     if (ctx->noalloc_counters) (void)hipHostFree(ctx->noalloc_counters);
     if (ctx->ev) {
         for (int i = 0; i < axr_ctx::kEventRing; ++i)
@@ -753,18 +793,24 @@ static int arena_settle_overflow(axr_ctx* ctx, FrameArena& fa) {
 int axr_sync(axr_ctx* ctx) {
     if (!ctx) return AXR_ERR_INVALID;
     (void)hipSetDevice(ctx->device);
-    // an event behind each arena's queued work, all recorded before the
-    // first wait: the streams' completions then overlap (a stream wait per
-    // arena in turn costs ~10 us each); the counters come back only from an
+    // a word stored behind the queued work of each arena that took any, all of
+    // them queued before the first wait; the counters come back only from an
     // arena whose kernels flagged an error
     int live[axr_ctx::kArenas];
     int n = 0;
     for (int k = 0; k < axr_ctx::kArenas; ++k)
-        if (arena_no(ctx, k).stream) live[n++] = k;
+        if (k == 0 || ctx->alt_used[k - 1]) live[n++] = k;
     hipError_t e = hipSuccess;
-    for (int i = 0; i < n && e == hipSuccess; ++i) e = hipEventRecord(ctx->sync_ev[live[i]], arena_no(ctx, live[i]).stream);
-    for (int i = 0; i < n && e == hipSuccess; ++i) e = hipEventSynchronize(ctx->sync_ev[live[i]]);
-    if (e != hipSuccess) return hip_fail(ctx->err, e, "hipEventSynchronize");
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
+        FrameArena& fa = arena_no(ctx, live[i]);
+        e = launch_done(fa.host_done, ++fa.done_seq, fa.stream);
+    }
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
+        FrameArena& fa = arena_no(ctx, live[i]);
+        e = wait_word(fa.host_done, fa.done_seq, fa.stream);
+    }
+    if (e != hipSuccess) return hip_fail(ctx->err, e, "axr_sync");
+    for (int k = 1; k < axr_ctx::kArenas; ++k) ctx->alt_used[k - 1] = ctx->alt_unjoined[k - 1] = false;
     int r = AXR_OK;
     for (int i = 0; i < n; ++i) {
         FrameArena& fa = arena_no(ctx, live[i]);
@@ -977,13 +1023,23 @@ int axr_fb_read(axr_fb* fb, uint8_t* bgra, float* depth, uint32_t* ids) {
     (void)hipSetDevice(ctx->device);
     const size_t n = (size_t)fb->w * fb->h;
     int r = fb_settle(fb);
-    if (r || (r = ctx_sync_all(ctx))) return r;
+    // behind what other streams still have queued, if axr_sync has not waited for it
+    const bool unjoined = std::any_of(std::begin(ctx->alt_unjoined), std::end(ctx->alt_unjoined), [](bool u) { return u; });
+    if (r || (unjoined && (r = ctx_join(ctx)))) return r;
     if (ids && !fb->ids) return fail(ctx->err, AXR_ERR_INVALID, "framebuffer has no id plane");
     // copies on the context's own stream: a copy on the null stream would
     // give the process one more hardware queue to share with the frame
     // arenas' streams, which then slows every later overlapped draw
     const hipStream_t st = ctx->main.stream;
+    FrameArena& fa = ctx->main;
+    ReadJob job{{fb->color, (const uint32_t*)fb->depth, fb->ids}, {(uint32_t*)bgra, (uint32_t*)depth, ids}, n};
     hipError_t e = hipSuccess;
+    // one plane, or memory that is not pinned: a runtime copy per plane
+    if ((bgra != nullptr) + (depth != nullptr) + (ids != nullptr) > 1 && pinned_planes(job)) {
+        e = launch_read(job, fa.a.counters + CNT_READ_BLOCKS, fa.host_done, ++fa.done_seq, st);
+        if (e == hipSuccess) e = wait_word(fa.host_done, fa.done_seq, st);
+        return e == hipSuccess ? AXR_OK : hip_fail(ctx->err, e, "framebuffer read");
+    }
     if (e == hipSuccess && bgra) e = hipMemcpyAsync(bgra, fb->color, n * 4, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess && depth) e = hipMemcpyAsync(depth, fb->depth, n * 4, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess && ids) e = hipMemcpyAsync(ids, fb->ids, n * 4, hipMemcpyDeviceToHost, st);
@@ -1048,7 +1104,7 @@ static int draw_pipelined(axr_ctx* ctx, axr_fb* fb, const KArgs& ka, const Frame
             if (e != hipSuccess) return hip_fail(ctx->err, e, "stream order");
         }
     }
-    if (x) ctx->alt_unjoined[x - 1] = true;   // before the launch: a failed one may have queued work
+    if (x) ctx->alt_unjoined[x - 1] = ctx->alt_used[x - 1] = true;   // before the launch: a failed one may have queued work
     if ((r = arena_launch(ctx->err, fa, ka, ev, wait))) return r;
     fb->clear_pending = false;   // written by this launch, even by a frame that overflows
     // the end of this draw's framebuffer pass, for the next draw to wait on
@@ -1121,8 +1177,7 @@ int axr_draw(axr_ctx* ctx, axr_fb* fb, const axr_mesh* mesh, const axr_draw_para
         if ((r = ctx_launch(ctx, ka))) return r;
         fb->clear_pending = false;   // written by this launch, even by a frame that overflows
         if (async) return AXR_OK;
-        const hipError_t e = hipStreamSynchronize(ctx->main.stream);
-        if (e != hipSuccess) return hip_fail(ctx->err, e, "hipStreamSynchronize");
+        if ((r = arena_wait(ctx->err, ctx->main))) return r;
         if ((r = arena_counters_after_wait(ctx->err, ctx->main))) return r;
         if (!ctx->main.host_counters[CNT_ERROR]) return AXR_OK;
         r = arena_check_overflow(ctx, ctx->err, ctx->main, fs);

@@ -41,6 +41,18 @@ hipError_t launch_clear(uint32_t* color, float* depth, uint32_t* ids, size_t n, 
 hipError_t launch_prep(const Arena& ar, uint32_t ntiles, hipStream_t st);
 hipError_t launch_clear_views(const ViewDesc* views, const uint32_t* pix_bases, uint32_t nviews, uint32_t total,
                               uint32_t bgra, float d, hipStream_t st);
+// A host wait without a runtime wait: the stream's next kernel stores `seq` to
+// a pinned word that the host polls.
+hipError_t launch_done(uint32_t* word, uint32_t seq, hipStream_t st);
+// The planes of `job` copied by one kernel whose last workgroup stores `seq`
+// to `word`; *blocks_done is zero before and after.
+hipError_t launch_read(const ReadJob& job, uint32_t* blocks_done, uint32_t* word, uint32_t seq, hipStream_t st);
+// Polls until *word == seq (launch_done / launch_read on st), for a few
+// milliseconds, then waits for the stream.
+hipError_t wait_word(const uint32_t* word, uint32_t seq, hipStream_t st);
+// The device addresses of the job's host planes, if all of them are pinned
+// host memory and 16-byte aligned.
+bool pinned_planes(ReadJob& job);
 // Bytes of a shader kind's vertex-stage output per vertex (0: none).
 uint32_t vary_bytes(int kind);
 
@@ -72,6 +84,8 @@ struct FrameArena {
     bool dirty = true;         // bin counts / counters need a k_prep before the next frame
     uint32_t* host_counters = nullptr;   // pinned, CNT_COUNT words (then host_err, on its own cache line)
     uint32_t* host_err = nullptr;        // pinned word the kernels set nonzero with any error bit
+    uint32_t* host_done = nullptr;       // pinned word the host polls to wait for the stream
+    uint32_t done_seq = 0;               // the last value asked for
     uint64_t* sig = nullptr;   // signal memory its stream writes after a framebuffer pass (null: use events)
 };
 
@@ -96,10 +110,10 @@ struct axr_ctx {
     static constexpr int kArenas = 4;
     axr::FrameArena alt[kArenas - 1];
     hipEvent_t join_ev[kArenas] = {};   // join_ev[k]: recorded on arena k's stream for another to wait on
-    hipEvent_t sync_ev[kArenas] = {};   // sync_ev[k]: recorded on arena k's stream for axr_sync to wait on
     int next_arena = 0;                 // arena of the next asynchronous visibility-mode draw
     int last_arena = 0;                 // arena whose stream took the latest framebuffer work
     bool alt_unjoined[kArenas - 1] = {};  // alt[k] took work main has not waited for
+    bool alt_used[kArenas - 1] = {};      // alt[k] took work since the last axr_sync
     axr::ArenaNeeds need_floor;         // the largest overflow needs reported: every arena is grown to them
     uint64_t last_value = 0;            // nonzero: that work was a draw whose stream then wrote this
                                         // value to its arena's signal (0: wait with an event)
@@ -188,6 +202,8 @@ int arena_read_counters(ErrSink& err, FrameArena& fa);
 // flagged an error in the pinned error word, else their host copy's error
 // word zeroed.
 int arena_counters_after_wait(ErrSink& err, FrameArena& fa);
+// Host wait for everything queued on the arena's stream.
+int arena_wait(ErrSink& err, FrameArena& fa);
 // k_prep if the arena is fresh or dirty, then the frame's kernels; ev (may
 // be null) times them.
 int arena_launch(ErrSink& err, FrameArena& fa, const KArgs& ka, StageEvents* ev, const FbWait& wait = {});
