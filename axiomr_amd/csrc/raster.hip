@@ -310,6 +310,34 @@ __device__ __forceinline__ bool cover(const RasterTri& t, int px, int py, float&
     return true;
 }
 
+// Keeps a branch that few waves take a branch: the compiler turns a short one
+// into selects, whose operations then run for every pixel.
+__device__ __forceinline__ void keep_branch() { asm volatile(""); }
+
+// cover()'s z for a pixel d past the anchor whose edge products are
+// x0 = a0 * (anchor + 0.5), ...: the walks take those once per run of pixels.
+// Few lanes of a wave are ever 8 or more past their anchor, so that step is a
+// branch on the wave's lanes.
+__device__ __forceinline__ bool cover_from(const RasterTri& t, float x0, float x1, float x2, int d, float pyc, float& z) {
+    float r0 = (x0 + t.b0 * pyc) + t.c0;
+    float r1 = (x1 + t.b1 * pyc) + t.c1;
+    float r2 = (x2 + t.b2 * pyc) + t.c2;
+    float lane = (float)d;
+    if (d >= 8) {
+        keep_branch();
+        r0 = r0 + t.a0 * 8.0f;
+        r1 = r1 + t.a1 * 8.0f;
+        r2 = r2 + t.a2 * 8.0f;
+        lane = lane - 8.0f;   // whole numbers: exact
+    }
+    const float e0 = r0 + t.a0 * lane;
+    const float e1 = r1 + t.a1 * lane;
+    const float e2 = r2 + t.a2 * lane;
+    if (!(e0 >= 0.f && e1 >= 0.f && e2 >= 0.f)) return false;
+    z = (t.z0 * (e0 * t.inv_area) + t.z1 * (e1 * t.inv_area)) + t.z2 * (e2 * t.inv_area);
+    return z < INFINITY;
+}
+
 // 64-bit depth key: order-preserving image of z (with -0 folded onto +0, the
 // reference's strict-less test treats them as equal) above the submission key.
 __device__ __forceinline__ unsigned long long depth_key(float z, uint32_t key) {
@@ -762,8 +790,10 @@ __device__ __forceinline__ void vis_span(const Arena& ar, const ViewDesc& V, con
     int px = x0 + (q0 - dy * w), py = y0 + dy;
     uint32_t flagged = ~0u;
     for (int q = q0; q < q1; ++q) {
-        float al, be, ga, z;
-        if (cover(rt, px, py, al, be, ga, z) && z < INFINITY) {
+        const int sx = imax(px & ~15, rt.fx0);
+        const float sxc = (float)sx + 0.5f;
+        float z;
+        if (cover_from(rt, rt.a0 * sxc, rt.a1 * sxc, rt.a2 * sxc, px - sx, (float)py + 0.5f, z)) {
             atomicMin(&vk[(size_t)py * (size_t)V.W + (size_t)px], depth_key(z, key));
             const uint32_t b = V.tile_base + (uint32_t)(py / T * V.tiles_x + px / T);
             if (b != flagged) ar.tile_count[b] = 1u;
@@ -1333,23 +1363,48 @@ __device__ __forceinline__ void resolve_tile_kind(const ViewDesc& V, const Arena
 // of its own rectangle; the rest of every longer rectangle is cut into
 // pieces of WALK_CAP pixels that the wave's lanes then take in turn.
 
-// Pixels [q0, q1) of the rectangle [x0, x0 + w) x [y0, ...) in row-major
-// order; every covered pixel takes the minimum of its key.
+// Pixels [q0, q1) of the rectangle [x0, x0 + w) x [y0, ...) (bin coordinates)
+// in row-major order; every covered pixel takes the minimum of its key.
+// A bin of up to 16 px lies in one of the reference's 16-pixel tile columns, so
+// the rectangle's pixels share one anchor, whose edge products are taken once
+// (the 4M-triangle soup's k_raster 194 -> 184 us).  At 32 px the walk would
+// have to be split at the columns' border, which cost the batch's kernel 3 %.
 template <int T>
 __device__ __forceinline__ void walk_span(const RasterTri& rt, int x0, int y0, int w, int q0, int q1, uint32_t key,
                                           unsigned long long* keys, int ox, int oy, float inv_w) {
     // row of q0 = floor(q0 / w): q0 < 2^16 and w <= 32, so (q0 + 0.5) / w is
     // at least 1/64 from an integer and its rounded product within 2^-7 of it
     const int dy = q0 == 0 ? 0 : (int)(((float)q0 + 0.5f) * inv_w);
-    int px = x0 + (q0 - dy * w), py = y0 + dy;
-    const int x1 = x0 + w;
-    for (int q = q0; q < q1; ++q) {
-        float al, be, ga, z;
-        if (cover(rt, px, py, al, be, ga, z) && z < INFINITY)
-            atomicMin(&keys[(py - oy) * T + (px - ox)], depth_key(z, key));
-        if (++px == x1) {
-            px = x0;
-            ++py;
+    if constexpr (T <= 16) {
+        const int lx = x0 + (q0 - dy * w), ly = y0 + dy;
+        const int sx = imax(ox & ~15, rt.fx0);
+        const float sxc = (float)sx + 0.5f;
+        const float a0 = rt.a0 * sxc, a1 = rt.a1 * sxc, a2 = rt.a2 * sxc;
+        int d = ox + lx - sx, at = ly * T + lx;
+        const int d1 = ox + x0 + w - sx;
+        float pyc = (float)(oy + ly) + 0.5f;   // halves below 2^23: adding 1 is exact
+        for (int q = q0; q < q1; ++q) {
+            float z;
+            if (cover_from(rt, a0, a1, a2, d, pyc, z)) atomicMin(&keys[at], depth_key(z, key));
+            ++at;
+            if (++d == d1) {
+                keep_branch();
+                d -= w;
+                at += T - w;
+                pyc += 1.0f;
+            }
+        }
+    } else {
+        int px = x0 + ox + (q0 - dy * w), py = y0 + oy + dy;
+        const int x1 = x0 + ox + w;
+        for (int q = q0; q < q1; ++q) {
+            float al, be, ga, z;
+            if (cover(rt, px, py, al, be, ga, z) && z < INFINITY)
+                atomicMin(&keys[(py - oy) * T + (px - ox)], depth_key(z, key));
+            if (++px == x1) {
+                px -= w;
+                ++py;
+            }
         }
     }
 }
@@ -1383,13 +1438,13 @@ __device__ __forceinline__ void get_piece(const WalkRefs* wp, const Arena& ar, u
 }
 
 // All 64 lanes call it with their own triangle (w = h = 0 for none); ref is
-// its bin entry's record reference.
+// its bin entry's record reference, (x0, y0, w, h) its rectangle in bin
+// coordinates.
 template <int T, class P>
 __device__ __forceinline__ void walk_wave(P* wp, const Arena& ar, const RasterTri& rt, uint32_t ref, int x0, int y0,
                                           int w, int h, uint32_t key, unsigned long long* keys, int ox, int oy) {
     const int fp = w * h;
-    const float inv_w = w ? 1.0f / (float)w : 0.0f;
-    walk_span<T>(rt, x0 + ox, y0 + oy, w, 0, imin(fp, WALK_CAP), key, keys, ox, oy, inv_w);
+    walk_span<T>(rt, x0, y0, w, 0, imin(fp, WALK_CAP), key, keys, ox, oy, 0.0f);
     const uint32_t pieces = fp > WALK_CAP ? (uint32_t)(fp - 1) / WALK_CAP : 0u;
     const uint32_t incl = wave_incl_scan(pieces);
     const uint32_t total = __shfl(incl, 63);
@@ -1412,7 +1467,7 @@ __device__ __forceinline__ void walk_wave(P* wp, const Arena& ar, const RasterTr
         const int rx = (int)(rect & 255u), ry = (int)((rect >> 8) & 255u);
         const int rw = (int)((rect >> 16) & 255u), rh = (int)(rect >> 24);
         const int q0 = WALK_CAP * (int)(j - wp->start[o] + 1);
-        walk_span<T>(t, rx + ox, ry + oy, rw, q0, imin(q0 + WALK_CAP, rw * rh), pkey, keys, ox, oy, 1.0f / (float)rw);
+        walk_span<T>(t, rx, ry, rw, q0, imin(q0 + WALK_CAP, rw * rh), pkey, keys, ox, oy, 1.0f / (float)rw);
     }
 }
 
