@@ -153,6 +153,7 @@ constexpr uint32_t ERR_SKIPPED = 16u;   // a pass the host skipped had work: the
 // Bins of binned mode: level k of a bin holds 2^(bin0_shift + k) entries, so
 // BIN_LEVELS levels reach past 2^31 entries for the smallest first level.
 constexpr uint32_t BIN0_MIN_SHIFT = 5, BIN0_MAX_SHIFT = 12;
+constexpr uint32_t COUNT_BLOCK = 8192;         // words of tile_count that bins are spread over
 constexpr uint32_t BIN_LEVELS = 27;
 constexpr uint32_t CHUNK_NONE = 0xFFFFFFFFu;   // a level the pools had no room for
 constexpr uint32_t POOL_SUBS = 64;
@@ -178,8 +179,8 @@ struct Arena {
     uint32_t* clip_faces;      // global face slots queued for clipping
     TriRec* clip_rec;          // clipped sub-triangles
     Vertex56* clip_verts;      // 3 per clip record
-    uint32_t* tile_count;      // per bin: its entries (binned mode), whether it holds
-                               // keys (visibility mode)
+    uint32_t* tile_count;      // per bin: its entries (binned mode, at count_word), whether
+                               // it holds keys (visibility mode)
     // binned mode: record refs by bin (see bin_put in raster.hip)
     uint32_t* bins;            // 2^bin0_shift first entries of every bin
     uint32_t* bin_chunks;      // BIN_LEVELS words per bin: where its further entries

@@ -173,7 +173,7 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     const uint64_t clip_recs = std::max<uint64_t>({2 * cap_clip_faces + 2 * clip_faces, need.clip_recs, a.cap_clip_recs});
     if ((r = grow(ctx, err, fa, fa.clip_rec, clip_recs * sizeof(TriRec))) ||
         (r = grow(ctx, err, fa, fa.clip_verts, clip_recs * 3 * sizeof(Vertex56))) ||
-        (r = grow(ctx, err, fa, fa.tile_count, (tiles + 1) * 4)) ||
+        (r = grow(ctx, err, fa, fa.tile_count, vis ? (tiles + 1) * 4 : (tiles + COUNT_BLOCK) / COUNT_BLOCK * COUNT_BLOCK * 4)) ||
         (!vis && ((r = grow(ctx, err, fa, fa.bins, (tiles << bin0_shift) * 4)) ||
                   (r = grow(ctx, err, fa, fa.bin_chunks, tiles * BIN_LEVELS * 4)) ||
                   (r = grow(ctx, err, fa, fa.bin_pool, (POOL_SUBS * sub + pool) * 4)) ||

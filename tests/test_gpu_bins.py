@@ -56,3 +56,15 @@ def test_levels_cover_every_slot_once():
         first = np.flatnonzero(offset == 0)
         assert (np.diff(level[first]) == 1).all() and level[0] == 0
         assert (np.diff(s)[np.diff(level) == 0] == 1).all()
+
+
+def test_count_words_are_a_permutation_of_each_block():
+    """count_word as the kernels compute it: every block of 8,192 bins maps
+    onto itself one to one, runs of four bins stay together, and neighbouring
+    runs lie in different 128-byte lines."""
+    t = np.arange(3 * 8192, dtype=np.int64)
+    w = (t & ~8191) | ((t & 0x3FC) << 3) | (t & 3) | ((t >> 8) & 28)
+    assert (np.sort(w) == t).all() and (w >> 13 == t >> 13).all()
+    assert (w[1::4] == w[0::4] + 1).all() and (w[3::4] == w[0::4] + 3).all()
+    line = w[0::4] >> 5
+    assert (line[1:] != line[:-1]).all()
