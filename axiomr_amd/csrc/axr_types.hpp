@@ -131,8 +131,8 @@ constexpr uint64_t MAX_BATCH_FACES = 0x7FFFFFFFull;
 
 // Counter block at the head of the frame arena.
 enum Counter : uint32_t {
-    CNT_CLIP_FACES = 0,   // faces queued for the full clipper
-    CNT_CLIP_RECS = 1,    // clip records reserved
+    CNT_CLIP_FACES = 0,   // faces in the clipper's shared queue
+    CNT_CLIP_RECS = 1,    // clip records reserved behind the sub-queues' own
     CNT_ERROR = 4,        // sticky error bits, see ERR_*
     CNT_NEED_CLIP_FACES = 5,
     CNT_NEED_CLIP_RECS = 6,
@@ -157,7 +157,8 @@ constexpr uint32_t COUNT_BLOCK = 8192;         // words of tile_count that bins 
 constexpr uint32_t BIN_LEVELS = 27;
 constexpr uint32_t CHUNK_NONE = 0xFFFFFFFFu;   // a level the pools had no room for
 constexpr uint32_t POOL_SUBS = 64;
-constexpr uint32_t POOL_STRIDE = 32;           // words between the pools' counters
+constexpr uint32_t CLIP_SUBS = 64;             // one per lane of a wave
+constexpr uint32_t POOL_STRIDE = 32;           // words between the pools' and sub-queues' counters
 
 // Raster modes (axr_config.raster_mode).
 enum RasterMode : int32_t {
@@ -176,7 +177,9 @@ struct Arena {
     TriRec* rec;               // binned mode: one record per face slot of every view
     uint32_t* clip_base;       // visibility mode (same memory as rec): first clip
                                // record of each clipped face slot
-    uint32_t* clip_faces;      // global face slots queued for clipping
+    uint32_t* clip_faces;      // global face slots queued for clipping: CLIP_SUBS
+                               // sub-queues of clip_sub_cap, then the shared queue
+    uint32_t* clip_next;       // the sub-queues' fill, POOL_STRIDE words apart
     TriRec* clip_rec;          // clipped sub-triangles
     Vertex56* clip_verts;      // 3 per clip record
     uint32_t* tile_count;      // per bin: its entries (binned mode, at count_word), whether
@@ -188,10 +191,10 @@ struct Arena {
     uint32_t* bin_pool;        // POOL_SUBS sub-pools of sub_cap entries, then a shared
                                // one of pool_cap
     uint32_t* pool_next;       // the pools' fill, POOL_STRIDE words apart
-    uint32_t cap_clip_faces;
+    uint32_t cap_clip_faces;   // entries of the shared queue
+    uint32_t clip_sub_cap;     // entry e of the sub-queues has the clip records 2e and
+                               // 2e + 1; 0: no sub-queues
     uint32_t cap_clip_recs;
-    uint32_t clip_static;      // queue entries with two clip records of their own
-                               // (clip_rec[2q], [2q + 1])
     uint32_t bin0_shift;
     uint32_t sub_cap;
     uint32_t pool_cap;

@@ -146,7 +146,12 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     // slot (only the first clip record of a clipped face, 4 bytes) and no
     // bin pairs; binned mode keeps a 48-byte record per face slot
     const bool vis = fs.pixels != 0;
-    uint64_t clip_faces = std::max<uint64_t>({4096, faces / 16, need.clip_faces, a.cap_clip_faces});
+    const uint64_t want_clip = std::max<uint64_t>({4096, faces / 16, need.clip_faces});
+    const uint64_t clip_faces = std::max<uint64_t>(want_clip, a.cap_clip_faces);
+    // the sub-queues beside the shared queue of clip_faces entries, and their
+    // two records each beside the 2 clip_faces others
+    const uint64_t clip_sub = std::max<uint64_t>({4096 / CLIP_SUBS, want_clip / 8 / CLIP_SUBS, a.clip_sub_cap});
+    const uint64_t clip_recs = std::max<uint64_t>({2 * CLIP_SUBS * clip_sub + 2 * clip_faces, need.clip_recs, a.cap_clip_recs});
     // binned mode: the first level of a bin holds four times the mean of faces
     // per bin (a power of two of at least 32 entries), the shared pool what
     // any spread of 2 faces + 16 bins + 4096 entries over the bins needs (a
@@ -166,11 +171,9 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     int r;
     if ((r = grow(ctx, err, fa, fa.counters, CNT_COUNT * 4)) ||
         (r = grow(ctx, err, fa, fa.rec, std::max<uint64_t>(faces, 1) * (vis ? 4 : sizeof(TriRec)))) ||
-        (r = grow(ctx, err, fa, fa.clip_faces, clip_faces * 4)))
+        (r = grow(ctx, err, fa, fa.clip_next, CLIP_SUBS * POOL_STRIDE * 4)) ||
+        (r = grow(ctx, err, fa, fa.clip_faces, (CLIP_SUBS * clip_sub + clip_faces) * 4)))
         return r;
-    // two records for every queue entry, and as many again for the faces with more
-    const uint64_t cap_clip_faces = std::min<uint64_t>(fa.clip_faces.bytes / 4, 0x1FFFFFFFull);
-    const uint64_t clip_recs = std::max<uint64_t>({2 * cap_clip_faces + 2 * clip_faces, need.clip_recs, a.cap_clip_recs});
     if ((r = grow(ctx, err, fa, fa.clip_rec, clip_recs * sizeof(TriRec))) ||
         (r = grow(ctx, err, fa, fa.clip_verts, clip_recs * 3 * sizeof(Vertex56))) ||
         (r = grow(ctx, err, fa, fa.tile_count, vis ? (tiles + 1) * 4 : (tiles + COUNT_BLOCK) / COUNT_BLOCK * COUNT_BLOCK * 4)) ||
@@ -199,8 +202,9 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     a.big_rec = (TriRec*)fa.big_rec.p;
     a.big_start = (uint32_t*)fa.big_start.p;
     a.vcol = (uint32_t*)fa.vcol.p;
-    a.cap_clip_faces = (uint32_t)cap_clip_faces;
-    a.clip_static = (uint32_t)cap_clip_faces;
+    a.clip_next = (uint32_t*)fa.clip_next.p;
+    a.clip_sub_cap = (uint32_t)clip_sub;
+    a.cap_clip_faces = (uint32_t)std::min<uint64_t>(fa.clip_faces.bytes / 4 - CLIP_SUBS * clip_sub, 0x1FFFFFFFull);
     a.cap_clip_recs = (uint32_t)std::min<uint64_t>(
         {fa.clip_rec.bytes / sizeof(TriRec), fa.clip_verts.bytes / (3 * sizeof(Vertex56)), 0x7FFFFFFFull});
     if (!vis) {
@@ -307,9 +311,9 @@ int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa) {
     return r ? r : arena_reset(err, fa);
 }
 
-constexpr int kArenaBufs = 14;
+constexpr int kArenaBufs = 15;
 static void arena_buffers(FrameArena& fa, DevBuf* (&out)[kArenaBufs]) {
-    DevBuf* bufs[kArenaBufs] = {&fa.counters, &fa.rec,        &fa.clip_faces, &fa.clip_rec,  &fa.clip_verts,
+    DevBuf* bufs[kArenaBufs] = {&fa.counters, &fa.rec,        &fa.clip_faces, &fa.clip_rec,  &fa.clip_verts, &fa.clip_next,
                                 &fa.tile_count, &fa.bins,     &fa.bin_chunks, &fa.bin_pool,  &fa.pool_next,
                                 &fa.vkeys,    &fa.big_rec,    &fa.big_start,  &fa.vcol};
     for (int i = 0; i < kArenaBufs; ++i) out[i] = bufs[i];

@@ -77,7 +77,7 @@ struct ArenaNeeds {
 // so batches on different lanes overlap on the device.
 struct FrameArena {
     hipStream_t stream = nullptr;
-    DevBuf counters, rec, clip_faces, clip_rec, clip_verts, tile_count, bins, bin_chunks, bin_pool, pool_next, vkeys,
+    DevBuf counters, rec, clip_faces, clip_next, clip_rec, clip_verts, tile_count, bins, bin_chunks, bin_pool, pool_next, vkeys,
         big_rec, big_start, vcol;
     Arena a{};
     uint64_t gen = 0;          // bumped whenever a buffer moves: captured graphs are stale

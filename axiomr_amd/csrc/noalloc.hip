@@ -94,8 +94,8 @@ uint64_t carve(unsigned char* base, uint64_t faces, uint64_t tiles, uint64_t pix
     a.cap_vkeys = (uint32_t)pixels;
     a.cap_big_recs = (uint32_t)big_recs;
     a.cap_big_items = (uint32_t)big_items;
-    // clip_static 0: every clip record from the shared counter; binned-mode
-    // fields stay empty: this path never bins
+    // no sub-queues: every clipped face in the shared queue; binned-mode fields
+    // stay empty: this path never bins
     return off;
 }
 

@@ -157,6 +157,44 @@ __device__ __forceinline__ void set_error(const Arena& ar, uint32_t bit, uint32_
     atomicMax(&ar.counters[need_slot], need);
 }
 
+// Queue face slot g of every lane with pred set for the clipper (the whole
+// wave calls it).  A wave's faces go to one of CLIP_SUBS sub-queues, what does
+// not fit there to the shared queue, whose size alone decides whether a frame
+// fits: one counter for all waves would serialize them, ~9 ns each, 250 us
+// for the 4M-triangle soup's 62,500 waves.
+__device__ __forceinline__ void queue_clip(const Arena& ar, bool pred, uint32_t g) {
+    const unsigned long long mask = __ballot(pred);
+    if (mask == 0ull) return;
+    const uint32_t sub = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) % CLIP_SUBS;
+    const uint32_t n = (uint32_t)__popcll(mask), mine = (uint32_t)__popcll(mask & __lanemask_lt());
+    const int leader = __ffsll((long long)mask) - 1;
+    const uint32_t cap = ar.clip_sub_cap;
+    uint32_t o = cap;
+    if (cap) {
+        if ((int)__lane_id() == leader) o = atomicAdd(&ar.clip_next[sub * POOL_STRIDE], n);
+        o = __shfl(o, leader);
+    }
+    const uint32_t fit = o < cap ? (cap - o < n ? cap - o : n) : 0u;   // the first `fit` of them
+    if (pred && mine < fit) ar.clip_faces[sub * cap + o + mine] = g;
+    if (fit == n) return;
+    uint32_t q = 0;
+    if ((int)__lane_id() == leader) q = atomicAdd(&ar.counters[CNT_CLIP_FACES], n - fit);
+    q = __shfl(q, leader) + mine - fit;
+    if (!pred || mine < fit) return;
+    if (q < ar.cap_clip_faces) ar.clip_faces[CLIP_SUBS * cap + q] = g;
+    else set_error(ar, ERR_CLIP_FACES, CNT_NEED_CLIP_FACES, q + 1);
+}
+
+// The frame's last pass leaves the clipper's counters zero (called by the
+// threads of one workgroup).
+__device__ __forceinline__ void reset_clip_counters(const Arena& ar) {
+    if (threadIdx.x == 0) {
+        ar.counters[CNT_CLIP_FACES] = 0;
+        ar.counters[CNT_CLIP_RECS] = 0;
+    }
+    if (ar.clip_next && threadIdx.x < CLIP_SUBS) ar.clip_next[threadIdx.x * POOL_STRIDE] = 0;
+}
+
 // reference tiled_pipeline.cpp:15-23
 __device__ __forceinline__ float clampW(float w) {
     const float tiny = 1e-6f;
@@ -361,7 +399,10 @@ __global__ void k_prep(Arena ar, uint32_t ntiles) {
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = tid; i < ntiles; i += stride) ar.tile_count[i] = 0;
     for (uint32_t i = tid; i < ar.cap_chunks; i += stride) ar.bin_chunks[i] = 0;
-    if (ar.cap_chunks && tid < (POOL_SUBS + 1) * POOL_STRIDE) ar.pool_next[tid] = 0;
+    if (ar.cap_chunks)
+        for (uint32_t i = tid; i < (POOL_SUBS + 1) * POOL_STRIDE; i += stride) ar.pool_next[i] = 0;
+    if (ar.clip_next)
+        for (uint32_t i = tid; i < CLIP_SUBS * POOL_STRIDE; i += stride) ar.clip_next[i] = 0;
     for (uint32_t i = tid; i < ar.cap_vkeys; i += stride) ar.vkeys[i] = ~0ull;
 }
 
@@ -704,12 +745,8 @@ __device__ __forceinline__ void setup_face(const KArgs& ka, const Arena& ar, uin
             }
         }
     }
-    const uint32_t cslot = wave_append(&ar.counters[CNT_CLIP_FACES], want_clip);
-    if (want_clip) {
-        if (cslot < ar.cap_clip_faces) ar.clip_faces[cslot] = g;
-        else set_error(ar, ERR_CLIP_FACES, CNT_NEED_CLIP_FACES, cslot + 1);
-        if (ka.skip_clip) raise_error(ar, ERR_SKIPPED);
-    }
+    queue_clip(ar, want_clip, g);
+    if (want_clip && ka.skip_clip) raise_error(ar, ERR_SKIPPED);
     emit_bins_wave<T>(ar, V, binnable, rc, g);
 }
 
@@ -927,11 +964,7 @@ __global__ __launch_bounds__(256, BATCH && SHARE ? 6 : 8) void k_vis(KArgs ka, A
     } else {
         if (small) vis_raster_rect<T>(ar, V, rt, rc, s * 8u);
     }
-    const uint32_t cslot = wave_append(&ar.counters[CNT_CLIP_FACES], want_clip);
-    if (want_clip) {
-        if (cslot < ar.cap_clip_faces) ar.clip_faces[cslot] = g;
-        else set_error(ar, ERR_CLIP_FACES, CNT_NEED_CLIP_FACES, cslot + 1);
-    }
+    queue_clip(ar, want_clip, g);
     if ((want_clip && ka.skip_clip) || (big && ka.skip_big)) raise_error(ar, ERR_SKIPPED);
     big_append_wave(ar, big, r, area);
 }
@@ -1088,13 +1121,23 @@ template <int T, bool BATCH, bool VIS>
 __global__ __launch_bounds__(64 * CLIP_WAVES) void k_clip(KArgs ka, Arena ar) {
     __shared__ ClipWave lds[CLIP_WAVES];
     if (ar.counters[CNT_ERROR]) return;
-    const uint32_t n = imin((int)ar.counters[CNT_CLIP_FACES], (int)ar.cap_clip_faces);
     const int lane = (int)__lane_id();
+    // the sub-queues' entries, one sub-queue per lane, then the shared ones
+    const uint32_t cap = ar.clip_sub_cap;
+    const uint32_t have = cap ? (uint32_t)imin((int)ar.clip_next[lane * POOL_STRIDE], (int)cap) : 0u;
+    const uint32_t upto = wave_incl_scan(have), in_subs = __shfl(upto, 63);
+    const uint32_t n = in_subs + (uint32_t)imin((int)ar.counters[CNT_CLIP_FACES], (int)ar.cap_clip_faces);
     ClipWave* w = lds + (threadIdx.x >> 6);
     // the same queue entry for the whole wave
     for (uint32_t q = __builtin_amdgcn_readfirstlane(blockIdx.x * CLIP_WAVES + (threadIdx.x >> 6)); q < n;
          q += gridDim.x * CLIP_WAVES) {
-        const uint32_t g = __builtin_amdgcn_readfirstlane(ar.clip_faces[q]);
+        uint32_t entry = CLIP_SUBS * cap + (q - in_subs);
+        if (q < in_subs) {
+            const int sub = __popcll(__ballot(upto <= q));
+            entry = (uint32_t)sub * cap + q - (__shfl(upto, sub) - __shfl(have, sub));
+        }
+        entry = __builtin_amdgcn_readfirstlane(entry);
+        const uint32_t g = __builtin_amdgcn_readfirstlane(ar.clip_faces[entry]);
         uint32_t vi = 0;
         if constexpr (BATCH) vi = wave_find_le(ka.face_bases, ka.nviews, g);
         const ViewDesc& V = view_at<BATCH>(ka, vi);
@@ -1118,12 +1161,12 @@ __global__ __launch_bounds__(64 * CLIP_WAVES) void k_clip(KArgs ka, Arena ar) {
         for (int plane = 0; plane < 6 && count; ++plane) count = clip_plane_wave(w, cur, count, plane);
         const uint32_t ntri = (uint32_t)(count / 3);
         if (ntri == 0) continue;
-        // one or two pieces (all but the faces across several planes) go to
-        // the queue entry's own two records; one counter for every face would
-        // serialize them (~11 ns each, 0.3 ms over the 4M-triangle soup)
-        uint32_t base = 2u * q;
-        if (ntri > 2u || q >= ar.clip_static) {
-            if (lane == 0) base = 2u * ar.clip_static + atomicAdd(&ar.counters[CNT_CLIP_RECS], ntri);
+        // one or two pieces (all but the faces across several planes) of a
+        // sub-queue's entry go to its own two records, the others to records
+        // that one counter hands out
+        uint32_t base = 2u * entry;
+        if (ntri > 2u || entry >= CLIP_SUBS * cap) {
+            if (lane == 0) base = 2u * CLIP_SUBS * cap + atomicAdd(&ar.counters[CNT_CLIP_RECS], ntri);
             base = __builtin_amdgcn_readfirstlane(base);
         }
         if (base + ntri > ar.cap_clip_recs) {
@@ -1593,10 +1636,7 @@ __global__ __launch_bounds__(NT, raster_min_waves(SK)) void k_raster(KArgs ka, A
     if (failed && !clear) return;
     if (blockIdx.x == 0 && !failed) {
         // the per-frame counters were last needed by k_clip
-        if (threadIdx.x == 0) {
-            ar.counters[CNT_CLIP_FACES] = 0;
-            ar.counters[CNT_CLIP_RECS] = 0;
-        }
+        reset_clip_counters(ar);
         for (uint32_t i = threadIdx.x; i <= POOL_SUBS; i += NT) ar.pool_next[i * POOL_STRIDE] = 0;
     }
     const uint32_t x = blockIdx.x % NUM_XCD, j = blockIdx.x / NUM_XCD;
@@ -1807,11 +1847,10 @@ __global__ __launch_bounds__(256) void k_resolve(KArgs ka, Arena ar) {
     const bool failed = ar.counters[CNT_ERROR] != 0u;
     const ClearSpec cs{ka.clear != 0, ka.clear_bgra, ka.clear_depth};
     if (failed && !cs.on) return;
-    if (!failed && blockIdx.x == 0 && threadIdx.x == 0) {
+    if (!failed && blockIdx.x == 0) {
         // the per-frame counters of this mode were last needed by k_big
-        ar.counters[CNT_CLIP_FACES] = 0;
-        ar.counters[CNT_CLIP_RECS] = 0;
-        *big_counter(ar) = 0ull;
+        reset_clip_counters(ar);
+        if (threadIdx.x == 0) *big_counter(ar) = 0ull;
     }
     if constexpr (T == 8) {
         // one wave per bin
@@ -1870,11 +1909,10 @@ template <int T, int SK, bool IDS, bool INSIDE = false>
 __global__ __launch_bounds__(256, (INSIDE && !IDS && SK != SHADER_PBR) ? 7 : 1) void k_shade(KArgs ka, Arena ar) {
     using S = typename ShaderOf<SK>::type;
     if (ar.counters[CNT_ERROR]) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (blockIdx.x == 0) {
         // the per-frame counters of this mode were last needed by k_big
-        ar.counters[CNT_CLIP_FACES] = 0;
-        ar.counters[CNT_CLIP_RECS] = 0;
-        *big_counter(ar) = 0ull;
+        reset_clip_counters(ar);
+        if (threadIdx.x == 0) *big_counter(ar) = 0ull;
     }
     const ViewDesc& V = ka.one;
     unsigned long long* vk = ar.vkeys + V.pix_base;
