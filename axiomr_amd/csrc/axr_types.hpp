@@ -83,6 +83,8 @@ struct ViewDesc {
                                    // mesh (the shader's Var type), computed by k_vary
                                    // earlier in the same launch; null: run it per pixel
     DevGroup g0;                   // groups[0], for single-group meshes without a load
+    DevGroup g1, g2, g3;           // groups[1..3], so that meshes of up to four groups are
+                                   // searched without loads (plain draws)
     uint32_t ngroups;
     uint32_t nfaces;               // faces in submission order (sum of group counts)
     // transform

@@ -578,6 +578,9 @@ ViewDesc make_view(const axr_mesh* m, uint32_t* color, float* depth, uint32_t* i
     v.face_colors = m->face_colors;
     v.groups = m->groups;
     v.g0 = m->g0;
+    v.g1 = m->more[0];
+    v.g2 = m->more[1];
+    v.g3 = m->more[2];
     v.materials = m->materials;
     v.ngroups = m->ngroups;
     v.nfaces = m->nfaces_sub;
@@ -902,6 +905,7 @@ int axr_mesh_create(axr_ctx* ctx, const float* verts56, uint64_t nverts, const u
     m->nmaterials = nmaterials;
     m->nfaces_sub = (uint32_t)rank;
     m->g0 = dg[0];
+    for (uint32_t g = 1; g < ngroups && g < 4; ++g) m->more[g - 1] = dg[g];
     std::vector<float> pos(3 * nverts);
     for (uint64_t i = 0; i < nverts; ++i)
         for (int k = 0; k < 3; ++k) pos[3 * i + k] = verts56[14 * i + k];

@@ -150,6 +150,7 @@ struct axr_mesh {
     uint32_t nfaces_sub = 0;   // faces in submission order
     uint32_t batch_refs = 0;   // views of live batches that draw this mesh
     axr::DevGroup g0{};        // first group (host copy)
+    axr::DevGroup more[3] = {};   // the next three, if there are
     size_t bytes = 0;
     // model-space bounds, for deciding on the host that a draw needs no
     // clipper or large-triangle pass: a sphere holding every vertex and the

@@ -77,8 +77,20 @@ __device__ __forceinline__ uint32_t wave_view_of(const uint32_t* bases, uint32_t
     return g < bases[v0 + 1] ? v0 : find_le(bases, nviews, g);
 }
 
+// The group of submission rank `rank`: the last one that starts at or before
+// it.  FEW: groups 1 to 3 are taken from the view (the kernel's arguments, in
+// scalar registers); the search in memory is two or three dependent loads
+// before a face's indices can be loaded.
+template <bool FEW>
 __device__ __forceinline__ DevGroup group_of(const ViewDesc& V, uint32_t rank) {
     if (V.ngroups == 1) return V.g0;
+    if (FEW && V.ngroups <= 4) {
+        DevGroup g = V.g0;
+        if (V.g1.rank_base <= rank) g = V.g1;
+        if (V.ngroups > 2 && V.g2.rank_base <= rank) g = V.g2;
+        if (V.ngroups > 3 && V.g3.rank_base <= rank) g = V.g3;
+        return g;
+    }
     uint32_t lo = 0, hi = V.ngroups;
     while (hi - lo > 1) {
         uint32_t mid = (lo + hi) >> 1;
@@ -100,8 +112,9 @@ struct FaceGeo {
     vec4 c0, c1, c2;
 };
 
+template <bool BATCH>
 __device__ __forceinline__ void face_geo(const ViewDesc& V, uint32_t s, FaceGeo& f) {
-    f.G = group_of(V, s);
+    f.G = group_of<!BATCH>(V, s);
     f.face = f.G.first + (s - f.G.rank_base);
     const uint3 ix = gld(reinterpret_cast<const uint3*>(V.idx), f.face);
     f.i0 = ix.x;
@@ -717,14 +730,14 @@ __device__ __forceinline__ void store_rec_nt(TriRec* p, const TriRec& r) {
 }
 
 // Face slot g of view V (all 64 lanes of the wave call it).
-template <int T, bool INSIDE>
+template <int T, bool BATCH, bool INSIDE>
 __device__ __forceinline__ void setup_face(const KArgs& ka, const Arena& ar, uint32_t g, bool active, const ViewDesc& V) {
     bool want_clip = false, binnable = false;
     Rect rc{0, 0, 0, 0};
     if (active) {
         const uint32_t s = g - V.face_base;
         FaceGeo f;
-        face_geo(V, s, f);
+        face_geo<BATCH>(V, s, f);
         int cls = CLS_INSIDE;
         if constexpr (!INSIDE) cls = classify(f.c0, f.c1, f.c2);
         want_clip = cls == CLS_CLIP;
@@ -766,23 +779,23 @@ __global__ __launch_bounds__(256) void k_setup(KArgs ka, Arena ar) {
             // the whole wave in one view (the usual case): the view's fields
             // in scalar registers, loaded once for the wave
             const ViewDesc V = wave_uniform(ka.table[v0]);
-            if (INSIDE || V.inside) setup_face<T, true>(ka, ar, g, active, V);
-            else setup_face<T, false>(ka, ar, g, active, V);
+            if (INSIDE || V.inside) setup_face<T, BATCH, true>(ka, ar, g, active, V);
+            else setup_face<T, BATCH, false>(ka, ar, g, active, V);
         } else {
-            setup_face<T, INSIDE>(ka, ar, g, active, ka.table[vi]);
+            setup_face<T, BATCH, INSIDE>(ka, ar, g, active, ka.table[vi]);
         }
     } else {
-        setup_face<T, INSIDE>(ka, ar, g, active, ka.one);
+        setup_face<T, BATCH, INSIDE>(ka, ar, g, active, ka.one);
     }
 }
 
 // ---------------------------------------------------------------------------
 // Walks of triangles' pixel rectangles by a wave (k_vis, k_raster): a lane
-// walks at most WALK_CAP pixels of its own rectangle, the rest of every
-// longer one is cut into pieces of WALK_CAP pixels that the wave's lanes take
-// in turn.  What a walker needs of a triangle, per lane, and the first piece
-// of each lane in the wave's numbering:
-constexpr int WALK_CAP = 8;
+// walks at most CAP pixels of its own rectangle, the rest of every longer one
+// is cut into pieces of CAP pixels that the wave's lanes take in turn.  What a
+// walker needs of a triangle, per lane, and the first piece of each lane in
+// the wave's numbering:
+constexpr int VIS_CAP = 8;
 struct WalkPieces {
     float4 e0[64];        // a0, b0, c0, a1
     float4 e1[64];        // b1, c1, a2, b2
@@ -816,8 +829,8 @@ __device__ __forceinline__ void get_piece(const WalkPieces* wp, const Arena&, ui
 // faces that cross a plane go to the clipper.
 
 // SHARE: where a rectangle of the wave outlasts VIS_SHARE pixels, its lanes
-// would idle while one walks it; then a lane walks WALK_CAP pixels of its own
-// rectangle and the rest goes in pieces of WALK_CAP to all lanes in turn, as
+// would idle while one walks it; then a lane walks VIS_CAP pixels of its own
+// rectangle and the rest goes in pieces of VIS_CAP to all lanes in turn, as
 // in k_raster.  At 1080p k_vis takes 38 us without and 18 with it for 32,000
 // faces, 22 and 10 for 2,000; but 21.2 and 22.1 for a million faces and 23.0
 // and 24.3 for 200,000, whose rectangles are a few pixels.  So the host takes
@@ -864,8 +877,8 @@ __device__ __forceinline__ void vis_walk_wave(VisPieces* wp, const KArgs& ka, co
                                               const Rect& rc, uint32_t vi, uint32_t key) {
     const uint32_t lane = __lane_id();
     const int w = on ? rc.x1 - rc.x0 : 0, fp = on ? w * (rc.y1 - rc.y0) : 0;
-    if (on) vis_span<T>(ar, view_at<BATCH>(ka, vi), rt, rc.x0, rc.y0, w, 0, imin(fp, WALK_CAP), key, 0.0f);
-    const uint32_t pieces = fp > WALK_CAP ? (uint32_t)(fp - 1) / WALK_CAP : 0u;
+    if (on) vis_span<T>(ar, view_at<BATCH>(ka, vi), rt, rc.x0, rc.y0, w, 0, imin(fp, VIS_CAP), key, 0.0f);
+    const uint32_t pieces = fp > VIS_CAP ? (uint32_t)(fp - 1) / VIS_CAP : 0u;
     const uint32_t incl = wave_incl_scan(pieces), total = __shfl(incl, 63);
     wp->start[lane] = incl - pieces;
     if (pieces) {
@@ -882,9 +895,9 @@ __device__ __forceinline__ void vis_walk_wave(VisPieces* wp, const KArgs& ka, co
         uint32_t rect, pkey;
         get_piece(wp, ar, o, t, rect, pkey);
         const int tw = (int)(wp->size[o] & 0xFFFFu), th = (int)(wp->size[o] >> 16);
-        const int q0 = WALK_CAP * (int)(j - wp->start[o] + 1);
+        const int q0 = VIS_CAP * (int)(j - wp->start[o] + 1);
         vis_span<T>(ar, view_at<BATCH>(ka, BATCH ? wp->view[o] : 0u), t, (int)(rect & 0xFFFFu), (int)(rect >> 16), tw, q0,
-                    imin(q0 + WALK_CAP, tw * th), pkey, 1.0f / (float)tw);
+                    imin(q0 + VIS_CAP, tw * th), pkey, 1.0f / (float)tw);
     }
 }
 
@@ -904,7 +917,7 @@ __global__ __launch_bounds__(256, BATCH && SHARE ? 6 : 8) void k_vis(KArgs ka, A
     vec3 p0, p1, p2;
     if (act) {
         s = g - V.face_base;
-        G = group_of(V, s);
+        G = group_of<!BATCH>(V, s);
         face = G.first + (s - G.rank_base);
         const uint3 ix = gld(reinterpret_cast<const uint3*>(V.idx), face);
         p0 = load_pos(V.pos, ix.x);
@@ -1142,7 +1155,7 @@ __global__ __launch_bounds__(64 * CLIP_WAVES) void k_clip(KArgs ka, Arena ar) {
         if constexpr (BATCH) vi = wave_find_le(ka.face_bases, ka.nviews, g);
         const ViewDesc& V = view_at<BATCH>(ka, vi);
         const uint32_t s = g - V.face_base;
-        const DevGroup G = group_of(V, s);
+        const DevGroup G = group_of<!BATCH>(V, s);
         const uint32_t face = G.first + (s - G.rank_base);
         int cur = 0;
         wave_lds_fence();   // the previous face's reads of the polygon are done
@@ -1281,7 +1294,7 @@ __device__ __forceinline__ vec4 shade_winner(const ViewDesc& V, const Arena& ar,
                                             bool clipped, uint32_t rank, vec3 bar, const DevMaterial* um = nullptr) {
     uint32_t prim, i0 = 0, i1 = 0, i2 = 0;
     if (clipped) {
-        const DevGroup G = group_of(V, rank);
+        const DevGroup G = group_of<false>(V, rank);
         prim = G.first + (rank - G.rank_base);
     } else {
         prim = r.c.z;
@@ -1412,13 +1425,13 @@ __device__ __forceinline__ void resolve_tile_kind(const ViewDesc& V, const Arena
 }
 
 // ---------------------------------------------------------------------------
-// Coverage of a bin's small triangles.  One lane per triangle walks its
-// pixel rectangle (bbox within the bin), which leaves most lanes idle while
-// the wave waits for its largest rectangle: on the 256-view batch the
-// rectangles average 11.5 pixels but a wave's largest is far bigger, and
-// 42% of the lane slots did work.  So a lane walks at most WALK_CAP pixels
-// of its own rectangle; the rest of every longer rectangle is cut into
-// pieces of WALK_CAP pixels that the wave's lanes then take in turn.
+// Coverage of a bin's triangles.  One lane per triangle walking its pixel
+// rectangle (bbox within the bin) leaves most lanes idle while the wave waits
+// for its largest rectangle: on the 256-view batch the rectangles average 11.5
+// pixels but a wave's largest is far bigger, and 42% of the lane slots did
+// work.  So the walks are capped and shared.  The cap weighs idle lanes
+// against the pieces' own cost: a search, then the edge setup from LDS or from
+// the record again (below).
 
 // Pixels [q0, q1) of the rectangle [x0, x0 + w) x [y0, ...) (bin coordinates)
 // in row-major order; every covered pixel takes the minimum of its key.
@@ -1466,7 +1479,7 @@ __device__ __forceinline__ void walk_span(const RasterTri& rt, int x0, int y0, i
     }
 }
 
-// A wave's triangles whose rectangles outlast WALK_CAP pixels, for the
+// A wave's triangles whose rectangles outlast the cap, for the
 // pieces: per lane what a walker needs of its triangle, and the first piece
 // of each lane in the wave's numbering.  Two layouts:
 //   WalkPieces  the edge setup itself, rectangle and key (17 words a lane);
@@ -1480,6 +1493,13 @@ struct WalkRefs {
     uint32_t start[64];
 };
 // rect: x0 | y0 << 8 | w << 16 | h << 24, in bin coordinates
+//
+// Pixels per piece.  k_raster in us with 4, 8 and 12: a 150k soup at 16 px
+// 20.6, 22.2, 25.0 and 12 PBR objects 17.3, 18.4, 20.2 with the edge setup in
+// LDS; with references the 1M-triangle frame at 16 px 43.7, 41.5, - and 40
+// mixed views at 32 px 218, 215, 202.
+template <int T, class P> constexpr int kWalkCap = T == 32 ? 8 : 4;
+template <int T> constexpr int kWalkCap<T, WalkRefs> = T == 32 ? 12 : 8;
 
 __device__ __forceinline__ void put_piece(WalkRefs* wp, uint32_t lane, const RasterTri&, uint32_t ref, uint32_t rect,
                                           uint32_t) {
@@ -1500,9 +1520,10 @@ __device__ __forceinline__ void get_piece(const WalkRefs* wp, const Arena& ar, u
 template <int T, class P>
 __device__ __forceinline__ void walk_wave(P* wp, const Arena& ar, const RasterTri& rt, uint32_t ref, int x0, int y0,
                                           int w, int h, uint32_t key, unsigned long long* keys, int ox, int oy) {
+    constexpr int CAP = kWalkCap<T, P>;
     const int fp = w * h;
-    walk_span<T>(rt, x0, y0, w, 0, imin(fp, WALK_CAP), key, keys, ox, oy, 0.0f);
-    const uint32_t pieces = fp > WALK_CAP ? (uint32_t)(fp - 1) / WALK_CAP : 0u;
+    walk_span<T>(rt, x0, y0, w, 0, imin(fp, CAP), key, keys, ox, oy, 0.0f);
+    const uint32_t pieces = fp > CAP ? (uint32_t)(fp - 1) / CAP : 0u;
     const uint32_t incl = wave_incl_scan(pieces);
     const uint32_t total = __shfl(incl, 63);
     if (total == 0) return;
@@ -1523,8 +1544,8 @@ __device__ __forceinline__ void walk_wave(P* wp, const Arena& ar, const RasterTr
         get_piece(wp, ar, o, t, rect, pkey);
         const int rx = (int)(rect & 255u), ry = (int)((rect >> 8) & 255u);
         const int rw = (int)((rect >> 16) & 255u), rh = (int)(rect >> 24);
-        const int q0 = WALK_CAP * (int)(j - wp->start[o] + 1);
-        walk_span<T>(t, rx, ry, rw, q0, imin(q0 + WALK_CAP, rw * rh), pkey, keys, ox, oy, 1.0f / (float)rw);
+        const int q0 = CAP * (int)(j - wp->start[o] + 1);
+        walk_span<T>(t, rx, ry, rw, q0, imin(q0 + CAP, rw * rh), pkey, keys, ox, oy, 1.0f / (float)rw);
     }
 }
 
@@ -1713,7 +1734,7 @@ __device__ __forceinline__ bool shade_vis_pixel(const ViewDesc& V, const Arena& 
                                                 int py, float dfb, float& z, uint32_t& bgra) {
     const uint32_t key = (uint32_t)k;
     const uint32_t s = key >> 3, j = key & 7u;
-    const DevGroup G = group_of(V, s);
+    const DevGroup G = group_of<!VARY>(V, s);
     const uint32_t face = G.first + (s - G.rank_base);
     const uint3 ix = gld(reinterpret_cast<const uint3*>(V.idx), face);
     const uint32_t i0 = ix.x, i1 = ix.y, i2 = ix.z;

@@ -96,3 +96,30 @@ def test_binned_clear_in_the_raster(tile, threads, depth):
             gs.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("mode", list(MODES))
+@pytest.mark.parametrize("counts", [(700, 0, 580), (1, 638, 0, 641), (3, 5, 7, 11, 1254), (0, 0, 1280)])
+def test_material_groups(mode, counts):
+    """Two to five groups (up to four are searched without loads), empty ones
+    among them, submitted in another order than the index buffer's, with a
+    material each."""
+    base = S.icosphere_scene(n=8, width=320, height=240, tex=64)
+    first = np.cumsum((0,) + counts[:-1])
+    order = list(range(len(counts)))[::-1]
+    mats, tex = [], dict(base.textures)
+    for i in range(len(counts)):
+        tex[f"albedo{i}"] = S.TextureData(S.noise_texture(32, 32, 50 + i), i % 2)
+        mats.append(S.MaterialData(diffuse=f"albedo{i}", bump="normal", specular_exponent=0.3 + 0.2 * i))
+    sc = S.with_shader(base, base.shader, materials=mats, textures=tex)
+    sc.groups = [(i, int(first[i]), int(counts[i])) for i in order]
+    assert sum(counts) == sc.nfaces
+    ctx = R.Context(0)
+    try:
+        ctx.set_config(raster_mode=MODES[mode])
+        ref = H.render_oracle(sc)
+        rep = H.compare(H.render_gpu(ctx, sc), ref)
+        H.assert_parity(rep, f"{mode} groups {counts}")
+        assert rep["covered"] > 1000
+    finally:
+        ctx.close()
