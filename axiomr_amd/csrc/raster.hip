@@ -1291,21 +1291,13 @@ __device__ __forceinline__ vec4 shade_at(const ViewDesc& V, const Arena& ar, uin
 
 template <class S>
 __device__ __forceinline__ vec4 shade_winner(const ViewDesc& V, const Arena& ar, const TriRec& r, uint32_t slot,
-                                            bool clipped, uint32_t rank, vec3 bar, const DevMaterial* um = nullptr) {
-    uint32_t prim, i0 = 0, i1 = 0, i2 = 0;
+                                            bool clipped, uint32_t rank, uint3 ix, vec3 bar, const DevMaterial* um = nullptr) {
+    uint32_t prim = r.c.z;
     if (clipped) {
         const DevGroup G = group_of<false>(V, rank);
         prim = G.first + (rank - G.rank_base);
-    } else {
-        prim = r.c.z;
-        if constexpr (sizeof(typename S::Var) > 1) {
-            const uint3 ix = gld(reinterpret_cast<const uint3*>(V.idx), prim);
-            i0 = ix.x;
-            i1 = ix.y;
-            i2 = ix.z;
-        }
     }
-    return shade_at<S>(V, ar, r.c.w, prim, clipped, slot, i0, i1, i2, bar, um);
+    return shade_at<S>(V, ar, r.c.w, prim, clipped, slot, ix.x, ix.y, ix.z, bar, um);
 }
 
 // A clear that a draw absorbs (its values; on = false: none).
@@ -1342,24 +1334,31 @@ __device__ __forceinline__ void resolve_pixel(const ViewDesc& V, const Arena& ar
                                               bool known, float known_depth, const ClearSpec& cs, const DevMaterial* um) {
     const uint32_t key = (uint32_t)k;
     const uint32_t rank = key >> 3, j = key & 7u;
+    // the framebuffer's depth is under way with the record, the corners'
+    // indices during the edge setup
+    const size_t pix = (size_t)py * (size_t)V.W + (size_t)px;
+    float dfb = known_depth;
+    if (!known) dfb = gld(V.depth, pix);
     TriRec r = ar.rec[V.face_base + rank];
     bool clipped = false;
     uint32_t slot = 0;
+    uint3 ix = make_uint3(0u, 0u, 0u);
     if (r.c.w & REC_CLIPPED) {
         clipped = true;
         slot = r.c.z + j;
         r = ar.clip_rec[slot];
+    } else if constexpr (sizeof(typename S::Var) > 1) {
+        ix = gld(reinterpret_cast<const uint3*>(V.idx), r.c.z);
     }
     RasterTri rt;
     raster_setup(r, rt);
     float al, be, ga, z;
     cover(rt, px, py, al, be, ga, z);
-    const size_t pix = (size_t)py * (size_t)V.W + (size_t)px;
-    if (!(z < (known ? known_depth : gld(V.depth, pix)))) {   // reference mergeTileResults: strict less
+    if (!(z < dfb)) {   // reference mergeTileResults: strict less
         if (cs.on) clear_pixel(V, pix, cs);
         return;
     }
-    const vec4 col = shade_winner<S>(V, ar, r, slot, clipped, rank, make3(al, be, ga), um);
+    const vec4 col = shade_winner<S>(V, ar, r, slot, clipped, rank, ix, make3(al, be, ga), um);
     gst_nt(V.depth, pix, z);
     gst_nt(V.color, pix, pack_bgra(col));
     if (V.ids) gst_nt(V.ids, pix, key);
@@ -1561,11 +1560,17 @@ __device__ __forceinline__ const ViewDesc& bin_view(const KArgs& ka, const ViewD
     else return ka.one;
 }
 
+// The entry a lane takes first.  Entries go to the waves in turn, so that a
+// bin with fewer entries than the workgroup has lanes keeps every wave at work.
+template <int NT>
+__device__ __forceinline__ uint32_t bin_lane() { return (threadIdx.x & 63u) * (NT / 64) + (threadIdx.x >> 6); }
+
+// ref: the lane's first entry, if that lies in the bin's first level.
 // sview (batches): the bin's view is copied into LDS once per bin, so that
 // every per-pixel read of its uniforms and pointers is an LDS read.
 template <int T, int NT, bool BATCH, int SK>
-__device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uint32_t t, uint32_t n, unsigned long long* keys,
-                                           uint32_t& ncov, uint16_t* plist, ViewDesc* sview,
+__device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uint32_t t, uint32_t n, uint32_t ref,
+                                           unsigned long long* keys, uint32_t& ncov, uint16_t* plist, ViewDesc* sview,
                                            typename PiecesOf<SK>::type* pieces) {
     if constexpr (BATCH) {
         const uint32_t vi = ka.tile_views[t];
@@ -1583,18 +1588,19 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
     // every wave has read n: the count is consumed, leave it zero for the next frame
     if (threadIdx.x == 0) ar.tile_count[count_word(t)] = 0;
 
-    // entries go to the waves in turn, so that a bin with fewer entries than
-    // the workgroup has lanes keeps every wave at work
     typename PiecesOf<SK>::type* wp = pieces + (threadIdx.x >> 6);
-    const uint32_t first = (threadIdx.x & 63u) * (NT / 64) + (threadIdx.x >> 6);
+    uint32_t next = bin_lane<NT>();
+    if ((next >> ar.bin0_shift) != 0u && next < n) ref = bin_get(ar, t, next);
     for (uint32_t b0 = 0; b0 < n; b0 += NT) {
-        const uint32_t i = b0 + first;
+        const uint32_t i = next, mine = ref;
         RasterTri rt;
         int x0 = 0, y0 = 0, w = 0, h = 0;
-        uint32_t key = 0, ref = 0;
+        uint32_t key = 0;
+        TriRec r;
+        if (i < n) r = rec_of(ar, mine);
+        next += NT;
+        if (next < n) ref = bin_get(ar, t, next);   // arrives during the walk
         if (i < n) {
-            ref = bin_get(ar, t, i);
-            const TriRec r = rec_of(ar, ref);
             if (raster_setup(r, rt)) {
                 x0 = imax(ox, rt.fx0);
                 y0 = imax(oy, rt.fy0);
@@ -1604,7 +1610,7 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
                 key = r.c.y;
             }
         }
-        walk_wave<T>(wp, ar, rt, ref, x0 - ox, y0 - oy, w, h, key, keys, ox, oy);
+        walk_wave<T>(wp, ar, rt, mine, x0 - ox, y0 - oy, w, h, key, keys, ox, oy);
         wave_lds_fence();   // the pieces are read before the next entries' are written
     }
     __syncthreads();
@@ -1662,7 +1668,20 @@ __global__ __launch_bounds__(NT, raster_min_waves(SK)) void k_raster(KArgs ka, A
     __shared__ uint32_t ncov;
     __shared__ ViewDesc sview[1];
     __shared__ typename PiecesOf<SK>::type pieces[NT / 64];
-    const bool failed = ar.counters[CNT_ERROR] != 0u;
+    // A bin that few others share the chip with is a chain of trips to memory,
+    // up to 0.9 us each for what another XCD wrote: the error word, the count
+    // and the lanes' first entries leave together (as the framebuffer's depth
+    // does with the record in resolve_pixel, and the indices during the edge
+    // setup).  512 flat faces at 256x256: 9.1 -> 8.4 us with the launch; twelve
+    // PBR draws at 1241x719: 17.5 -> 16.8 each; 40 mixed views: 202 -> 193.
+    const uint32_t t = bin_of_block(blockIdx.x), error = ar.counters[CNT_ERROR];
+    uint32_t count = 0, ref = 0;
+    if (t < ka.total_tiles) {
+        count = ar.tile_count[count_word(t)];
+        const uint32_t i = bin_lane<NT>();
+        if ((i >> ar.bin0_shift) == 0u) ref = ar.bins[((size_t)t << ar.bin0_shift) + i];
+    }
+    const bool failed = error != 0u;
     const bool clear = !BATCH && ka.clear != 0;
     if (failed && !clear) return;
     if (blockIdx.x == 0 && !failed) {
@@ -1670,9 +1689,8 @@ __global__ __launch_bounds__(NT, raster_min_waves(SK)) void k_raster(KArgs ka, A
         reset_clip_counters(ar);
         for (uint32_t i = threadIdx.x; i <= POOL_SUBS; i += NT) ar.pool_next[i * POOL_STRIDE] = 0;
     }
-    const uint32_t t = bin_of_block(blockIdx.x);
     if (t >= ka.total_tiles) return;
-    const uint32_t n = failed ? 0u : ar.tile_count[count_word(t)];
+    const uint32_t n = failed ? 0u : count;
     if (n == 0u) {
         // an empty bin, or a failed frame: only the clear, if the draw absorbs
         // one, as a separate clear pass would have
@@ -1683,7 +1701,7 @@ __global__ __launch_bounds__(NT, raster_min_waves(SK)) void k_raster(KArgs ka, A
         }
         return;
     }
-    raster_bin<T, NT, BATCH, SK>(ka, ar, t, n, keys, ncov, plist, sview, pieces);
+    raster_bin<T, NT, BATCH, SK>(ka, ar, t, n, ref, keys, ncov, plist, sview, pieces);
 }
 
 // ---------------------------------------------------------------------------
@@ -1881,7 +1899,11 @@ __device__ __forceinline__ void resolve_vis_tile_kind(const ViewDesc& V, const A
 // batch's views carry vertex-stage outputs (VARY = BATCH).
 template <int T, bool BATCH, int SK, bool INSIDE = false>
 __global__ __launch_bounds__(256) void k_resolve(KArgs ka, Arena ar) {
-    const bool failed = ar.counters[CNT_ERROR] != 0u;
+    // the bin's flag leaves with the error word (as in k_raster)
+    const uint32_t t = bin_of_block(blockIdx.x), error = ar.counters[CNT_ERROR];
+    uint32_t flag = 0;
+    if (T > 8 && t < ka.total_tiles) flag = ar.tile_count[t];
+    const bool failed = error != 0u;
     const ClearSpec cs{ka.clear != 0, ka.clear_bgra, ka.clear_depth};
     if (failed && !cs.on) return;
     if (!failed && blockIdx.x == 0) {
@@ -1908,9 +1930,8 @@ __global__ __launch_bounds__(256) void k_resolve(KArgs ka, Arena ar) {
         }
     } else {
         // one workgroup (four waves, a pixel or more per thread) per bin
-        const uint32_t t = bin_of_block(blockIdx.x);
         if (t >= ka.total_tiles) return;
-        const bool keys = !failed && ar.tile_count[t] != 0u;
+        const bool keys = flag != 0u && !failed;
         if (!keys && !cs.on) return;
         uint32_t vi = 0;
         if constexpr (BATCH) vi = ka.tile_views[t];
