@@ -720,7 +720,7 @@ __device__ __forceinline__ uint32_t face_slot(const KArgs& ka) {
 }
 
 // A triangle record stored with the non-temporal hint: the batch's records
-// far exceed the caches and are read back only after the scatter.
+// far exceed the caches and are read back only by the raster.
 __device__ __forceinline__ void store_rec_nt(TriRec* p, const TriRec& r) {
     typedef unsigned int v4u __attribute__((ext_vector_type(4)));
     v4u* q = reinterpret_cast<v4u*>(p);
