@@ -1,12 +1,12 @@
 """Autotuner for the render path's tunables (axr_config): raster mode
 (binned / visibility buffer), bin edge (8/16/32 px), threads per bin
-workgroup (64/128/256), per-wave bin-pair capacity (64..1024, binned mode)
-and the one-lane footprint threshold.  None of them changes a pixel; they
+workgroup (64/128/256), bin capacity (64..1024, binned mode; without effect
+since bins grow by themselves) and the one-lane footprint threshold.  None of them changes a pixel; they
 only move time between the kernels.
 
 Coordinate descent, two rounds: raster mode x bin edge x workgroup size
 (18 points), then the bin capacity (binned mode only; the smallest within
-1 % of the fastest, since it sizes memory), then the footprint threshold,
+1 % of the fastest), then the footprint threshold,
 each point timed as the median of a few synchronised runs of the
 caller's frame function.  Results are cached in a JSON file keyed by device
 and workload name.
@@ -98,9 +98,8 @@ def tune(ctx, make_frame: Callable[[], Callable[[], None]], log: Optional[Callab
         if best.get("raster_mode", 0) == 0:
             for cap in CAPACITIES:
                 consider({**best, "bin_capacity": cap})
-            # the capacity sizes the per-wave pair regions (setup waves x
-            # capacity x 16 B): take the smallest within CAPACITY_SLACK of
-            # the fastest, whose edge is below the timing noise
+            # take the smallest within CAPACITY_SLACK of the fastest, whose
+            # edge is below the timing noise
             times = {t["bin_capacity"]: t["seconds"] for t in trials
                      if all(t[k] == v for k, v in best.items() if k != "bin_capacity")}
             for cap in sorted(times):

@@ -153,8 +153,8 @@ constexpr uint32_t ERR_BIG = 8u;
 constexpr uint32_t ERR_SKIPPED = 16u;   // a pass the host skipped had work: the frame is redrawn with it
 
 // Bins of binned mode: level k of a bin holds 2^(bin0_shift + k) entries, so
-// BIN_LEVELS levels reach past 2^31 entries for the smallest first level.
-constexpr uint32_t BIN0_MIN_SHIFT = 5, BIN0_MAX_SHIFT = 12;
+// BIN_LEVELS levels reach 2^31 entries for the smallest first level.
+constexpr uint32_t BIN0_LEAN_SHIFT = 4, BIN0_MIN_SHIFT = 5, BIN0_MAX_SHIFT = 12;
 constexpr uint32_t COUNT_BLOCK = 8192;         // words of tile_count that bins are spread over
 constexpr uint32_t BIN_LEVELS = 27;
 constexpr uint32_t CHUNK_NONE = 0xFFFFFFFFu;   // a level the pools had no room for

@@ -106,7 +106,7 @@ static void free_buf(axr_ctx* ctx, DevBuf& b) {
 
 static int grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, DevBuf& b, size_t bytes) {
     if (b.bytes >= bytes) return AXR_OK;
-    bytes = std::max(bytes, b.bytes + b.bytes / 4);
+    if (!fa.lean) bytes = std::max(bytes, b.bytes + b.bytes / 4);
     hipError_t e = hipStreamSynchronize(fa.stream);
     if (e != hipSuccess) return hip_fail(err, e, "sync before arena growth");
     free_buf(ctx, b);
@@ -150,17 +150,26 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     const uint64_t clip_faces = std::max<uint64_t>(want_clip, a.cap_clip_faces);
     // the sub-queues beside the shared queue of clip_faces entries, and their
     // two records each beside the 2 clip_faces others
-    const uint64_t clip_sub = std::max<uint64_t>({4096 / CLIP_SUBS, want_clip / 8 / CLIP_SUBS, a.clip_sub_cap});
+    const uint64_t clip_sub =
+        fa.lean ? 0 : std::max<uint64_t>({4096 / CLIP_SUBS, want_clip / 8 / CLIP_SUBS, a.clip_sub_cap});
     const uint64_t clip_recs = std::max<uint64_t>({2 * CLIP_SUBS * clip_sub + 2 * clip_faces, need.clip_recs, a.cap_clip_recs});
     // binned mode: the first level of a bin holds four times the mean of faces
     // per bin (a power of two of at least 32 entries), the shared pool what
     // any spread of 2 faces + 16 bins + 4096 entries over the bins needs (a
     // bin's further levels hold less than twice its entries), the sub-pools
-    // half as much again
-    uint32_t bin0_shift = BIN0_MIN_SHIFT;
-    while (bin0_shift < BIN0_MAX_SHIFT && (tiles << bin0_shift) < 4 * faces) ++bin0_shift;
+    // half as much again.  An arena that an HBM budget counts (lean: a
+    // context with one, a server's lanes) has smaller first levels and
+    // sub-pools and no sub-queues for the clipper, and so takes no more than
+    // 28 bytes a face and 332 a bin beside the records, what an arena with
+    // sorted pairs took, which budgets were chosen for: what fitted one still
+    // fits.
+    uint32_t bin0_shift = fa.lean ? BIN0_LEAN_SHIFT : BIN0_MIN_SHIFT;
+    while (bin0_shift < BIN0_MAX_SHIFT &&
+           (fa.lean ? (tiles << (bin0_shift + 1)) <= (tiles << BIN0_LEAN_SHIFT) + faces : (tiles << bin0_shift) < 4 * faces))
+        ++bin0_shift;
     const uint64_t pool = std::max<uint64_t>({2 * (2 * faces + 16 * tiles + 4096), need.pairs, a.pool_cap});
-    const uint64_t sub = std::max<uint64_t>((2 * faces + 16 * tiles + 4096) / POOL_SUBS, a.sub_cap);
+    const uint64_t sub =
+        std::max<uint64_t>((fa.lean ? 2 * faces : 2 * faces + 16 * tiles + 4096) / POOL_SUBS, a.sub_cap);
     // visibility mode: large triangles and their 256-pixel work items
     uint64_t big_recs = 0, big_items = 0;
     if (fs.pixels) {
@@ -171,7 +180,7 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     int r;
     if ((r = grow(ctx, err, fa, fa.counters, CNT_COUNT * 4)) ||
         (r = grow(ctx, err, fa, fa.rec, std::max<uint64_t>(faces, 1) * (vis ? 4 : sizeof(TriRec)))) ||
-        (r = grow(ctx, err, fa, fa.clip_next, CLIP_SUBS * POOL_STRIDE * 4)) ||
+        (r = grow(ctx, err, fa, fa.clip_next, clip_sub ? CLIP_SUBS * POOL_STRIDE * 4 : 0)) ||
         (r = grow(ctx, err, fa, fa.clip_faces, (CLIP_SUBS * clip_sub + clip_faces) * 4)))
         return r;
     if ((r = grow(ctx, err, fa, fa.clip_rec, clip_recs * sizeof(TriRec))) ||
@@ -289,7 +298,8 @@ void sig_release(int device, uint64_t* p) {
 constexpr uint32_t HOST_ERR_WORD = (CNT_COUNT + 31) / 32 * 32 + 32;
 constexpr uint32_t HOST_DONE_WORD = HOST_ERR_WORD + 32;
 
-int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa) {
+int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa, bool lean) {
+    fa.lean = lean || ctx->budget != 0;
     hipError_t e = hipStreamCreateWithFlags(&fa.stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipHostMalloc((void**)&fa.host_counters, (HOST_DONE_WORD + 32) * 4, hipHostMallocDefault);
     if (e != hipSuccess) return hip_fail(err, e, "frame arena stream");

@@ -81,6 +81,7 @@ struct FrameArena {
         big_rec, big_start, vcol;
     Arena a{};
     uint64_t gen = 0;          // bumped whenever a buffer moves: captured graphs are stale
+    bool lean = false;         // counted in an HBM budget: smaller where that only costs time (arena_ensure)
     bool dirty = true;         // bin counts / counters need a k_prep before the next frame
     uint32_t* host_counters = nullptr;   // pinned, CNT_COUNT words (then host_err, on its own cache line)
     uint32_t* host_err = nullptr;        // pinned word the kernels set nonzero with any error bit
@@ -194,7 +195,7 @@ struct FrameSize {
 // High-water marks the kernels reported after an overflow.
 FrameSize frame_size(const KArgs& ka);
 
-int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa);
+int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa, bool lean = false);
 void arena_destroy(axr_ctx* ctx, FrameArena& fa);
 uint64_t arena_bytes(const FrameArena& fa);
 int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs, const ArenaNeeds& need = {});

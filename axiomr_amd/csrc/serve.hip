@@ -75,7 +75,7 @@ public:
     int init() {
         (void)hipSetDevice(ctx_->device);
         for (Lane& l : lanes_) {
-            int r = arena_create(ctx_, err_, l.fa);
+            int r = arena_create(ctx_, err_, l.fa, true);   // the budget counts the lanes' arenas
             if (r) return r;
             // sized for a full batch up front (max_batch_faces faces over
             // max_batch_pixels pixels) so that serving does not grow it; only
