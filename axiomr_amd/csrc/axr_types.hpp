@@ -245,6 +245,7 @@ struct KArgs {
     uint32_t nviews;
     uint32_t total_faces;
     uint32_t total_tiles;
+    uint32_t first_bin = 0;     // of a launch over part of the bins (launch_bins)
     int32_t tile_size;          // bin edge in pixels: 8, 16 or 32
     int32_t raster_threads;     // least workgroup size of k_raster: 64, 128 or 256
     int32_t small_footprint;    // visibility mode: a triangle whose rectangle has at

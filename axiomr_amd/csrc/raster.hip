@@ -1645,6 +1645,9 @@ static uint32_t bin_blocks(uint32_t n) {
     const uint32_t round = NUM_XCD * XCD_RUN;
     return (n + round - 1) / round * round;
 }
+// A launch holds fewer than 2^32 threads: more bins go in several.
+constexpr uint32_t LAUNCH_BINS = 1u << 23;
+static_assert(LAUNCH_BINS % (NUM_XCD * XCD_RUN) == 0, "whole rounds");
 
 // Register bounds per shader kind (waves per SIMD the registers allow; the
 // LDS of a 128-thread block at 32 px bins, 19.9 KB with the full walk
@@ -1674,7 +1677,7 @@ __global__ __launch_bounds__(NT, raster_min_waves(SK)) void k_raster(KArgs ka, A
     // does with the record in resolve_pixel, and the indices during the edge
     // setup).  512 flat faces at 256x256: 9.1 -> 8.4 us with the launch; twelve
     // PBR draws at 1241x719: 17.5 -> 16.8 each; 40 mixed views: 202 -> 193.
-    const uint32_t t = bin_of_block(blockIdx.x), error = ar.counters[CNT_ERROR];
+    const uint32_t t = ka.first_bin + bin_of_block(blockIdx.x), error = ar.counters[CNT_ERROR];
     uint32_t count = 0, ref = 0;
     if (t < ka.total_tiles) {
         count = ar.tile_count[count_word(t)];
@@ -1900,7 +1903,7 @@ __device__ __forceinline__ void resolve_vis_tile_kind(const ViewDesc& V, const A
 template <int T, bool BATCH, int SK, bool INSIDE = false>
 __global__ __launch_bounds__(256) void k_resolve(KArgs ka, Arena ar) {
     // the bin's flag leaves with the error word (as in k_raster)
-    const uint32_t t = bin_of_block(blockIdx.x), error = ar.counters[CNT_ERROR];
+    const uint32_t t = ka.first_bin + bin_of_block(blockIdx.x), error = ar.counters[CNT_ERROR];
     uint32_t flag = 0;
     if (T > 8 && t < ka.total_tiles) flag = ar.tile_count[t];
     const bool failed = error != 0u;
@@ -2264,6 +2267,18 @@ static void stage_launch1(void (*kern)(KA...), dim3 grid, dim3 block, hipStream_
     stage_launch(kern, grid, block, st, ev, stage, true, true, args...);
 }
 
+// A kernel with a workgroup of `threads` per bin, in bin_of_block's order.
+static void launch_bins(void (*kern)(KArgs, Arena), uint32_t threads, hipStream_t st, StageEvents* ev, int stage,
+                        const KArgs& args, const Arena& ar) {
+    KArgs ka = args;
+    const uint32_t n = ka.total_tiles;
+    do {
+        const uint32_t left = n - ka.first_bin, take = left < LAUNCH_BINS ? left : LAUNCH_BINS;
+        stage_launch(kern, dim3(bin_blocks(take ? take : 1u)), dim3(threads), st, ev, stage, ka.first_bin == 0u, take == left, ka, ar);
+        ka.first_bin += take;
+    } while (ka.first_bin < n);
+}
+
 static hipError_t fb_wait(hipStream_t st, const FbWait& w) {
     if (w.sig) return hipStreamWaitValue64(st, w.sig, w.value, hipStreamWaitValueGte);
     if (w.ev) return hipStreamWaitEvent(st, w.ev, 0);
@@ -2354,12 +2369,13 @@ static hipError_t launch_vis_t(const KArgs& ka, const Arena& ar, hipStream_t st,
     // the framebuffer pass waits for what other streams were asked to do first
     hipError_t e = fb_wait(st, wait);
     if (e != hipSuccess) return e;
-    // T = 8: four bins per workgroup; larger bins: one bin per workgroup
-    const uint32_t rb = T == 8 ? (uint32_t)imax(1, imin((int)((ka.total_tiles + 3) / 4), RESOLVE_MAX_BLOCKS))
-                               : bin_blocks((uint32_t)imax(1, (int)ka.total_tiles));
     const auto resolve = (!BATCH && ka.skip_clip) ? by_shader<ResolveK<T, false, true>::template K>(ka.shader)
                                                   : by_shader<ResolveK<T, BATCH, false>::template K>(ka.shader);
-    stage_launch1(resolve, dim3(rb), dim3(256), st, ev, 4, ka, ar);
+    // T = 8: four bins per workgroup; larger bins: one bin per workgroup
+    if constexpr (T == 8)
+        stage_launch1(resolve, dim3(imax(1, imin((int)((ka.total_tiles + 3) / 4), RESOLVE_MAX_BLOCKS))), dim3(256), st, ev, 4, ka, ar);
+    else
+        launch_bins(resolve, 256, st, ev, 4, ka, ar);
     return hipGetLastError();
 }
 
@@ -2369,17 +2385,15 @@ static hipError_t launch_frame_t(const KArgs& ka, const Arena& ar, hipStream_t s
                                  const FbWait& wait) {
     if (ka.mode == RASTER_VISIBILITY) return launch_vis_t<T, BATCH>(ka, ar, st, ev, wait);
     t_phases = kBinnedPhases;
-    const uint32_t ntiles = ka.total_tiles;
     const uint32_t setup_blocks = face_blocks(ka);
     if (setup_blocks) {
         if (ka.skip_clip) stage_launch1(k_setup<T, BATCH, true>, dim3(setup_blocks), dim3(256), st, ev, 0, ka, ar);
         else stage_launch1(k_setup<T, BATCH>, dim3(setup_blocks), dim3(256), st, ev, 0, ka, ar);
     }
     if (!ka.skip_clip) stage_launch1(k_clip<T, BATCH, false>, dim3(CLIP_BLOCKS), dim3(64 * CLIP_WAVES), st, ev, 1, ka, ar);
-    const uint32_t rblocks = bin_blocks((uint32_t)imax(1, (int)ntiles));
     hipError_t e = fb_wait(st, wait);
     if (e != hipSuccess) return e;
-    stage_launch1(by_shader<RasterK<T, NT, BATCH>::template K>(ka.shader), dim3(rblocks), dim3(NT), st, ev, 4, ka, ar);
+    launch_bins(by_shader<RasterK<T, NT, BATCH>::template K>(ka.shader), NT, st, ev, 4, ka, ar);
     return hipGetLastError();
 }
 
