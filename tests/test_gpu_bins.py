@@ -1,7 +1,7 @@
 """Binned mode's bins: entries written straight into a bin's first level and,
 past it, into levels from the pools (raster.hip bin_put / bin_get), by the
 wave's rounds (grouped or lane by lane) and by its flattened pairs; and the
-wave-per-face clipper that feeds them.  Every frame equals the checker's,
+wave-per-face clipper that feeds them.  Every frame equals the oracle's,
 bit for bit in coverage, depth and winner."""
 import numpy as np
 import pytest
@@ -29,7 +29,7 @@ def _scene(kind):
 @pytest.mark.gpu
 @pytest.mark.parametrize("tile", [8, 16, 32])
 @pytest.mark.parametrize("kind", ["clustered", "one_bin", "large", "inside", "clipped", "soup"])
-def test_bins_equal_checker(kind, tile):
+def test_bins_equal_oracle(kind, tile):
     sc = _scene(kind)
     ref = H.render_oracle(sc)
     ctx = R.Context(0)

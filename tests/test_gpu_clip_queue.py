@@ -1,6 +1,6 @@
 """The clipper's queue: faces within the sub-queues, past them into the shared
 queue, and past that (the arena grows and the frame is drawn again), one to
-several pieces a face; every frame equals the checker's."""
+several pieces a face; every frame equals the oracle's."""
 import numpy as np
 import pytest
 
@@ -37,7 +37,7 @@ def edge_scene(n, corner, seed=8, width=403, height=301):
 
 @pytest.mark.parametrize("mode", [N.RASTER_BINNED, N.RASTER_VISIBILITY])
 @pytest.mark.parametrize("n,corner", [(65, False), (3000, False), (3000, True), (7000, False), (20_000, True)])
-def test_clip_queue_equals_checker(mode, n, corner):
+def test_clip_queue_equals_oracle(mode, n, corner):
     sc = edge_scene(n, corner)
     ref = H.render_oracle(sc)
     ctx = R.Context(0)

@@ -1,7 +1,7 @@
 """Passes over faces by their launch rules: 16 or 64 faces per wave, walks of
 larger rectangles shared by the wave or not (k_vis), bin entries laid end to
 end, workgroup sizes of the binned raster, and clears absorbed by it.  Every
-frame equals the checker's; batched views whose faces share a wave equal
+frame equals the oracle's; batched views whose faces share a wave equal
 their solo draws."""
 import numpy as np
 import pytest
@@ -24,7 +24,7 @@ MODES = {"binned": N.RASTER_BINNED, "visibility": N.RASTER_VISIBILITY}
     (41, 1280, 720, 12),        # 33,620: 64 per wave, shared
     (41, 640, 480, 128),        # 9 pixels per face: not shared
 ])
-def test_face_waves_equal_checker(mode, n, width, height, footprint):
+def test_face_waves_equal_oracle(mode, n, width, height, footprint):
     sc = S.icosphere_scene(n=n, width=width, height=height, tex=64, radius=2.3)
     ref = H.render_oracle(sc)
     ctx = R.Context(0)
