@@ -4,6 +4,7 @@
 #pragma once
 #include <cstdint>
 #include "axr_math.hpp"
+#include "bins.hpp"
 
 namespace axr {
 
@@ -152,12 +153,7 @@ constexpr uint32_t ERR_PAIRS = 4u;
 constexpr uint32_t ERR_BIG = 8u;
 constexpr uint32_t ERR_SKIPPED = 16u;   // a pass the host skipped had work: the frame is redrawn with it
 
-// Bins of binned mode: level k of a bin holds 2^(bin0_shift + k) entries, so
-// BIN_LEVELS levels reach 2^31 entries for the smallest first level.
-constexpr uint32_t BIN0_LEAN_SHIFT = 4, BIN0_MIN_SHIFT = 5, BIN0_MAX_SHIFT = 12;
-constexpr uint32_t COUNT_BLOCK = 8192;         // words of tile_count that bins are spread over
-constexpr uint32_t BIN_LEVELS = 27;
-constexpr uint32_t CHUNK_NONE = 0xFFFFFFFFu;   // a level the pools had no room for
+// Binned mode's pools and sub-queues (its bins: bins.hpp).
 constexpr uint32_t POOL_SUBS = 64;
 constexpr uint32_t CLIP_SUBS = 64;             // one per lane of a wave
 constexpr uint32_t POOL_STRIDE = 32;           // words between the pools' and sub-queues' counters
@@ -186,7 +182,7 @@ struct Arena {
     Vertex56* clip_verts;      // 3 per clip record
     uint32_t* tile_count;      // per bin: its entries (binned mode, at count_word), whether
                                // it holds keys (visibility mode)
-    // binned mode: record refs by bin (see bin_put in raster.hip)
+    // binned mode: record refs by bin (see BinStore in raster.hip)
     uint32_t* bins;            // 2^bin0_shift first entries of every bin
     uint32_t* bin_chunks;      // BIN_LEVELS words per bin: where its further entries
                                // are (first entry in bin_pool + 1); 0: not allocated

@@ -460,27 +460,6 @@ __device__ __forceinline__ uint32_t bin_of(uint32_t first, uint32_t pitch, uint3
 // 4M-triangle soup's 730).  The host sizes the first level for four times the
 // mean of faces per bin, so most bins of most frames never leave it.
 
-// The word of tile_count that counts bin t's entries.  Atomics on one cache
-// line wait for each other (~9 ns each, whatever word they name: 7M spread
-// over 3,600 neighbouring words take 530 us, over twice the lines 290), and a
-// mesh fills neighbouring bins at the same time, so a block of 8,192 words
-// holds its bins in runs of four, each run in another of its 256 lines.  The
-// runs are there for triangles over two or three bins, whose atomics on one
-// line travel together (the 4M-triangle soup's k_setup 255 us, 279 with every
-// bin in another line).  k_setup of 40 mixed views 88 -> 65 us, of a 150k soup
-// 25 -> 20, of the 1M-triangle frame 20.7 -> 17.5.
-__device__ __forceinline__ uint32_t count_word(uint32_t t) {
-    return (t & ~(COUNT_BLOCK - 1u)) | ((t & 0x3FCu) << 3) | (t & 3u) | ((t >> 8) & 28u);
-}
-
-struct BinSlot {
-    uint32_t level, offset;   // entry `offset` of level `level`
-};
-__device__ __forceinline__ BinSlot bin_slot(const Arena& ar, uint32_t slot) {
-    const uint32_t level = 31u - (uint32_t)__clz((int)((slot >> ar.bin0_shift) + 1u));
-    return BinSlot{level, slot - (((1u << level) - 1u) << ar.bin0_shift)};
-}
-
 // Room for one chunk of n entries: from the sub-pool that the bin's number
 // picks (one counter for all bins would serialize the allocations, ~11 ns
 // each) or, when that is full or the chunk a large part of it, the shared
@@ -499,38 +478,47 @@ __device__ __forceinline__ uint32_t pool_take(const Arena& ar, uint32_t bin, uin
     return 0u;
 }
 
-// Store entry `slot` of `bin` (act: this lane has one; all 64 lanes call
-// it).  The lane that took a level's first slot allocates the level and
-// publishes it in the chunk table; the others wait for that word.  The wait
-// ends: a level's first slot was taken before any later one of it, and
-// between taking it and publishing that lane waits for nothing (the loop
-// below comes after the publishing in every lane of the wave; the ballots
-// keep the wave together).
+// Store this lane's Q entries (act: it has one), whose slots the wave has
+// taken; all 64 lanes call it.  The lane that took a level's first slot
+// allocates the level and publishes it in the chunk table; the others wait for
+// that word.  The wait ends: a level's first slot was taken before any later
+// one of it, and the wave that took it publishes all the levels it opened
+// before it waits for any other wave's (place_entries).
 constexpr uint32_t BIN_WAIT_TRIES = 1u << 20;   // about a second
-__device__ __forceinline__ void bin_put(const Arena& ar, bool act, uint32_t bin, uint32_t slot, uint32_t ref) {
-    const BinSlot b = bin_slot(ar, slot);
-    const bool spill = act && b.level != 0u;
-    if (act && !spill) ar.bins[((size_t)bin << ar.bin0_shift) + slot] = ref;
-    if (__ballot(spill) == 0ull) return;
-    uint32_t* cell = ar.bin_chunks + (size_t)bin * BIN_LEVELS + b.level;
-    if (spill && b.offset == 0u) {
-        const uint32_t at = pool_take(ar, bin, 1u << (ar.bin0_shift + b.level));
-        __hip_atomic_store(cell, at ? at : CHUNK_NONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+template <uint32_t Q>
+struct BinStore {
+    const Arena& ar;
+    const bool (&act)[Q];
+    const uint32_t (&bin)[Q], (&slot)[Q], (&ref)[Q];
+    __device__ __forceinline__ uint32_t* cell(uint32_t q, const BinSlot& b) const {
+        return ar.bin_chunks + (size_t)bin[q] * BIN_LEVELS + b.level;
     }
-    uint32_t at = 0u;
-    for (uint32_t tries = 0; __ballot(spill && at == 0u) != 0ull; ++tries) {
-        if (spill && at == 0u) at = __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (tries == BIN_WAIT_TRIES && spill && at == 0u) {   // never seen; a frame that is redrawn, not a hang
-            raise_error(ar, ERR_PAIRS);
-            at = CHUNK_NONE;
+    __device__ __forceinline__ void open(uint32_t q) {
+        const BinSlot b = bin_slot(ar.bin0_shift, slot[q]);
+        if (act[q] && b.level == 0u) ar.bins[((size_t)bin[q] << ar.bin0_shift) + slot[q]] = ref[q];
+        if (act[q] && b.level != 0u && b.offset == 0u) {
+            const uint32_t at = pool_take(ar, bin[q], 1u << (ar.bin0_shift + b.level));
+            __hip_atomic_store(cell(q, b), at ? at : CHUNK_NONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    if (spill && at != CHUNK_NONE) ar.bin_pool[(size_t)(at - 1u) + b.offset] = ref;
-}
+    __device__ __forceinline__ void fill(uint32_t q) {
+        const BinSlot b = bin_slot(ar.bin0_shift, slot[q]);
+        const bool spill = act[q] && b.level != 0u;
+        uint32_t at = 0u;
+        for (uint32_t tries = 0; __ballot(spill && at == 0u) != 0ull; ++tries) {
+            if (spill && at == 0u) at = __hip_atomic_load(cell(q, b), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (tries == BIN_WAIT_TRIES && spill && at == 0u) {   // never seen; a frame that is redrawn, not a hang
+                raise_error(ar, ERR_PAIRS);
+                at = CHUNK_NONE;
+            }
+        }
+        if (spill && at != CHUNK_NONE) ar.bin_pool[(size_t)(at - 1u) + b.offset] = ref[q];
+    }
+};
 
 // Entry i of bin t.
 __device__ __forceinline__ uint32_t bin_get(const Arena& ar, uint32_t t, uint32_t i) {
-    const BinSlot b = bin_slot(ar, i);
+    const BinSlot b = bin_slot(ar.bin0_shift, i);
     if (b.level == 0u) return ar.bins[((size_t)t << ar.bin0_shift) + i];
     return ar.bin_pool[(size_t)(ar.bin_chunks[(size_t)t * BIN_LEVELS + b.level] - 1u) + b.offset];
 }
@@ -578,11 +566,15 @@ __device__ __forceinline__ void emit_bins_wave(const Arena& ar, const ViewDesc& 
             }
             if (act && leader_of_mine == (int)lane) slot = atomicAdd(&ar.tile_count[count_word(bin)], (uint32_t)__popcll(mine));
             slot = __shfl(slot, leader_of_mine) + (uint32_t)__popcll(mine & __lanemask_lt());
-            bin_put(ar, act, bin, slot, ref);
+            const bool acts[1] = {act};
+            const uint32_t bins[1] = {bin}, slots[1] = {slot}, refs[1] = {ref};
+            BinStore<1> store{ar, acts, bins, slots, refs};
+            place_entries<1>(store);
         }
     }
     const uint32_t incl = wave_incl_scan(n), start = incl - n, total = __shfl(incl, 63);
     for (uint32_t j0 = 0; j0 < total; j0 += 64u * EMIT_AHEAD) {
+        bool act[EMIT_AHEAD];
         uint32_t bin[EMIT_AHEAD], slot[EMIT_AHEAD], r[EMIT_AHEAD];
 #pragma unroll
         for (uint32_t q = 0; q < EMIT_AHEAD; ++q) {
@@ -597,13 +589,14 @@ __device__ __forceinline__ void emit_bins_wave(const Arena& ar, const ViewDesc& 
             const uint32_t k = j - __shfl(start, o);
             r[q] = __shfl(ref, o);
             slot[q] = bin[q] = 0u;
-            if (j < total) {
+            act[q] = j < total;
+            if (act[q]) {
                 bin[q] = bin_of(first, pitch, nx, k);
                 slot[q] = atomicAdd(&ar.tile_count[count_word(bin[q])], 1u);
             }
         }
-#pragma unroll
-        for (uint32_t q = 0; q < EMIT_AHEAD; ++q) bin_put(ar, j0 + 64u * q + lane < total, bin[q], slot[q], r[q]);
+        BinStore<EMIT_AHEAD> store{ar, act, bin, slot, r};
+        place_entries<EMIT_AHEAD>(store);
     }
 }
 
@@ -1616,7 +1609,7 @@ __device__ __forceinline__ void raster_bin(const KArgs& ka, const Arena& ar, uin
     __syncthreads();
 
     // every entry has been read: leave the chunk table empty as well
-    if (threadIdx.x > 0 && threadIdx.x <= bin_slot(ar, n - 1).level) ar.bin_chunks[(size_t)t * BIN_LEVELS + threadIdx.x] = 0;
+    if (threadIdx.x > 0 && threadIdx.x <= bin_slot(ar.bin0_shift, n - 1).level) ar.bin_chunks[(size_t)t * BIN_LEVELS + threadIdx.x] = 0;
 
     // a batch's clear is a pass of its own before the frame (k_clear_views)
     const ClearSpec cs{!BATCH && ka.clear != 0, ka.clear_bgra, ka.clear_depth};
