@@ -136,7 +136,7 @@ FrameSize frame_size(const KArgs& ka) {
     return fs;
 }
 
-int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs, const ArenaNeeds& need) {
+static int arena_grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs, const ArenaNeeds& need) {
     const uint64_t faces = fs.faces, tiles = fs.tiles;
     if (faces > 0x7FFFFFFFull || tiles > 0x7FFFFFFFull || fs.pixels > 0xFFFFFFFFull)
         return fail(err, AXR_ERR_INVALID, "draw too large (%llu faces, %llu bins, %llu pixels)",
@@ -176,7 +176,6 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
         big_recs = std::max<uint64_t>({4096, faces / 8, need.big_recs, a.cap_big_recs});
         big_items = std::max<uint64_t>({16384, faces / 4 + fs.pixels / 32, need.big_items, a.cap_big_items});
     }
-    const uint64_t gen_start = fa.gen;
     int r;
     if ((r = grow(ctx, err, fa, fa.counters, CNT_COUNT * 4)) ||
         (r = grow(ctx, err, fa, fa.rec, std::max<uint64_t>(faces, 1) * (vis ? 4 : sizeof(TriRec)))) ||
@@ -216,21 +215,33 @@ int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs
     a.cap_clip_faces = (uint32_t)std::min<uint64_t>(fa.clip_faces.bytes / 4 - CLIP_SUBS * clip_sub, 0x1FFFFFFFull);
     a.cap_clip_recs = (uint32_t)std::min<uint64_t>(
         {fa.clip_rec.bytes / sizeof(TriRec), fa.clip_verts.bytes / (3 * sizeof(Vertex56)), 0x7FFFFFFFull});
+    // whatever the mode: k_prep empties the chunk table that is there (none
+    // after a growth that failed, until a binned draw asks for it again)
+    a.cap_chunks = (uint32_t)std::min<uint64_t>(fa.bin_chunks.bytes / 4, 0xFFFFFFFFull);
     if (!vis) {
         // sub-pool sizes keep their place between draws; a captured graph
         // holds its own copy of these, and its buffers' moves change gen
         a.bin0_shift = bin0_shift;
         a.sub_cap = (uint32_t)std::min<uint64_t>(sub, 0x7FFFFFFFull / POOL_SUBS / 2);
         a.pool_cap = (uint32_t)std::min<uint64_t>(fa.bin_pool.bytes / 4 - (uint64_t)POOL_SUBS * a.sub_cap, 0x7FFFFFFFull);
-        a.cap_chunks = (uint32_t)std::min<uint64_t>(fa.bin_chunks.bytes / 4, 0xFFFFFFFFull);
     }
     a.cap_vkeys = (uint32_t)std::min<uint64_t>(fa.vkeys.bytes / 8, 0xFFFFFFFFull);
     a.cap_big_recs = (uint32_t)std::min<uint64_t>(
         {fa.big_rec.bytes / sizeof(TriRec), fa.big_start.bytes / 4, 0x7FFFFFFFull});
     // items are only counted (no storage): the cap bounds the work of k_big
     a.cap_big_items = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(big_items, a.cap_big_items), 0x7FFFFFFFull);
-    if (fa.gen != gen_start) fa.dirty = true;
     return AXR_OK;
+}
+
+// A growth that fails has freed the buffer it could not replace and may have
+// replaced others, whose new memory is not cleared: either way the next frame
+// starts with a k_prep, and captured graphs are stale.
+int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs, const ArenaNeeds& need) {
+    const uint64_t gen_start = fa.gen;
+    const int r = arena_grow(ctx, err, fa, fs, need);
+    if (r) ++fa.gen;
+    if (fa.gen != gen_start) fa.dirty = true;
+    return r;
 }
 
 // Zero the whole counter block (including the sticky error and the

@@ -412,7 +412,7 @@ __global__ void k_prep(Arena ar, uint32_t ntiles) {
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = tid; i < ntiles; i += stride) ar.tile_count[i] = 0;
     for (uint32_t i = tid; i < ar.cap_chunks; i += stride) ar.bin_chunks[i] = 0;
-    if (ar.cap_chunks)
+    if (ar.pool_next)
         for (uint32_t i = tid; i < (POOL_SUBS + 1) * POOL_STRIDE; i += stride) ar.pool_next[i] = 0;
     if (ar.clip_next)
         for (uint32_t i = tid; i < CLIP_SUBS * POOL_STRIDE; i += stride) ar.clip_next[i] = 0;
