@@ -146,6 +146,8 @@ static int arena_grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSiz
     // slot (only the first clip record of a clipped face, 4 bytes) and no
     // bin pairs; binned mode keeps a 48-byte record per face slot
     const bool vis = fs.pixels != 0;
+    // no frame (a frame has a bin): what overflowing frames of either mode reported
+    const bool needs_only = tiles == 0;
     const uint64_t want_clip = std::max<uint64_t>({4096, faces / 16, need.clip_faces});
     const uint64_t clip_faces = std::max<uint64_t>(want_clip, a.cap_clip_faces);
     // the sub-queues beside the shared queue of clip_faces entries, and their
@@ -172,9 +174,12 @@ static int arena_grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSiz
         std::max<uint64_t>((fa.lean ? 2 * faces : 2 * faces + 16 * tiles + 4096) / POOL_SUBS, a.sub_cap);
     // visibility mode: large triangles and their 256-pixel work items
     uint64_t big_recs = 0, big_items = 0;
-    if (fs.pixels) {
+    if (vis) {
         big_recs = std::max<uint64_t>({4096, faces / 8, need.big_recs, a.cap_big_recs});
         big_items = std::max<uint64_t>({16384, faces / 4 + fs.pixels / 32, need.big_items, a.cap_big_items});
+    } else if (needs_only) {
+        big_recs = need.big_recs;
+        big_items = need.big_items;
     }
     int r;
     if ((r = grow(ctx, err, fa, fa.counters, CNT_COUNT * 4)) ||
@@ -221,7 +226,7 @@ static int arena_grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSiz
     if (!vis) {
         // sub-pool sizes keep their place between draws; a captured graph
         // holds its own copy of these, and its buffers' moves change gen
-        a.bin0_shift = bin0_shift;
+        if (!needs_only) a.bin0_shift = bin0_shift;
         a.sub_cap = (uint32_t)std::min<uint64_t>(sub, 0x7FFFFFFFull / POOL_SUBS / 2);
         a.pool_cap = (uint32_t)std::min<uint64_t>(fa.bin_pool.bytes / 4 - (uint64_t)POOL_SUBS * a.sub_cap, 0x7FFFFFFFull);
     }
@@ -808,14 +813,11 @@ int axr_ctx_memory(const axr_ctx* ctx, uint64_t* in_use, uint64_t* arena) {
 
 // After a host wait and arena_counters_after_wait: an arena whose frames
 // overflowed is grown to what the kernels reported (the current capacity is
-// the floor) and reset.
+// the floor) and reset.  Which of the frames since the last wait that was, of
+// which size and mode, is not known here: the arena grows by the needs alone
+// (a frame's own sizes are met when it is drawn again).
 static int arena_settle_overflow(axr_ctx* ctx, FrameArena& fa) {
-    if (!fa.host_counters[CNT_ERROR]) return AXR_OK;
-    FrameSize fs;
-    fs.faces = fa.rec.bytes / sizeof(TriRec);
-    fs.tiles = fa.tile_count.bytes / 4 - 1;
-    fs.pixels = fa.vkeys.bytes / 8;
-    return arena_check_overflow(ctx, ctx->err, fa, fs);
+    return arena_check_overflow(ctx, ctx->err, fa, FrameSize{});
 }
 
 int axr_sync(axr_ctx* ctx) {

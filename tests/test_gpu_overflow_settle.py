@@ -1,0 +1,107 @@
+"""Frames that overflow their arena and are waited for with axr_sync: one
+report, an arena grown to what the frames reported and no further, and the
+same frames drawn again in full, whatever the arena drew before."""
+import numpy as np
+import pytest
+
+import axiomr_amd as axr
+import harness as H
+from axiomr_amd import _native as N
+from axiomr_amd import render as R
+from axiomr_amd import scenes as S
+
+pytestmark = pytest.mark.gpu
+
+TILE = 8
+
+
+def layered_scene(n, width, height, seed=3):
+    """n triangles one behind the other in random order, each inside the
+    frustum with a pixel rectangle that touches every bin."""
+    rng = np.random.default_rng(seed)
+    z = rng.permutation(np.linspace(1.0, 2.0, n))
+    t = 0.995 * np.tan(np.radians(30.0)) * z
+    v = np.zeros((n, 3, 14), np.float32)
+    for k, (sx, sy) in enumerate(((-1, -1), (1, -1), (-1, 1))):
+        v[:, k, 0] = sx * t * width / height
+        v[:, k, 1] = sy * t
+        v[:, k, 2] = -z
+    v[:, :, 5:8] = (0.0, 0.0, 1.0)
+    colors = rng.integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32)
+    return S.SceneData(name=f"layers_{n}", vertices=v.reshape(-1, 14), faces=np.arange(3 * n, dtype=np.uint32).reshape(n, 3),
+                       width=width, height=height, camera_pos=(0.0, 0.0, 0.0), camera_target=(0.0, 0.0, -1.0), fov=60.0,
+                       shader={"kind": 5}, groups=[(0, 0, n)], materials=[S.MaterialData()], face_colors=colors)
+
+
+def overflow_code(ctx):
+    with pytest.raises(axr.AxrError) as e:
+        ctx.sync()
+    return e.value.code
+
+
+@pytest.mark.parametrize("visibility_first", [False, True])
+def test_batch_after_an_overflow(visibility_first):
+    """A binned batch whose entries do not fit the shared pool, in a context
+    that has drawn in visibility mode or has not."""
+    scenes = [layered_scene(300, 256, 256, seed) for seed in (3, 4)]
+    refs = [H.render_oracle(sc) for sc in scenes]
+    ctx = R.Context(0)
+    gs, fbs, batch = [], [], None
+    try:
+        gs = [H.GpuScene(ctx, sc) for sc in scenes]
+        fbs = [R.Framebuffer(ctx, sc.width, sc.height, with_ids=True) for sc in scenes]
+        ps = [H.params_of(sc) for sc in scenes]
+        if visibility_first:
+            ctx.set_config(raster_mode=N.RASTER_VISIBILITY)
+            ctx.check(ctx._lib.axr_draw(ctx.handle, fbs[0].handle, gs[0].mesh.handle, R.C.byref(ps[0])))
+        ctx.set_config(raster_mode=N.RASTER_BINNED, tile_size=TILE)
+        batch = R.Batch(ctx, fbs, [g.mesh for g in gs], ps)
+        batch.set_clear(H.BLACK)
+        batch.launch()
+        assert overflow_code(ctx) == N.AXR_ERR_OVERFLOW
+        for again in range(3):
+            batch.launch()
+            ctx.sync()
+            for fb, ref in zip(fbs, refs):
+                H.assert_parity(H.compare(fb.read(), ref), f"launch {again}")
+    finally:
+        for x in [batch] * (batch is not None) + fbs + gs:
+            x.close()
+        ctx.close()
+
+
+def test_growth_by_the_reported_needs():
+    """A queued frame over 64 bins that overflows in a context whose budget
+    holds what the frame needs and little more."""
+    n, bins = 3000, 64
+    sc = layered_scene(n, 64, 64)
+    # levels of 32, 64, ... entries hold a bin's 3,000 in 32 (2^7 - 1) of them,
+    # the first level's in its own place; a quarter is added to the need
+    bound = 4 * bins * (32 * 127 - 32) * 5 // 4
+    ref = H.render_oracle(sc)
+
+    def run(budget):
+        ctx = R.Context(0, budget)
+        gs = fb = None
+        try:
+            ctx.set_config(raster_mode=N.RASTER_BINNED, tile_size=TILE)
+            gs, fb = H.GpuScene(ctx, sc), R.Framebuffer(ctx, sc.width, sc.height, with_ids=True)
+            p = H.params_of(sc, flags=N.AXR_DRAW_ASYNC)
+            for attempt in range(3):
+                fb.clear(H.BLACK)
+                ctx.check(ctx._lib.axr_draw(ctx.handle, fb.handle, gs.mesh.handle, R.C.byref(p)))
+                if attempt:
+                    ctx.sync()
+                    H.assert_parity(H.compare(fb.read(), ref), f"frame {attempt}")
+                else:
+                    before = ctx.memory()      # with the frame's own sizes, which the draw asked for
+                    assert overflow_code(ctx) == N.AXR_ERR_OVERFLOW
+                    assert 0 < ctx.memory()[1] - before[1] <= bound
+            return sum(before)
+        finally:
+            for x in (fb, gs):
+                if x is not None:
+                    x.close()
+            ctx.close()
+
+    run(run(8 << 30) + bound)
