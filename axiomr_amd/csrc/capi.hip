@@ -233,8 +233,11 @@ static int arena_grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSiz
     a.cap_vkeys = (uint32_t)std::min<uint64_t>(fa.vkeys.bytes / 8, 0xFFFFFFFFull);
     a.cap_big_recs = (uint32_t)std::min<uint64_t>(
         {fa.big_rec.bytes / sizeof(TriRec), fa.big_start.bytes / 4, 0x7FFFFFFFull});
-    // items are only counted (no storage): the cap bounds the work of k_big
-    a.cap_big_items = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(big_items, a.cap_big_items), 0x7FFFFFFFull);
+    // items are only counted (no storage): the cap bounds the work of k_big.
+    // A captured graph holds the cap it was captured with.
+    const uint32_t items = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(big_items, a.cap_big_items), 0x7FFFFFFFull);
+    if (items != a.cap_big_items) ++fa.gen;
+    a.cap_big_items = items;
     return AXR_OK;
 }
 

@@ -39,10 +39,11 @@ def overflow_code(ctx):
     return e.value.code
 
 
-@pytest.mark.parametrize("visibility_first", [False, True])
-def test_batch_after_an_overflow(visibility_first):
+@pytest.mark.parametrize("mode,visibility_first", [(N.RASTER_BINNED, False), (N.RASTER_BINNED, True), (N.RASTER_VISIBILITY, False)])
+def test_batch_after_an_overflow(mode, visibility_first):
     """A binned batch whose entries do not fit the shared pool, in a context
-    that has drawn in visibility mode or has not."""
+    that has drawn in visibility mode or has not; a visibility batch of few
+    large triangles with more work items than the arena counts on."""
     scenes = [layered_scene(300, 256, 256, seed) for seed in (3, 4)]
     refs = [H.render_oracle(sc) for sc in scenes]
     ctx = R.Context(0)
@@ -54,7 +55,7 @@ def test_batch_after_an_overflow(visibility_first):
         if visibility_first:
             ctx.set_config(raster_mode=N.RASTER_VISIBILITY)
             ctx.check(ctx._lib.axr_draw(ctx.handle, fbs[0].handle, gs[0].mesh.handle, R.C.byref(ps[0])))
-        ctx.set_config(raster_mode=N.RASTER_BINNED, tile_size=TILE)
+        ctx.set_config(raster_mode=mode, tile_size=TILE)
         batch = R.Batch(ctx, fbs, [g.mesh for g in gs], ps)
         batch.set_clear(H.BLACK)
         batch.launch()
