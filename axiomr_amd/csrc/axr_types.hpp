@@ -155,6 +155,8 @@ constexpr uint32_t ERR_SKIPPED = 16u;   // a pass the host skipped had work: the
 
 // Binned mode's pools and sub-queues (its bins: bins.hpp).
 constexpr uint32_t POOL_SUBS = 64;
+constexpr uint64_t POOL_SUB_MAX = 1u << 24;    // entries of one sub-pool at most
+constexpr uint64_t POOL_ENTRIES = CHUNK_NONE - 1ull;   // of all pools: a chunk's first entry + 1 is below CHUNK_NONE
 constexpr uint32_t CLIP_SUBS = 64;             // one per lane of a wave
 constexpr uint32_t POOL_STRIDE = 32;           // words between the pools' and sub-queues' counters
 

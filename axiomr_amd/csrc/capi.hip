@@ -169,9 +169,12 @@ static int arena_grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSiz
     while (bin0_shift < BIN0_MAX_SHIFT &&
            (fa.lean ? (tiles << (bin0_shift + 1)) <= (tiles << BIN0_LEAN_SHIFT) + faces : (tiles << bin0_shift) < 4 * faces))
         ++bin0_shift;
-    const uint64_t pool = std::max<uint64_t>({2 * (2 * faces + 16 * tiles + 4096), need.pairs, a.pool_cap});
-    const uint64_t sub =
-        std::max<uint64_t>((fa.lean ? 2 * faces : 2 * faces + 16 * tiles + 4096) / POOL_SUBS, a.sub_cap);
+    const uint64_t sub = std::min<uint64_t>(
+        std::max<uint64_t>((fa.lean ? 2 * faces : 2 * faces + 16 * tiles + 4096) / POOL_SUBS, a.sub_cap), POOL_SUB_MAX);
+    // the pools' entries together are numbered in 32 bits: a frame of nearly
+    // 2^31 entries may take twice as many, in levels that are half empty
+    const uint64_t pool = std::min<uint64_t>(
+        std::max<uint64_t>({2 * (2 * faces + 16 * tiles + 4096), need.pairs, a.pool_cap}), POOL_ENTRIES - POOL_SUBS * sub);
     // visibility mode: large triangles and their 256-pixel work items
     uint64_t big_recs = 0, big_items = 0;
     if (vis) {
@@ -227,8 +230,8 @@ static int arena_grow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSiz
         // sub-pool sizes keep their place between draws; a captured graph
         // holds its own copy of these, and its buffers' moves change gen
         if (!needs_only) a.bin0_shift = bin0_shift;
-        a.sub_cap = (uint32_t)std::min<uint64_t>(sub, 0x7FFFFFFFull / POOL_SUBS / 2);
-        a.pool_cap = (uint32_t)std::min<uint64_t>(fa.bin_pool.bytes / 4 - (uint64_t)POOL_SUBS * a.sub_cap, 0x7FFFFFFFull);
+        a.sub_cap = (uint32_t)sub;
+        a.pool_cap = (uint32_t)(std::min<uint64_t>(fa.bin_pool.bytes / 4, POOL_ENTRIES) - POOL_SUBS * sub);
     }
     a.cap_vkeys = (uint32_t)std::min<uint64_t>(fa.vkeys.bytes / 8, 0xFFFFFFFFull);
     a.cap_big_recs = (uint32_t)std::min<uint64_t>(

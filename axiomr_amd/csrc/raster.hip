@@ -474,7 +474,7 @@ __device__ __forceinline__ uint32_t pool_take(const Arena& ar, uint32_t bin, uin
     }
     const uint32_t o = atomicAdd(ar.pool_next + POOL_SUBS * POOL_STRIDE, n);
     if ((unsigned long long)o + n <= ar.pool_cap) return POOL_SUBS * ar.sub_cap + o + 1u;
-    set_error(ar, ERR_PAIRS, CNT_NEED_PAIRS, o + n);
+    set_error(ar, ERR_PAIRS, CNT_NEED_PAIRS, o + n < o ? ~0u : o + n);
     return 0u;
 }
 

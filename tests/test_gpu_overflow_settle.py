@@ -106,3 +106,29 @@ def test_growth_by_the_reported_needs():
             ctx.close()
 
     run(run(8 << 30) + bound)
+
+
+def test_frame_of_a_thousand_million_entries():
+    """8,200 triangles over 140,000 bins: 1.15e9 entries, whose levels (the last
+    of a bin has room for 8,192 and holds 40) number more than 2^31."""
+    sc = layered_scene(8200, 2800, 3200)
+    ctx = R.Context(0)
+    gs = fb = None
+    try:
+        gs, fb = H.GpuScene(ctx, sc), R.Framebuffer(ctx, sc.width, sc.height, with_ids=True)
+        p = H.params_of(sc)
+        got = {}
+        for mode in (N.RASTER_VISIBILITY, N.RASTER_BINNED):
+            ctx.set_config(raster_mode=mode, tile_size=TILE)
+            fb.clear(H.BLACK)
+            print(f"mode {mode}", flush=True)
+            ctx.check(ctx._lib.axr_draw(ctx.handle, fb.handle, gs.mesh.handle, R.C.byref(p)))
+            got[mode] = fb.read()
+        for a, b in zip(got[N.RASTER_BINNED], got[N.RASTER_VISIBILITY]):
+            assert (a.view(np.uint8) == b.view(np.uint8)).all()
+        assert (got[N.RASTER_BINNED][2] != H.EMPTY_ID).sum() > 2800 * 3200 * 0.48
+    finally:
+        for x in (fb, gs):
+            if x is not None:
+                x.close()
+        ctx.close()
