@@ -37,15 +37,20 @@ AXR_HD BinSlot bin_slot(uint32_t bin0_shift, uint32_t slot) {
 }
 
 // Stores the Q entries per lane whose slots a wave has taken, waves against
-// waves: s.open(q) publishes the level that entry q opens, if it does, and
-// waits for nothing; s.fill(q) stores entry q, after waiting for its level if
-// another lane opens that.  Every open comes before every fill: a wave that
-// waited with a level of its own unpublished could wait for a wave that waits
-// for that level (the slots are taken by atomics on different words, in
-// flight together, so either wave may be the first on one word and the second
-// on the other).
+// waves: s.near(q) stores entry q if it lies in its bin's first level, else
+// returns true; where the wave has such entries (s.any), s.open(q) publishes
+// the level that entry q opens, if it does, and waits for nothing, and
+// s.fill(q) stores entry q, after waiting for its level if another lane opens
+// that.  Every open comes before every fill: a wave that waited with a level
+// of its own unpublished could wait for a wave that waits for that level (the
+// slots are taken by atomics on different words, in flight together, so either
+// wave may be the first on one word and the second on the other).
 template <uint32_t Q, class Store>
 AXR_HD void place_entries(Store& s) {
+    bool far = false;
+#pragma unroll
+    for (uint32_t q = 0; q < Q; ++q) far |= s.near(q);
+    if (!s.any(far)) return;
 #pragma unroll
     for (uint32_t q = 0; q < Q; ++q) s.open(q);
 #pragma unroll

@@ -493,9 +493,14 @@ struct BinStore {
     __device__ __forceinline__ uint32_t* cell(uint32_t q, const BinSlot& b) const {
         return ar.bin_chunks + (size_t)bin[q] * BIN_LEVELS + b.level;
     }
+    __device__ __forceinline__ bool near(uint32_t q) {
+        const bool first = (slot[q] >> ar.bin0_shift) == 0u;
+        if (act[q] && first) ar.bins[((size_t)bin[q] << ar.bin0_shift) + slot[q]] = ref[q];
+        return act[q] && !first;
+    }
+    __device__ __forceinline__ bool any(bool far) const { return __ballot(far) != 0ull; }
     __device__ __forceinline__ void open(uint32_t q) {
         const BinSlot b = bin_slot(ar.bin0_shift, slot[q]);
-        if (act[q] && b.level == 0u) ar.bins[((size_t)bin[q] << ar.bin0_shift) + slot[q]] = ref[q];
         if (act[q] && b.level != 0u && b.offset == 0u) {
             const uint32_t at = pool_take(ar, bin[q], 1u << (ar.bin0_shift + b.level));
             __hip_atomic_store(cell(q, b), at ? at : CHUNK_NONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

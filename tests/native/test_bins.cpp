@@ -90,10 +90,19 @@ struct Wave {
 struct WaveStore {
     Bins& bins;
     const std::vector<Entry> (&e)[Q];
+    bool near(uint32_t q) {
+        bool far = false;
+        for (const Entry& x : e[q]) {
+            const bool first = bin_slot(SHIFT, x.slot).level == 0u;
+            if (x.act && first) bins.first[(x.bin << SHIFT) + x.slot] = x.ref;
+            far |= x.act && !first;
+        }
+        return far;
+    }
+    bool any(bool far) const { return far; }
     void open(uint32_t q) {
         for (const Entry& x : e[q]) {
             const BinSlot b = bin_slot(SHIFT, x.slot);
-            if (x.act && b.level == 0u) bins.first[(x.bin << SHIFT) + x.slot] = x.ref;
             if (x.act && b.level != 0u && b.offset == 0u) {
                 const uint32_t o = bins.next.fetch_add(1u << (SHIFT + b.level));
                 bins.cells[x.bin * BIN_LEVELS + b.level].store(o + 1u, std::memory_order_relaxed);
