@@ -1046,8 +1046,8 @@ int axr_fb_destroy(axr_fb* fb) {
 
 int axr_fb_clear(axr_fb* fb, uint32_t bgra, float depth) {
     if (!fb) return AXR_ERR_INVALID;
-    // recorded, not written: the next draw in visibility mode writes it as
-    // part of its last pass; any other use of the planes writes it first
+    // recorded, not written: the next axr_draw writes it as part of its last
+    // pass; any other use of the planes writes it first
     fb->clear_pending = true;
     fb->clear_bgra = bgra;
     fb->clear_depth = depth;
@@ -1219,7 +1219,8 @@ int axr_draw(axr_ctx* ctx, axr_fb* fb, const axr_mesh* mesh, const axr_draw_para
         if (!ctx->main.host_counters[CNT_ERROR]) return AXR_OK;
         r = arena_check_overflow(ctx, ctx->err, ctx->main, fs);
         if (r != AXR_ERR_OVERFLOW) return r;
-        // the raster stage was skipped, so the framebuffer is untouched: redraw
+        // the raster stage was skipped, so the framebuffer holds what it held, or
+        // the clear that the draw absorbs: redraw
     }
     return fail(ctx->err, AXR_ERR_OVERFLOW, "axr_draw: frame arena kept overflowing");
 }

@@ -168,9 +168,9 @@ struct axr_fb {
     uint32_t* ids = nullptr;
     size_t bytes = 0;
     uint32_t batch_refs = 0;   // live batches with this framebuffer as a view
-    // A clear not yet written: the next visibility-mode draw writes it as
-    // part of its resolve; anything else that reads or draws into the planes
-    // writes it first (axr::fb_settle).
+    // A clear not yet written: the next axr_draw writes it as part of its last
+    // pass; anything else that reads or draws into the planes writes it first
+    // (axr::fb_settle).
     bool clear_pending = false;
     uint32_t clear_bgra = 0;
     float clear_depth = 0.0f;
@@ -192,12 +192,13 @@ struct FrameSize {
     uint64_t pixels = 0;     // visibility-buffer pixels (0 in binned mode)
     uint64_t color_slots = 0; // pixels of a two-pass resolve into a framebuffer with ids
 };
-// High-water marks the kernels reported after an overflow.
 FrameSize frame_size(const KArgs& ka);
 
 int arena_create(axr_ctx* ctx, ErrSink& err, FrameArena& fa, bool lean = false);
 void arena_destroy(axr_ctx* ctx, FrameArena& fa);
 uint64_t arena_bytes(const FrameArena& fa);
+// Grows the arena for a frame of size fs and for what overflowing frames
+// reported (fs of no bins: for the latter alone).
 int arena_ensure(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs, const ArenaNeeds& need = {});
 int arena_read_counters(ErrSink& err, FrameArena& fa);
 // With the arena's work finished: the counters copied back if a kernel
@@ -213,11 +214,10 @@ int arena_launch(ErrSink& err, FrameArena& fa, const KArgs& ka, StageEvents* ev,
 // high-water marks, reset it and return AXR_ERR_OVERFLOW.
 int arena_check_overflow(axr_ctx* ctx, ErrSink& err, FrameArena& fa, const FrameSize& fs);
 
-// The uniforms drawMesh sets (reference tiled_pipeline.cpp:148-155).
-// Queue on the main stream behind everything queued on the second arena's
-// stream (no host wait).
+// Queue on the main stream behind everything queued on the other arenas'
+// streams (no host wait).
 int ctx_join(axr_ctx* ctx);
-// Host wait for both streams.
+// Host wait for every arena's stream.
 int ctx_sync_all(axr_ctx* ctx);
 // Write a framebuffer's pending clear, if any (stream-ordered).
 int fb_settle(axr_fb* fb);
@@ -236,6 +236,7 @@ struct PassSkips {
     double sign = 0.0, tau = 0.0;
 };
 PassSkips pass_skips(const axr_mesh* m, const mat4& mvp, int W, int H, int footprint);
+// The uniforms drawMesh sets (reference tiled_pipeline.cpp:148-155).
 ViewDesc make_view(const axr_mesh* m, uint32_t* color, float* depth, uint32_t* ids, int w, int h,
                    const axr_draw_params* p, int tile);
 bool shader_ok(const axr_draw_params* p);
